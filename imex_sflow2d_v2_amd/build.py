@@ -1,9 +1,11 @@
 """Build the gfx950 library ``libimexsw.so`` in-tree with hipcc.
 
 The library is one C-ABI translation unit (``imexsw.hip``) plus
-``imexsw_ns.hip`` compiled once per number of solid classes (0..6), which
-holds the kernels templated on it; the objects compile in parallel and are
-linked into one shared library.
+``imexsw_ns.hip`` compiled once per number of solid classes (0..6) and part
+(the plain stencils, the local pass, the tableau-driven stages, the profile
+stencils, the ensemble), which holds the kernels templated on the number of
+classes; the objects compile in parallel and are linked into one shared
+library.
 
 FP policy: IEEE division and square root (hipcc defaults), no FMA
 contraction (``-ffp-contract=off``) so device results follow the reference's
@@ -19,6 +21,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libimexsw.so")
 NS_VALUES = range(0, 7)
+PARTS = range(0, 5)
 SOURCES = ["imexsw.hip", "imexsw_ns.hip"]
 HEADERS = ["imexsw_math.h", "imexsw_physics.h", "imexsw_newton.h", "imexsw_kernels.h",
            "imexsw_batch.h", "imexsw_mlp.h", "imexsw_q2d.h", "imexsw_ctx.h",
@@ -58,10 +61,15 @@ def compile_units(extra=()):
     units = [([hipcc()] + HIPCC_FLAGS + list(extra) + ["-c", os.path.join(CSRC, "imexsw.hip"),
                                                       "-o", os.path.join(OBJ, "imexsw.o")],
               os.path.join(OBJ, "imexsw.o"))]
-    for ns in NS_VALUES:
-        o = os.path.join(OBJ, "imexsw_ns%d.o" % ns)
-        units.append(([hipcc()] + HIPCC_FLAGS + list(extra) +
-                      ["-DIMEXSW_NS=%d" % ns, "-c", os.path.join(CSRC, "imexsw_ns.hip"), "-o", o], o))
+    # the largest objects first, so that the last ones to finish are small
+    for ns in reversed(NS_VALUES):
+        for part in PARTS:
+            if part == 4 and not 1 <= ns <= 3:
+                continue  # ensembles: 1 to 3 classes
+            o = os.path.join(OBJ, "imexsw_ns%d_%d.o" % (ns, part))
+            units.append(([hipcc()] + HIPCC_FLAGS + list(extra) +
+                          ["-DIMEXSW_NS=%d" % ns, "-DIMEXSW_PART=%d" % part, "-c",
+                           os.path.join(CSRC, "imexsw_ns.hip"), "-o", o], o))
     return units
 
 

@@ -123,12 +123,15 @@ inline BatchLists batch_lists(imexsw_ensemble* e) {
 }
 
 // Launches of the kernels templated on the number of solid classes NS,
-// defined in imexsw_ns.hip (one object per NS).
+// defined in imexsw_ns.hip (five objects per NS).
 // rows: the six-wavefront row stencil (sparse steps); else strips.  D: the
 // context's pointers, or a copy whose state and residual planes are a
 // stage's (N_RK != 2)
 template <int NS>
 void launch_stencil(imexsw_ctx* c, const DevPtrs& D, int compute_dt, bool rows);
+// the same with the vertical profiles; items: (listed tile, strip) pairs at most
+template <int NS>
+void launch_stencil_vp(imexsw_ctx* c, const DevPtrs& D, int compute_dt, int items);
 // fused: stage update, erosion and diagnostics of a row in one pass (sparse
 // steps without the learned warm start); else up to two kernels
 template <int NS>

@@ -1,10 +1,11 @@
 // imexsw_ns.hip -- launches of the kernels templated on the number of solid
-// classes, compiled once per value with -DIMEXSW_NS=<0..6> so that the
-// instantiations build in parallel (the C ABI is in imexsw.hip).
+// classes, compiled once per value and part with -DIMEXSW_NS=<0..6>
+// -DIMEXSW_PART=<0..4> so that the instantiations build in parallel (the C
+// ABI is in imexsw.hip).
 #include "imexsw_ctx.h"
 
-#ifndef IMEXSW_NS
-#error "compile with -DIMEXSW_NS=<number of solid classes>"
+#if !defined(IMEXSW_NS) || !defined(IMEXSW_PART)
+#error "compile with -DIMEXSW_NS=<number of solid classes> -DIMEXSW_PART=<0..4>"
 #endif
 
 namespace imexsw {
@@ -19,28 +20,7 @@ void launch_stencil(imexsw_ctx* c, const DevPtrs& D, int compute_dt, bool rows) 
     hipLaunchKernelGGL((k_stencil_rows<NS>), dim3(std::min(c->n_tiles * kTileH, res)),
                        dim3(384), 0, c->stream, c->P, D, compute_dt);
   } else if (c->P.vp) {
-    // the profile closures (general path only)
-    static int res2 = 0, res1 = 0, res_s = 0, res_v = 0;
-    if (c->P.ny > 1 && D.sides && D.qpp) {
-      // the state's stored physical variables: its face sides first
-      if (!res_s) res_s = resident_grid(k_vp_sides<NS>, 256, c->n_cu, 1 << 30);
-      if (!res_v) res_v = resident_grid(k_stencil_vp<NS>, 64, c->n_cu, 1 << 30);
-      hipLaunchKernelGGL((k_vp_sides<NS>), dim3(std::min(c->n_tiles, res_s)), dim3(256), 0,
-                         c->stream, c->P, D);
-      hipLaunchKernelGGL((k_stencil_vp<NS>), dim3(std::min(items, res_v)), dim3(64), 0,
-                         c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                         compute_dt);
-    } else if (c->P.ny > 1) {
-      if (!res2) res2 = resident_grid(k_stencil<NS, true, true>, 64, c->n_cu, 1 << 30);
-      hipLaunchKernelGGL((k_stencil<NS, true, true>), dim3(std::min(items, res2)), dim3(64), 0,
-                         c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                         compute_dt);
-    } else {
-      if (!res1) res1 = resident_grid(k_stencil<NS, false, true>, 64, c->n_cu, 1 << 30);
-      hipLaunchKernelGGL((k_stencil<NS, false, true>), dim3(std::min(items, res1)), dim3(64), 0,
-                         c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                         compute_dt);
-    }
+    launch_stencil_vp<NS>(c, D, compute_dt, items);
   } else if (c->P.ny > 1) {
     static int res = 0;
     if (!res) res = resident_grid(k_stencil<NS, true>, 64, c->n_cu, 1 << 30);
@@ -55,6 +35,33 @@ void launch_stencil(imexsw_ctx* c, const DevPtrs& D, int compute_dt, bool rows) 
                        compute_dt);
   }
 }
+#if IMEXSW_PART == 3
+// the profile closures (general path only)
+template <int NS>
+void launch_stencil_vp(imexsw_ctx* c, const DevPtrs& D, int compute_dt, int items) {
+  static int res2 = 0, res1 = 0, res_s = 0, res_v = 0;
+  if (c->P.ny > 1 && D.sides && D.qpp) {
+    // the state's stored physical variables: its face sides first
+    if (!res_s) res_s = resident_grid(k_vp_sides<NS>, 256, c->n_cu, 1 << 30);
+    if (!res_v) res_v = resident_grid(k_stencil_vp<NS>, 64, c->n_cu, 1 << 30);
+    hipLaunchKernelGGL((k_vp_sides<NS>), dim3(std::min(c->n_tiles, res_s)), dim3(256), 0,
+                       c->stream, c->P, D);
+    hipLaunchKernelGGL((k_stencil_vp<NS>), dim3(std::min(items, res_v)), dim3(64), 0,
+                       c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
+                       compute_dt);
+  } else if (c->P.ny > 1) {
+    if (!res2) res2 = resident_grid(k_stencil<NS, true, true>, 64, c->n_cu, 1 << 30);
+    hipLaunchKernelGGL((k_stencil<NS, true, true>), dim3(std::min(items, res2)), dim3(64), 0,
+                       c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
+                       compute_dt);
+  } else {
+    if (!res1) res1 = resident_grid(k_stencil<NS, false, true>, 64, c->n_cu, 1 << 30);
+    hipLaunchKernelGGL((k_stencil<NS, false, true>), dim3(std::min(items, res1)), dim3(64), 0,
+                       c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
+                       compute_dt);
+  }
+}
+#endif
 template <int NS>
 void launch_local(imexsw_ctx* c, int ops, bool fused) {
   // work items: listed tile rows, four per workgroup
@@ -190,16 +197,21 @@ void launch_batch_local(imexsw_ensemble* e) {
                      e->d_params, e->d_ptrs, L, (int)(OP_EROSION | OP_POST));
 }
 
+#if IMEXSW_PART == 0
 template void launch_stencil<IMEXSW_NS>(imexsw_ctx*, const DevPtrs&, int, bool);
-template void launch_stage<IMEXSW_NS>(imexsw_ctx*, int, int);
-template void launch_assemble<IMEXSW_NS>(imexsw_ctx*, int);
-template void launch_local<IMEXSW_NS>(imexsw_ctx*, int, bool);
 template void launch_qp<IMEXSW_NS>(imexsw_ctx*, double*, int, int);
 template void launch_qp_planes<IMEXSW_NS>(imexsw_ctx*);
 template void launch_convert<IMEXSW_NS>(const DevParams&, hipStream_t, int, long long,
                                         const double*, const double*, const double*, double*,
                                         int);
-#if IMEXSW_NS >= 1 && IMEXSW_NS <= 3
+#elif IMEXSW_PART == 1
+template void launch_local<IMEXSW_NS>(imexsw_ctx*, int, bool);
+#elif IMEXSW_PART == 2
+template void launch_stage<IMEXSW_NS>(imexsw_ctx*, int, int);
+template void launch_assemble<IMEXSW_NS>(imexsw_ctx*, int);
+#elif IMEXSW_PART == 3
+template void launch_stencil_vp<IMEXSW_NS>(imexsw_ctx*, const DevPtrs&, int, int);
+#elif IMEXSW_PART == 4 && IMEXSW_NS >= 1 && IMEXSW_NS <= 3
 template void launch_batch_stencil<IMEXSW_NS>(imexsw_ensemble*);
 template void launch_batch_local<IMEXSW_NS>(imexsw_ensemble*);
 #endif
