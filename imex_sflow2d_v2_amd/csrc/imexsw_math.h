@@ -22,6 +22,48 @@ constexpr double kLn2Hi = 6.93147180369123816490e-01;  // 0x3fe62e42fee00000
 constexpr double kLn2Lo = 1.90821492927058770002e-10;
 constexpr double kInvLn2 = 1.44269504088896338700e+00;
 
+// ---------------------------------------------------------------------------
+// IEEE division and square root, one step at a time.  The compiler expands a
+// double division into two scalings, a reciprocal estimate refined twice, the
+// quotient with one correction and a fix-up of the special cases: 12
+// instructions on one dependent chain, and both scalings and the correction
+// go through the one VCC register, so neighbouring divisions cannot overlap.
+// rcp_of and div_by are the same chain without the scalings, which change
+// nothing unless an operand is near the ends of the exponent range: the
+// quotient has the same bits for |b| in [2^-1022, 2^1021] and |a| in
+// [2^-969, 2^767 |b|], and for a zero, an infinity or a NaN (the fix-up
+// decides those).  Numerators below 2^-969 lose the exact last bit of a
+// quotient of order 1e-290.  Divisions by one value share its reciprocal:
+// 4 instructions each after the first.
+// ---------------------------------------------------------------------------
+struct Rcp {
+  double b, r;  // the divisor and its refined reciprocal
+};
+__device__ __forceinline__ Rcp rcp_of(double b) {
+  double r = __builtin_amdgcn_rcp(b);
+  r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+  r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+  return Rcp{b, r};
+}
+__device__ __forceinline__ double div_by(double a, const Rcp& d) {
+  const double q = a * d.r;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.b, q, a), d.r, q), d.b, a);
+}
+__device__ __forceinline__ double fdiv(double a, double b) { return div_by(a, rcp_of(b)); }
+
+// sqrt(x) without the scaling of arguments below 2^-767 (the same bits above
+// it, and for zero, infinity and NaN)
+__device__ __forceinline__ double fsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = y * 0.5;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0, +infinity
+}
+
 // The special cases are selected after the fact rather than branched
 // around, so that the straight-line code of independent calls can overlap.
 __device__ __forceinline__ double det_log(double x) {

@@ -18,9 +18,8 @@ __device__ __forceinline__ void finish_f(const double* qj, const double* qold,
   double s = 0.0;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    double nh = (i == 1) ? nh1 : (i == 2) ? nh2 : 0.0;
-    double R = Rj[i] - a_diag * nh;
-    f[i] = 1.0 * (qj[i] - qold[i] + dt * R);
+    const double R = (i == 1) ? Rj[1] - a_diag * nh1 : (i == 2) ? Rj[2] - a_diag * nh2 : Rj[i];
+    f[i] = qj[i] - qold[i] + dt * R;
   }
 #pragma unroll
   for (int i = 0; i < NV; i++) s += f[i] * f[i];
@@ -31,13 +30,9 @@ __device__ __forceinline__ void eval_f(const DevParams& P, const double* qj,
                                        const double* qold, const double* Rj,
                                        double a_diag, double dt, double Bx,
                                        double By, double* f, double& scal) {
-  constexpr int NV = 4 + NS;
-  cpx cq[NV];
-#pragma unroll
-  for (int i = 0; i < NV; i++) cq[i] = mk(qj[i], 0.0);
-  cpx n1, n2;
-  implicit_c<NS, RM>(P, cq, Bx, By, n1, n2);
-  finish_f<NS>(qj, qold, Rj, a_diag, dt, n1.re, n2.re, f, scal);
+  ImplPt b;
+  implicit_real<NS, RM>(P, qj, Bx, By, b);
+  finish_f<NS>(qj, qold, Rj, a_diag, dt, b.n1, b.n2, f, scal);
 }
 
 // gfortran NORM2 (scaled sum of squares)
@@ -67,6 +62,133 @@ struct NewtonOut {
   int ls_evals;  // residual evaluations inside the line search
 };
 
+// The Newton step from the residual rt and the implicit terms' derivatives
+// J1[], J2[] (d nh_{1,2} / d rel_1, rel_2): the partitioned solve of
+// src/solver_2d.f90:1846-1925 on the 2x2 momentum block (the other unknowns'
+// columns are the diagonal org, their right-hand side terms are zero).
+// L receives the block (11, 21, 12, 22).
+template <int NS>
+__device__ __forceinline__ void newton_step(const double* org, const double* rt, double dta,
+                                            const double* J1, const double* J2, double* L,
+                                            double* desc) {
+  constexpr int NV = 4 + NS;
+  L[0] = org[1] - dta * J1[0];
+  L[1] = 0.0 - dta * J1[1];
+  L[2] = 0.0 - dta * J2[0];
+  L[3] = org[2] - dta * J2[1];
+  const double inv_det = fdiv(1.0, L[0] * L[3] - L[1] * L[2]);
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    if (i == 1) desc[i] = -((rt[1] * L[3] - rt[2] * L[2]) * inv_det) + 0.0;
+    else if (i == 2) desc[i] = -((L[0] * rt[2] - L[1] * rt[1]) * inv_det) + 0.0;
+    else desc[i] = 0.0 + -fdiv(rt[i], org[i]);
+  }
+}
+
+// What lnsrch (src/solver_2d.f90:2019-2224) forms ahead of its first trial.
+// The step's norm is only compared with stpmax >= 100 NV, and the smallest
+// step alamin only matters after a rejected trial, so neither is formed
+// while the largest component of the step is at most 100: the norm is then
+// below stpmax / 2.  slope: desc . (rt . L) with L's zero entries left out.
+struct LineSearch {
+  double slope, dmax, mx;
+  bool have_mx;  // mx is known (else formed by below_alamin when needed)
+  bool none;     // alamin == 0: no trial, the step is dropped
+};
+constexpr double kTolX = kEps;
+
+template <int NV>
+__device__ __forceinline__ double ls_mx(const double* desc, const double* old) {
+  double mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const double v = fdiv(fabs(desc[i]), fmax(fabs(old[i]), 1.0));
+    if (v > mx) mx = v;
+  }
+  return mx;
+}
+template <int NS>
+__device__ __forceinline__ LineSearch ls_begin(const double* org, const double* old,
+                                               const double* rt, const double* L,
+                                               double* desc) {
+  constexpr int NV = 4 + NS;
+  LineSearch s{0.0, -1.0, 0.0, false, false};
+#pragma unroll
+  for (int i = 0; i < NV; i++) s.dmax = fmax(s.dmax, fabs(desc[i]));
+  if (!(s.dmax >= 0.0 && s.dmax <= 100.0)) {
+    double dd = 0.0;
+#pragma unroll
+    for (int i = 0; i < NV; i++) dd += old[i] * old[i];
+    const double stpmax = 100.0 * fmax(sqrt(dd), (double)NV);
+    const double dabs = norm2_<NV>(desc);
+    if (dabs > stpmax) {
+#pragma unroll
+      for (int i = 0; i < NV; i++) desc[i] = desc[i] * stpmax / dabs;
+    }
+    s.mx = ls_mx<NV>(desc, old);
+    s.have_mx = true;
+    s.none = (kTolX / s.mx) == 0.0;
+  }
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const double g = (i == 1) ? rt[1] * L[0] + rt[2] * L[1]
+                     : (i == 2) ? rt[1] * L[2] + rt[2] * L[3] : rt[i] * org[i];
+    s.slope += g * desc[i];
+  }
+  return s;
+}
+// alam < alamin = TOLX / mx, mx the largest |desc| / max(|old|, 1): decided
+// without the divisions unless alam is within 1e-6 of alamin's bounds
+template <int NV>
+__device__ __forceinline__ bool below_alamin(LineSearch& s, double alam, const double* desc,
+                                             const double* old) {
+  if (!s.have_mx) {
+    double om = 1.0;
+#pragma unroll
+    for (int i = 0; i < NV; i++) om = fmax(om, fabs(old[i]));
+    const double hi = alam * s.dmax;
+    if (hi < 0.999999 * kTolX) return true;
+    if (hi > 1.000001 * kTolX * om) return false;
+    s.mx = ls_mx<NV>(desc, old);
+    s.have_mx = true;
+  }
+  return alam < kTolX / s.mx;
+}
+
+// org = max(|q|, 1e-3), rel = q / org (+-1 where |q| is the larger).  Returns
+// whether rel * org is q again (it may be a rounding off below 1e-3).
+template <int NV>
+__device__ __forceinline__ bool newton_scale(const double* q, double* org, double* rel) {
+  const Rcp rm = rcp_of(1.0e-3);
+  bool same = true;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const double a = fabs(q[i]);
+    org[i] = fmax(a, 1.0e-3);
+    rel[i] = (a >= 1.0e-3 && a < INFINITY) ? copysign(1.0, q[i]) : div_by(q[i], rm);
+    if (a == INFINITY) rel[i] = __builtin_nan("");
+    same = same && rel[i] * org[i] == q[i];
+  }
+  return same;
+}
+
+template <int NV>
+__device__ __forceinline__ double max_abs(const double* x) {
+  double m = 0.0;
+#pragma unroll
+  for (int i = 0; i < NV; i++) m = fmax(m, fabs(x[i]));
+  return m;
+}
+// max |rel - old| / max(|rel|, 1) < TOLX (a power of two: the product is exact)
+template <int NV>
+__device__ __forceinline__ bool step_below_tolx(const double* rel, const double* old) {
+  bool below = true;
+#pragma unroll
+  for (int i = 0; i < NV; i++)
+    below = below && !(fabs(rel[i] - old[i]) >= kTolX * fmax(fabs(rel[i]), 1.0));
+  return below;
+}
+
 // solve_rk_step with eval_jacobian and lnsrch (src/solver_2d.f90:1660-2365);
 // RM = 6: the implicit terms of rheology model 6.
 // The implicit unknowns are the momenta (implicit_flag = F,T,T,F,...,
@@ -77,204 +199,104 @@ template <int NS, int RM = 1>
 __device__ __forceinline__ NewtonOut solve_rk_step(const DevParams& P, double* qj,
                                                   const double* qold,
                                                   const double* Rj, double a_diag,
-                                                  double dt, double Bx, double By,
-                                                  const double* rt0 = nullptr,
-                                                  double scal0 = 0.0) {
+                                                  double dt, double Bx, double By) {
   constexpr int NV = 4 + NS;
   const double TOLF = 1.0e-10;
-  const double TOLX = kEps;
   double org[NV], rel[NV], rt[NV], old[NV], desc[NV];
-  double scal, scal_old;
-#pragma unroll
-  for (int i = 0; i < NV; i++) org[i] = fmax(fabs(qj[i]), 1.0e-3);
-#pragma unroll
-  for (int i = 0; i < NV; i++) rel[i] = qj[i] / org[i];
+  double scal = 0.0;
+  const bool same = newton_scale<NV>(qj, org, rel);
   NewtonOut out{0, 0, 0};
   int it;
-  // rt / scal already hold the residual at qj when the previous iteration
-  // ended on an evaluated point (an accepted line-search point or the full
-  // first step); the reference evaluates it again at the top of the
-  // iteration, with the same operands, so that evaluation is skipped
+  // b, rt and scal already belong to qj when the previous iteration ended
+  // on an evaluated point (an accepted line-search point or the full first
+  // step); the reference evaluates it again at the top of the iteration,
+  // with the same operands, so that evaluation is skipped
+  ImplPt b;
   bool fresh = false;
-  if (rt0) {
-    // residual at the starting point already evaluated by the caller
-#pragma unroll
-    for (int i = 0; i < NV; i++) rt[i] = rt0[i];
-    scal = scal0;
-    fresh = true;
-  }
   for (it = 1; it <= 100; it++) {
-    if (!fresh) eval_f<NS, RM>(P, qj, qold, Rj, a_diag, dt, Bx, By, rt, scal);
-    bool restored = false;
-    double mf = 0.0;
+    if (!fresh) {
+      // the residual at qj; the Jacobian's point is rel * org, which in the
+      // first iteration may be a rounding off qj
+#pragma unroll 1
+      for (int e = 0; e < 2; e++) {
+        double q[NV];
 #pragma unroll
-    for (int i = 0; i < NV; i++) mf = fmax(mf, fabs(rt[i]));
-    if (mf < TOLF) {
+        for (int m = 0; m < NV; m++) q[m] = e ? rel[m] * org[m] : qj[m];
+        implicit_real<NS, RM>(P, q, Bx, By, b);
+        if (e == 0) finish_f<NS>(qj, qold, Rj, a_diag, dt, b.n1, b.n2, rt, scal);
+        if (it > 1 || same) break;
+      }
+    }
+    bool restored = false;
+    if (max_abs<NV>(rt) < TOLF) {
       out.conv = 1;
       break;
     }
     // --- Jacobian: complex step on the two momentum columns
-    const double dta = dt * a_diag;
-    double J1[3], J2[3];  // d nh_{1,2} / d rel_{1}, d nh_{1,2} / d rel_{2}
+    double J1[2], J2[2], L[4];
     {
-      cpx cq[NV];
+      const double q1 = rel[1] * org[1], q2 = rel[2] * org[2];
+      const double d1 = P.h_cs * org[1], d2 = P.h_cs * org[2];
+      bool ok = implicit_col<RM>(P, b, q1, q2, d1, 0.0, Bx, By, J1[0], J1[1]);
+      ok = implicit_col<RM>(P, b, q1, q2, 0.0, d2, Bx, By, J2[0], J2[1]) && ok;
+      if (!ok) {
+        double q[NV];
 #pragma unroll
-      for (int m = 0; m < NV; m++) cq[m] = mk(rel[m], 0.0);
-      cq[1] = mk(rel[1], P.h_cs);
-#pragma unroll
-      for (int m = 0; m < NV; m++) cq[m] = cmulr(cq[m], org[m]);
-      cpx n1, n2;
-      implicit_c<NS, RM>(P, cq, Bx, By, n1, n2);
-      J1[1] = 1.0 * n1.im * P.one_by_h;
-      J1[2] = 1.0 * n2.im * P.one_by_h;
-    }
-    {
-      cpx cq[NV];
-#pragma unroll
-      for (int m = 0; m < NV; m++) cq[m] = mk(rel[m], 0.0);
-      cq[2] = mk(rel[2], P.h_cs);
-#pragma unroll
-      for (int m = 0; m < NV; m++) cq[m] = cmulr(cq[m], org[m]);
-      cpx n1, n2;
-      implicit_c<NS, RM>(P, cq, Bx, By, n1, n2);
-      J2[1] = 1.0 * n1.im * P.one_by_h;
-      J2[2] = 1.0 * n2.im * P.one_by_h;
-    }
-    // left_matrix entries (column 1 and 2 of the momentum block); rows of
-    // the other equations of those columns are 0 - dta*(1.0*0*one_by_h) = 0
-    const double zJ = 1.0 * 0.0 * P.one_by_h;
-    const double L11 = 1.0 * org[1] - dta * J1[1];
-    const double L21 = 0.0 - dta * J1[2];
-    const double L12 = 0.0 - dta * J2[1];
-    const double L22 = 1.0 * org[2] - dta * J2[2];
-    const double Lz = 0.0 - dta * zJ;  // off-block rows of the implicit columns
-    // partitioned solve (:1846-1925)
-    double d1[NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++) d1[i] = (i == 1 || i == 2) ? 0.0 : rt[i] / (1.0 * org[i]);
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++)
-      if (i != 1 && i != 2) s += d1[i] * 0.0;
-    double b1 = rt[1] - s, b2 = rt[2] - s;
-    {
-      // the same partial sum for both implicit rows (MATMUL over zeros)
-      double inv_det = 1.0 / (L11 * L22 - L21 * L12);
-      double x1 = (b1 * L22 - b2 * L12) * inv_det;
-      double x2 = (L11 * b2 - L21 * b1) * inv_det;
-#pragma unroll
-      for (int i = 0; i < NV; i++) {
-        if (i == 1) desc[i] = -x1 + 0.0;
-        else if (i == 2) desc[i] = -x2 + 0.0;
-        else desc[i] = 0.0 + -d1[i];
+        for (int m = 0; m < NV; m++) q[m] = rel[m] * org[m];
+#pragma unroll 1
+        for (int p = 0; p < 2; p++) {
+          double a, c;
+          implicit_col_c<NS, RM>(P, q, p ? 0.0 : d1, p ? d2 : 0.0, Bx, By, a, c);
+          J1[0] = p ? J1[0] : a;
+          J1[1] = p ? J1[1] : c;
+          J2[0] = a;
+          J2[1] = c;
+        }
       }
+      J1[0] = J1[0] * P.one_by_h;
+      J1[1] = J1[1] * P.one_by_h;
+      J2[0] = J2[0] * P.one_by_h;
+      J2[1] = J2[1] * P.one_by_h;
     }
+    newton_step<NS>(org, rt, dt * a_diag, J1, J2, L, desc);
 #pragma unroll
     for (int i = 0; i < NV; i++) old[i] = rel[i];
-    scal_old = scal;
-    if (it > 1) {
-      double dd = 0.0;
+    double alam = 1.0;
+    LineSearch ls{};
+    if (it > 1) ls = ls_begin<NS>(org, old, rt, L, desc);
+    const double scal_old = scal;
+    // The trials of lnsrch: the full step (accepted as it is in the first
+    // iteration), then max(quadratic model, 0.5), then halvings (the cubic
+    // model is capped at half the last step, so max(model, 0.5 * alam) is
+    // always 0.5 * alam).  alam at least halves every pass after the first,
+    // so it falls below alamin (>= ~1e-16 relative) within a few dozen
+    // passes; the bound only guards against NaN states.
+    for (int tr = 0; tr < 256 && !ls.none; tr++) {
 #pragma unroll
-      for (int i = 0; i < NV; i++) dd += rel[i] * rel[i];
-      double stpmax = 100.0 * fmax(sqrt(dd), (double)NV);
-      double grad[NV];
-#pragma unroll
-      for (int i = 0; i < NV; i++) {
-        double g = 0.0;
-#pragma unroll
-        for (int r = 0; r < NV; r++) {
-          double Lri;
-          if (i == 1) Lri = (r == 1) ? L11 : (r == 2) ? L21 : Lz;
-          else if (i == 2) Lri = (r == 1) ? L12 : (r == 2) ? L22 : Lz;
-          else Lri = (r == i) ? 1.0 * org[i] : 0.0;
-          g += rt[r] * Lri;
-        }
-        grad[i] = g;
-      }
-      // ---- lnsrch (:2019-2224)
-      double dabs = norm2_<NV>(desc);
-      if (dabs > stpmax) {
-#pragma unroll
-        for (int i = 0; i < NV; i++) desc[i] = desc[i] * stpmax / dabs;
-      }
-      double slope = 0.0;
-#pragma unroll
-      for (int i = 0; i < NV; i++) slope += grad[i] * desc[i];
-      double mx = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < NV; i++) {
-        double v = fabs(desc[i]) / fmax(fabs(old[i]), 1.0);
-        if (v > mx) mx = v;
-      }
-      double alamin = TOLX / mx;
-      if (alamin == 0.0) {
-#pragma unroll
-        for (int i = 0; i < NV; i++) rel[i] = old[i];
-      } else {
-        double alam = 1.0, alam2 = 0.0, f2 = 0.0, tmplam = 0.0;
-        // alam at least halves every pass after the first, so it falls
-        // below alamin (>= ~1e-16 relative) within a few dozen passes; the
-        // bound only guards against NaN states
-        for (int ls = 0; ls < 256; ls++) {
-          double q[NV];
-#pragma unroll
-          for (int i = 0; i < NV; i++) rel[i] = old[i] + alam * desc[i];
-#pragma unroll
-          for (int i = 0; i < NV; i++) q[i] = rel[i] * org[i];
-          eval_f<NS, RM>(P, q, qold, Rj, a_diag, dt, Bx, By, rt, scal);
-          out.ls_evals++;
-          if (scal <= 0.9 * scal_old) break;
-          if (alam < alamin) {
-#pragma unroll
-            for (int i = 0; i < NV; i++) rel[i] = old[i];
-            scal = scal_old;
-            restored = true;  // rt belongs to the rejected trial point
-            break;
-          }
-          if (alam == 1.0) {
-            tmplam = -(slope / (2.0 * (scal - scal_old - slope)));
-          } else {
-            double rhs1 = scal - scal_old - alam * slope;
-            double rhs2 = f2 - scal_old - alam2 * slope;
-            double a = (rhs1 / (alam * alam) - rhs2 / (alam2 * alam2)) / (alam - alam2);
-            double b = (-(alam2 * rhs1 / (alam * alam)) + alam * rhs2 / (alam2 * alam2)) /
-                       (alam - alam2);
-            if (a == 0.0) {
-              tmplam = -(slope / (2.0 * b));
-            } else {
-              double disc = b * b - 3.0 * a * slope;
-              if (disc < 0.0) tmplam = 0.5 * alam;
-              else if (b <= 0.0) tmplam = (-b + sqrt(disc)) / (3.0 * a);
-              else tmplam = -(slope / (b + sqrt(disc)));
-            }
-            if (tmplam > 0.5 * alam) tmplam = 0.5 * alam;
-          }
-          alam2 = alam;
-          f2 = scal;
-          alam = fmax(tmplam, 0.5 * alam);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NV; i++) rel[i] = old[i] + desc[i];
+      for (int i = 0; i < NV; i++) rel[i] = old[i] + alam * desc[i];
 #pragma unroll
       for (int i = 0; i < NV; i++) qj[i] = rel[i] * org[i];
-      eval_f<NS, RM>(P, qj, qold, Rj, a_diag, dt, Bx, By, rt, scal);
+      implicit_real<NS, RM>(P, qj, Bx, By, b);
+      finish_f<NS>(qj, qold, Rj, a_diag, dt, b.n1, b.n2, rt, scal);
+      if (it == 1) break;
+      out.ls_evals++;
+      if (scal <= 0.9 * scal_old) break;
+      if (below_alamin<NV>(ls, alam, desc, old)) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) rel[i] = old[i];
+        scal = scal_old;
+        restored = true;  // rt belongs to the rejected trial point
+        break;
+      }
+      const double half = 0.5 * alam;
+      alam = (tr == 0)
+                 ? fmax(-fdiv(ls.slope, 2.0 * (scal - scal_old - ls.slope)), half)
+                 : half;
     }
 #pragma unroll
     for (int i = 0; i < NV; i++) qj[i] = rel[i] * org[i];
     fresh = !restored;
-    mf = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++) mf = fmax(mf, fabs(rt[i]));
-    if (mf < TOLF) {
-      out.conv = 1;
-      break;
-    }
-    double mx = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++) mx = fmax(mx, fabs(rel[i] - old[i]) / fmax(fabs(rel[i]), 1.0));
-    if (mx < TOLX) {
+    if (max_abs<NV>(rt) < TOLF || step_below_tolx<NV>(rel, old)) {
       out.conv = 1;
       break;
     }
@@ -284,15 +306,13 @@ __device__ __forceinline__ NewtonOut solve_rk_step(const DevParams& P, double* q
 }
 
 // solve_rk_step on four lanes (4i .. 4i+3, the same cell and operands on
-// each).  One implicit-term evaluation per lane and round: lanes 0 and 1 of
-// the quad the two complex-step Jacobian columns, lane 2 the residual.  A
-// full Newton step (the first iteration) and the line search's first trial
-// (alam = 1) evaluate the residual at the trial point and, at the same time,
-// the Jacobian there, which the next iteration uses when the trial is
-// accepted: the same operands the plain solver would give its Jacobian
-// evaluation, so the same bits, one evaluation earlier.  Every value the
-// control flow depends on is taken from one lane of the quad, so the four
-// lanes stay together.
+// each).  Each evaluation runs the real chain on every lane and the two
+// complex-step Jacobian columns on lanes 0 and 1 of the quad, so residual and
+// Jacobian of a point come from one round: at the start, at the full first
+// step and at the line search's first trial (alam = 1), where lane 3
+// evaluates the trial 0.5 that usually follows a rejection.  The operands are
+// the plain solver's, so the same bits.  Every value the control flow depends
+// on is taken from one lane of the quad, so the four lanes stay together.
 template <int NS>
 __device__ __forceinline__ double quad_from(double v, int role) {
   const int src = (threadIdx.x & 60) | role;
@@ -302,258 +322,143 @@ __device__ __forceinline__ double quad_from(double v, int role) {
   return __hiloint2double(hi, lo);
 }
 
-// One quad round at the point q = rel * org: J1/J2 (columns 1, 2) and the
-// residual rt, scal (when `want_f`; else lanes 2, 3 duplicate column 1)
+// One quad round: this lane's implicit terms nh1, nh2 at its own point q,
+// and J1/J2 (columns 1, 2) at the point of lanes 0 and 1
 template <int NS>
 __device__ __forceinline__ void quad_round(const DevParams& P, const double* q, const double* org,
-                                           const double* qold, const double* Rj, double a_diag,
-                                           double dt, double Bx, double By, bool want_f,
-                                           double* J1, double* J2, double* rt, double& scal) {
-  constexpr int NV = 4 + NS;
+                                           double Bx, double By, double* J1, double* J2,
+                                           double& nh1, double& nh2) {
   const int role = threadIdx.x & 3;
-  const int pcol = (role == 1) ? 2 : (role == 0 || !want_f) ? 1 : -1;  // -1: none
-  cpx cq[NV];
-#pragma unroll
-  for (int m = 0; m < NV; m++) cq[m] = mk(q[m], (m == pcol) ? P.h_cs * org[m] : 0.0);
-  cpx n1, n2;
-  implicit_c<NS>(P, cq, Bx, By, n1, n2);
-  const double a = 1.0 * n1.im * P.one_by_h, b = 1.0 * n2.im * P.one_by_h;
-  J1[1] = quad_from<NS>(a, 0);
-  J1[2] = quad_from<NS>(b, 0);
-  J2[1] = quad_from<NS>(a, 1);
-  J2[2] = quad_from<NS>(b, 1);
-  if (want_f) {
-    const double nh1 = quad_from<NS>(n1.re, 2), nh2 = quad_from<NS>(n2.re, 2);
-    finish_f<NS>(q, qold, Rj, a_diag, dt, nh1, nh2, rt, scal);
-  }
+  ImplPt b;
+  implicit_real<NS>(P, q, Bx, By, b);
+  nh1 = b.n1;
+  nh2 = b.n2;
+  const double d1 = (role == 0) ? P.h_cs * org[1] : 0.0;
+  const double d2 = (role == 1) ? P.h_cs * org[2] : 0.0;
+  double a, c;
+  const bool ok = implicit_col<1>(P, b, q[1], q[2], d1, d2, Bx, By, a, c);
+  if (!ok && role < 2) implicit_col_c<NS>(P, q, d1, d2, Bx, By, a, c);
+  a = a * P.one_by_h;
+  c = c * P.one_by_h;
+  J1[0] = quad_from<NS>(a, 0);
+  J1[1] = quad_from<NS>(c, 0);
+  J2[0] = quad_from<NS>(a, 1);
+  J2[1] = quad_from<NS>(c, 1);
 }
 
 template <int NS>
 __device__ __forceinline__ NewtonOut solve_rk_step_quad(const DevParams& P, double* qj,
                                                        const double* qold, const double* Rj,
                                                        double a_diag, double dt, double Bx,
-                                                       double By, const double* rt0 = nullptr,
-                                                       double scal0 = 0.0) {
+                                                       double By) {
   constexpr int NV = 4 + NS;
   const double TOLF = 1.0e-10;
-  const double TOLX = kEps;
+  const int role = threadIdx.x & 3;
   double org[NV], rel[NV], rt[NV], old[NV], desc[NV];
-  double scal, scal_old;
-#pragma unroll
-  for (int i = 0; i < NV; i++) org[i] = fmax(fabs(qj[i]), 1.0e-3);
-#pragma unroll
-  for (int i = 0; i < NV; i++) rel[i] = qj[i] / org[i];
+  double scal = 0.0;
+  (void)newton_scale<NV>(qj, org, rel);
   NewtonOut out{0, 0, 0};
   int it;
-  bool fresh = false;
-  if (rt0) {
-    // residual at the starting point already evaluated by the caller
-#pragma unroll
-    for (int i = 0; i < NV; i++) rt[i] = rt0[i];
-    scal = scal0;
-    fresh = true;
-  }
-  bool jnext = false;       // J1n/J2n hold the Jacobian at the current point
-  double J1n[3], J2n[3];
+  bool fresh = false;  // rt and scal belong to qj, J1/J2 too
+  double J1[2] = {0.0, 0.0}, J2[2] = {0.0, 0.0};
   for (it = 1; it <= 100; it++) {
-    if (!fresh) eval_f<NS>(P, qj, qold, Rj, a_diag, dt, Bx, By, rt, scal);
-    bool restored = false;
-    double mf = 0.0;
+    if (!fresh) {
+      // the residual at qj (lane 2), the Jacobian at rel * org, which in the
+      // first iteration may be a rounding off qj (lanes 0, 1)
+      double q[NV], h1, h2;
 #pragma unroll
-    for (int i = 0; i < NV; i++) mf = fmax(mf, fabs(rt[i]));
-    if (mf < TOLF) {
+      for (int m = 0; m < NV; m++) q[m] = (role < 2) ? rel[m] * org[m] : qj[m];
+      quad_round<NS>(P, q, org, Bx, By, J1, J2, h1, h2);
+      finish_f<NS>(qj, qold, Rj, a_diag, dt, quad_from<NS>(h1, 2), quad_from<NS>(h2, 2), rt, scal);
+    }
+    bool restored = false;
+    if (max_abs<NV>(rt) < TOLF) {
       out.conv = 1;
       break;
     }
-    const double dta = dt * a_diag;
-    double J1[3], J2[3];
-    if (jnext) {
-      J1[1] = J1n[1];
-      J1[2] = J1n[2];
-      J2[1] = J2n[1];
-      J2[2] = J2n[2];
-    } else {
-      double q[NV], rdum[NV], sdum;
-#pragma unroll
-      for (int m = 0; m < NV; m++) q[m] = rel[m] * org[m];
-      quad_round<NS>(P, q, org, qold, Rj, a_diag, dt, Bx, By, false, J1, J2, rdum, sdum);
-    }
-    jnext = false;
-    const double zJ = 1.0 * 0.0 * P.one_by_h;
-    const double L11 = 1.0 * org[1] - dta * J1[1];
-    const double L21 = 0.0 - dta * J1[2];
-    const double L12 = 0.0 - dta * J2[1];
-    const double L22 = 1.0 * org[2] - dta * J2[2];
-    const double Lz = 0.0 - dta * zJ;
-    double d1[NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++) d1[i] = (i == 1 || i == 2) ? 0.0 : rt[i] / (1.0 * org[i]);
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++)
-      if (i != 1 && i != 2) s += d1[i] * 0.0;
-    double b1 = rt[1] - s, b2 = rt[2] - s;
-    {
-      double inv_det = 1.0 / (L11 * L22 - L21 * L12);
-      double x1 = (b1 * L22 - b2 * L12) * inv_det;
-      double x2 = (L11 * b2 - L21 * b1) * inv_det;
-#pragma unroll
-      for (int i = 0; i < NV; i++) {
-        if (i == 1) desc[i] = -x1 + 0.0;
-        else if (i == 2) desc[i] = -x2 + 0.0;
-        else desc[i] = 0.0 + -d1[i];
-      }
-    }
+    double L[4];
+    newton_step<NS>(org, rt, dt * a_diag, J1, J2, L, desc);
 #pragma unroll
     for (int i = 0; i < NV; i++) old[i] = rel[i];
-    scal_old = scal;
-    if (it > 1) {
-      double dd = 0.0;
+    LineSearch ls{};
+    if (it > 1) ls = ls_begin<NS>(org, old, rt, L, desc);
+    const double scal_old = scal;
+    if (!ls.none) {
+      double n1a, n2a;  // this lane's implicit terms
+      // trial `alam` from the implicit terms of lane `src`; returns true
+      // when the search ends with it (accepted, or below alamin)
+      bool acc = false;
+      auto take = [&](double alam, int src) -> bool {
+        const double h1 = quad_from<NS>(n1a, src), h2 = quad_from<NS>(n2a, src);
 #pragma unroll
-      for (int i = 0; i < NV; i++) dd += rel[i] * rel[i];
-      double stpmax = 100.0 * fmax(sqrt(dd), (double)NV);
-      double grad[NV];
+        for (int i = 0; i < NV; i++) rel[i] = old[i] + alam * desc[i];
 #pragma unroll
-      for (int i = 0; i < NV; i++) {
-        double g = 0.0;
-#pragma unroll
-        for (int r = 0; r < NV; r++) {
-          double Lri;
-          if (i == 1) Lri = (r == 1) ? L11 : (r == 2) ? L21 : Lz;
-          else if (i == 2) Lri = (r == 1) ? L12 : (r == 2) ? L22 : Lz;
-          else Lri = (r == i) ? 1.0 * org[i] : 0.0;
-          g += rt[r] * Lri;
+        for (int i = 0; i < NV; i++) qj[i] = rel[i] * org[i];
+        finish_f<NS>(qj, qold, Rj, a_diag, dt, h1, h2, rt, scal);
+        if (it == 1) {
+          acc = true;
+          return true;
         }
-        grad[i] = g;
-      }
-      double dabs = norm2_<NV>(desc);
-      if (dabs > stpmax) {
+        out.ls_evals++;
+        acc = scal <= 0.9 * scal_old;
+        if (acc) return true;
+        if (below_alamin<NV>(ls, alam, desc, old)) {
 #pragma unroll
-        for (int i = 0; i < NV; i++) desc[i] = desc[i] * stpmax / dabs;
-      }
-      double slope = 0.0;
-#pragma unroll
-      for (int i = 0; i < NV; i++) slope += grad[i] * desc[i];
-      double mx = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < NV; i++) {
-        double v = fabs(desc[i]) / fmax(fabs(old[i]), 1.0);
-        if (v > mx) mx = v;
-      }
-      double alamin = TOLX / mx;
-      if (alamin == 0.0) {
-#pragma unroll
-        for (int i = 0; i < NV; i++) rel[i] = old[i];
-      } else {
-        // lnsrch's trials: 1, then a2 = max(quadratic model, 0.5), then
-        // halvings (the cubic model is capped at half the last step, so
-        // max(tmplam, 0.5 * alam) is always 0.5 * alam).  Lane r of a batch
-        // evaluates one trial; the trials are then taken in order with the
-        // serial rules, so the accepted point and the count are the serial
-        // ones.  First batch: the Jacobian at trial 1 (lanes 0, 1), trial 1
-        // (lane 2), and the trial 0.5 that follows whenever a2 = 0.5 (lane 3).
-        const int role = threadIdx.x & 3;
-        double n1a, n2a;  // this lane's implicit terms (real parts)
-        {
-          const double al = (role == 3) ? 0.5 : 1.0;
-          const int pcol = (role == 0) ? 1 : (role == 1) ? 2 : -1;
-          cpx cq[NV];
-#pragma unroll
-          for (int m = 0; m < NV; m++) {
-            const double rm = old[m] + al * desc[m];
-            cq[m] = mk(rm * org[m], (m == pcol) ? P.h_cs * org[m] : 0.0);
-          }
-          cpx n1, n2;
-          implicit_c<NS>(P, cq, Bx, By, n1, n2);
-          const double a = 1.0 * n1.im * P.one_by_h, b = 1.0 * n2.im * P.one_by_h;
-          J1n[1] = quad_from<NS>(a, 0);
-          J1n[2] = quad_from<NS>(b, 0);
-          J2n[1] = quad_from<NS>(a, 1);
-          J2n[2] = quad_from<NS>(b, 1);
-          n1a = n1.re;
-          n2a = n2.re;
+          for (int i = 0; i < NV; i++) rel[i] = old[i];
+          scal = scal_old;
+          restored = true;
+          return true;
         }
-        // trial `alam` from the implicit terms of lane `src`; returns true
-        // when the search ends with it (accepted, or below alamin)
-        auto take = [&](double alam, int src, bool& accepted) -> bool {
-          const double h1 = quad_from<NS>(n1a, src), h2 = quad_from<NS>(n2a, src);
+        return false;
+      };
+      {
+        double q[NV];
+        const double al = (role == 3 && it > 1) ? 0.5 : 1.0;
+#pragma unroll
+        for (int m = 0; m < NV; m++) q[m] = (old[m] + al * desc[m]) * org[m];
+        quad_round<NS>(P, q, org, Bx, By, J1, J2, n1a, n2a);
+      }
+      bool end = take(1.0, 2);
+      fresh = end && acc;
+      if (!end) {
+        // max(quadratic model, 0.5), then halvings (see solve_rk_step), four
+        // at a time: lane r evaluates alam * 0.5^r, and the trials are taken
+        // in order with the serial rules
+        double alam = fmax(-fdiv(ls.slope, 2.0 * (scal - scal_old - ls.slope)), 0.5);
+        int trials = 1;
+        if (alam == 0.5) {
+          end = take(0.5, 3);
+          alam = 0.25;
+          trials++;
+        }
+        while (!end && trials < 256) {
+          double al = alam;
+#pragma unroll
+          for (int r = 0; r < 3; r++)
+            if (role > r) al = al * 0.5;
           double q[NV];
 #pragma unroll
-          for (int i = 0; i < NV; i++) rel[i] = old[i] + alam * desc[i];
-#pragma unroll
-          for (int i = 0; i < NV; i++) q[i] = rel[i] * org[i];
-          finish_f<NS>(q, qold, Rj, a_diag, dt, h1, h2, rt, scal);
-          out.ls_evals++;
-          accepted = scal <= 0.9 * scal_old;
-          if (accepted) return true;
-          if (alam < alamin) {
-#pragma unroll
-            for (int i = 0; i < NV; i++) rel[i] = old[i];
-            scal = scal_old;
-            restored = true;
-            return true;
-          }
-          return false;
-        };
-        bool acc = false;
-        bool end = take(1.0, 2, acc);
-        jnext = acc;
-        if (!end) {
-          const double tq = -(slope / (2.0 * (scal - scal_old - slope)));
-          double alam = fmax(tq, 0.5 * 1.0);
-          int trials = 1;
-          if (alam == 0.5) {
-            end = take(0.5, 3, acc);
-            alam = 0.25;
+          for (int m = 0; m < NV; m++) q[m] = (old[m] + al * desc[m]) * org[m];
+          ImplPt b;
+          implicit_real<NS>(P, q, Bx, By, b);
+          n1a = b.n1;
+          n2a = b.n2;
+          for (int r = 0; r < 4 && !end && trials < 256; r++) {
+            end = take(alam, r);
+            alam = alam * 0.5;
             trials++;
-          }
-          while (!end && trials < 256) {
-            // four halvings at once: lane r evaluates alam * 0.5^r
-            double al = alam;
-#pragma unroll
-            for (int r = 0; r < 3; r++)
-              if (role > r) al = al * 0.5;
-            {
-              cpx cq[NV];
-#pragma unroll
-              for (int m = 0; m < NV; m++) cq[m] = mk((old[m] + al * desc[m]) * org[m], 0.0);
-              cpx n1, n2;
-              implicit_c<NS>(P, cq, Bx, By, n1, n2);
-              n1a = n1.re;
-              n2a = n2.re;
-            }
-            for (int r = 0; r < 4 && !end && trials < 256; r++) {
-              end = take(alam, r, acc);
-              alam = alam * 0.5;
-              trials++;
-            }
           }
         }
       }
     } else {
-#pragma unroll
-      for (int i = 0; i < NV; i++) rel[i] = old[i] + desc[i];
-#pragma unroll
-      for (int i = 0; i < NV; i++) qj[i] = rel[i] * org[i];
-      // the residual and, speculatively, the Jacobian at the full step
-      quad_round<NS>(P, qj, org, qold, Rj, a_diag, dt, Bx, By, true, J1n, J2n, rt, scal);
-      jnext = true;
+      fresh = false;
     }
 #pragma unroll
     for (int i = 0; i < NV; i++) qj[i] = rel[i] * org[i];
-    fresh = !restored;
-    if (restored) jnext = false;
-    mf = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++) mf = fmax(mf, fabs(rt[i]));
-    if (mf < TOLF) {
-      out.conv = 1;
-      break;
-    }
-    double mx = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++) mx = fmax(mx, fabs(rel[i] - old[i]) / fmax(fabs(rel[i]), 1.0));
-    if (mx < TOLX) {
+    // an accepted shorter trial has its residual but not its Jacobian: the
+    // round at the top of the next iteration gives both (the same residual)
+    if (restored) fresh = false;
+    if (max_abs<NV>(rt) < TOLF || step_below_tolx<NV>(rel, old)) {
       out.conv = 1;
       break;
     }
@@ -725,34 +630,26 @@ __device__ __forceinline__ int stage2(const DevParams& P, const double* q0,
     // starts from it when it already meets the tolerance or has the smaller
     // residual of it and the plain predictor (the plain one stays the
     // fallback), and the equation solved is the same
-    double qw[NV], rtw[NV], rtp[NV], sw, sp = 0.0;
+    double qw[NV], rtw[NV], sw;
 #pragma unroll
     for (int i = 0; i < NV; i++) qw[i] = q_si[i];
     qw[1] = mg[0];
     qw[2] = mg[1];
     eval_f<NS>(P, qw, q0, Rj, 1.0, dt, Bx, By, rtw, sw);
-    double mfw = 0.0;
-#pragma unroll
-    for (int i = 0; i < NV; i++) mfw = fmax(mfw, fabs(rtw[i]));
-    bool use = mfw < 1.0e-10;
+    bool use = max_abs<NV>(rtw) < 1.0e-10;
     if (!use) {
+      double rtp[NV], sp;
       eval_f<NS>(P, q, q0, Rj, 1.0, dt, Bx, By, rtp, sp);
       use = sw < sp;
     }
     *warm_used = use ? 1 : 0;
-    if (use) {
-#pragma unroll
-      for (int i = 0; i < NV; i++) q[i] = qw[i];
-    }
-    no = (LANES == 4)
-             ? solve_rk_step_quad<NS>(P, q, q0, Rj, 1.0, dt, Bx, By, use ? rtw : rtp,
-                                      use ? sw : sp)
-             : solve_rk_step<NS>(P, q, q0, Rj, 1.0, dt, Bx, By, use ? rtw : rtp, use ? sw : sp);
-  } else {
-    if (warm_used) *warm_used = (closed || warm) ? 0 : -1;
-    no = (LANES == 4) ? solve_rk_step_quad<NS>(P, q, q0, Rj, 1.0, dt, Bx, By)
-                      : solve_rk_step<NS>(P, q, q0, Rj, 1.0, dt, Bx, By);
+    q[1] = use ? qw[1] : q[1];
+    q[2] = use ? qw[2] : q[2];
+  } else if (warm_used) {
+    *warm_used = (closed || warm) ? 0 : -1;
   }
+  no = (LANES == 4) ? solve_rk_step_quad<NS>(P, q, q0, Rj, 1.0, dt, Bx, By)
+                    : solve_rk_step<NS>(P, q, q0, Rj, 1.0, dt, Bx, By);
   nonconv = !no.conv;
   ls_evals = no.ls_evals;
   if (harvest && no.conv) {

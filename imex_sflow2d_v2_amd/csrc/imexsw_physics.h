@@ -634,6 +634,171 @@ __device__ __forceinline__ void implicit_c(const DevParams& P, const cpx* cq,
   }
 }
 
+// ---------------------------------------------------------------------------
+// The implicit terms and their complex-step derivatives without complex
+// arithmetic.  Every argument of implicit_c but one momentum is real in the
+// Newton solve, so the mixture chain (q1, the mass fractions, the heat
+// capacities) carries zero imaginary parts, and the imaginary part of the
+// perturbed momentum is of the order of the rounding unit: its square
+// vanishes in every real part.  implicit_real evaluates the real chain once;
+// implicit_col propagates the imaginary parts of one column through it,
+// operation for operation as implicit_c does, with the real chain's
+// reciprocals.  Both give implicit_c's bits.  implicit_col verifies that the
+// squares did vanish (exactly where the rounded sum can be compared, else by
+// a relative size below 2^-28 of the imaginary part) and returns false where
+// they did not (a state at rest, or nearly so): the caller then takes
+// implicit_c.
+//
+// What it replaces: three evaluations of implicit_c per Newton iteration,
+// each about 21 divisions and two square roots on Smith's quotient (two
+// dependent divisions each), were some 90 % of the stage update.  Now one
+// chain of 6 reciprocals and 9 quotients and, per column, 11 quotients of 4
+// instructions each.
+// ---------------------------------------------------------------------------
+struct ImplPt {
+  double n1, n2;  // the implicit momentum terms
+  bool moving;    // n1, n2 come from the friction law (else zero)
+  bool heat;      // the temperature depends on the momenta
+  bool thin;      // desingularised velocities (q1 <= eps_sing)
+  double inv_q1, u, v, w, s2, mvh2, mv2, turb;
+  double xc, rgc, irm, rho, dr, rg, m, mx;
+  double thin_f;  // q1 sqrt(2)
+  Rcp rT, rirm, rrho, rmv, rthin;
+};
+
+template <int NS, int RM = 1>
+__device__ __forceinline__ void implicit_real(const DevParams& P, const double* q, double Bx,
+                                              double By, ImplPt& b) {
+  b.n1 = 0.0;
+  b.n2 = 0.0;
+  b.moving = false;
+  if (!P.rheo || (RM == 1 && P.rheo_model != 1) || !(q[0] > kEps)) return;
+  const Rcp rq = rcp_of(q[0]);
+  b.inv_q1 = div_by(1.0, rq);
+  double xs_tot = 0.0, dsh = 0.0, dinv = 0.0;
+#pragma unroll
+  for (int i = 0; i < NS; i++) {
+    const double xs = q[4 + i] * b.inv_q1;
+    xs_tot = xs_tot + xs;
+    dsh = dsh + xs * P.sp_heat_s[i];
+    dinv = dinv + xs * P.inv_rho_s[i];
+  }
+  b.xc = 1.0 - xs_tot;
+  const Rcp rxc = rcp_of(b.xc);
+  const double shc = div_by(b.xc * P.sp_heat_a, rxc);
+  b.rgc = div_by(b.xc * P.sp_gas_const_a, rxc);
+  const double shm = dsh + b.xc * shc;
+  b.s2 = q[1] * q[1] + q[2] * q[2];
+  b.thin = !(q[0] > P.eps_sing);
+  b.rT = rcp_of(q[0] * shm);
+  const double A = P.energy ? q[3] - (b.s2 * 0.5) * b.inv_q1 : q[3];
+  double T = div_by(A, b.rT);
+  const bool clamp = b.thin || T <= 0.0;
+  T = clamp ? P.T_ambient : T;
+  b.heat = P.energy && !clamp;
+  b.irm = dinv + b.xc * ((b.rgc * T) * P.inv_pres);
+  b.rirm = rcp_of(b.irm);
+  b.rho = div_by(1.0, b.rirm);
+  b.thin_f = q[0] * sqrt(2.0);
+  if (b.thin) {
+    const double q1sq = q[0] * q[0];
+    b.rthin = rcp_of(fsqrt(q1sq * q1sq + P.eps_sing4));
+    b.u = div_by(b.thin_f * q[1], b.rthin);
+    b.v = div_by(b.thin_f * q[2], b.rthin);
+  } else {
+    b.rthin = Rcp{1.0, 1.0};
+    b.u = q[1] * b.inv_q1;
+    b.v = q[2] * b.inv_q1;
+  }
+  b.w = P.slope ? b.u * Bx + b.v * By : 0.0;
+  b.mvh2 = b.u * b.u + b.v * b.v;
+  b.mv2 = b.mvh2 + b.w * b.w;
+  if (b.mv2 == 0.0) return;
+  b.moving = true;
+  if (RM == 6) {
+    b.rmv = rcp_of(fsqrt(b.mvh2));
+    b.n1 = 0.0 - ((b.rho * div_by(b.u, b.rmv)) * P.ff) * b.mv2;
+    b.n2 = 0.0 - ((b.rho * div_by(b.v, b.rmv)) * P.ff) * b.mv2;
+  } else {
+    b.dr = b.rho - P.rho_a_amb;
+    b.rrho = rcp_of(b.rho);
+    b.rg = div_by(b.dr, b.rrho) * P.grav;
+    b.m = b.rho * b.rg;
+    b.mx = fdiv(b.m, P.xi);
+    b.turb = b.mx * b.mv2;
+    b.rmv = rcp_of(fsqrt(b.mv2));
+    b.n1 = 0.0 - b.turb * div_by(b.u, b.rmv);
+    b.n2 = 0.0 - b.turb * div_by(b.v, b.rmv);
+  }
+}
+
+// Imaginary parts of the implicit terms at the point of `b` when the momenta
+// q[1], q[2] carry the imaginary parts d1, d2 (one of them zero).
+template <int RM = 1>
+__device__ __forceinline__ bool implicit_col(const DevParams& P, const ImplPt& b, double q1,
+                                             double q2, double d1, double d2, double Bx,
+                                             double By, double& n1i, double& n2i) {
+  constexpr double kTiny = 3.7252902984619140625e-9;  // 2^-28
+  // velocities and their squares
+  const double du = b.thin ? div_by(b.thin_f * d1, b.rthin) : d1 * b.inv_q1;
+  const double dv = b.thin ? div_by(b.thin_f * d2, b.rthin) : d2 * b.inv_q1;
+  const double dw = P.slope ? du * Bx + dv * By : 0.0;
+  const double mvh2c = (b.u * b.u - du * du) + (b.v * b.v - dv * dv);
+  const double mv2c = mvh2c + (b.w * b.w - dw * dw);
+  const double mvh2i = (b.u * du + du * b.u) + (b.v * dv + dv * b.v);
+  const double mv2i = mvh2i + (b.w * dw + dw * b.w);
+  bool ok = b.moving && mv2c == b.mv2;
+  // temperature, density
+  const double s2c = (q1 * q1 - d1 * d1) + (q2 * q2 - d2 * d2);
+  ok = ok && s2c == b.s2;
+  const double s2i = (q1 * d1 + d1 * q1) + (q2 * d2 + d2 * q2);
+  const double Ti = b.heat ? div_by(0.0 - (s2i * 0.5) * b.inv_q1, b.rT) : 0.0;
+  const double irmi = b.xc * ((b.rgc * Ti) * P.inv_pres);
+  ok = ok && fabs(irmi) <= kTiny * b.irm;
+  const double rhoi = div_by(-div_by(irmi, b.rirm), b.rirm);
+  if (RM == 6) {
+    ok = ok && mvh2c == b.mvh2 && fabs(mvh2i) <= kTiny * b.mvh2;
+    const double mi = 0.5 * div_by(mvh2i, b.rmv);  // of the speed |(u, v)|
+    const double ra = div_by(mi, b.rmv);
+    const double er = div_by(du * ra + b.u, b.rmv), ei = div_by(du - b.u * ra, b.rmv);
+    const double fr = div_by(dv * ra + b.v, b.rmv), fi = div_by(dv - b.v * ra, b.rmv);
+    const double p1r = (b.rho * er - rhoi * ei) * P.ff, p1i = (b.rho * ei + rhoi * er) * P.ff;
+    const double p2r = (b.rho * fr - rhoi * fi) * P.ff, p2i = (b.rho * fi + rhoi * fr) * P.ff;
+    n1i = 0.0 - (p1r * mv2i + p1i * b.mv2);
+    n2i = 0.0 - (p2r * mv2i + p2i * b.mv2);
+    return ok;
+  }
+  ok = ok && fabs(mv2i) <= kTiny * b.mv2;
+  const double rr = div_by(rhoi, b.rrho);
+  ok = ok && rhoi * rr + b.dr == b.dr;
+  const double rgi = div_by(rhoi - b.dr * rr, b.rrho) * P.grav;
+  ok = ok && b.m - rhoi * rgi == b.m;
+  const double mxi = fdiv(b.rho * rgi + rhoi * b.rg, P.xi);
+  ok = ok && b.turb - mxi * mv2i == b.turb;
+  const double ti = b.mx * mv2i + mxi * b.mv2;
+  const double mi = 0.5 * div_by(mv2i, b.rmv);
+  const double ra = div_by(mi, b.rmv);
+  const double er = div_by(du * ra + b.u, b.rmv), ei = div_by(du - b.u * ra, b.rmv);
+  const double fr = div_by(dv * ra + b.v, b.rmv), fi = div_by(dv - b.v * ra, b.rmv);
+  n1i = 0.0 - (b.turb * ei + ti * er);
+  n2i = 0.0 - (b.turb * fi + ti * fr);
+  return ok;
+}
+
+// the same from implicit_c, for the points implicit_col leaves
+template <int NS, int RM = 1>
+__device__ __forceinline__ void implicit_col_c(const DevParams& P, const double* q, double d1,
+                                               double d2, double Bx, double By, double& n1i,
+                                               double& n2i) {
+  constexpr int NV = 4 + NS;
+  cpx cq[NV], n1, n2;
+#pragma unroll
+  for (int m = 0; m < NV; m++) cq[m] = mk(q[m], (m == 1) ? d1 : (m == 2) ? d2 : 0.0);
+  implicit_c<NS, RM>(P, cq, Bx, By, n1, n2);
+  n1i = n1.im;
+  n2i = n2.im;
+}
+
 // eval_source_bdry (src/constitutive_2d.f90:5024-5130), split into the
 // time factors (the same for every ring cell of a step) and the per-cell
 // part that scales them by the cell's direction vector
