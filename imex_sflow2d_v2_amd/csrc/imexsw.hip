@@ -596,6 +596,8 @@ int imexsw_create(const imexsw_params* params, imexsw_ctx** out) {
   P.lim_c = 0;
   for (int i = 0; i < IMEXSW_MAX_VARS + 2; i++)
     P.lim_c |= (p.limiter[i] >= 3 && p.limiter[i] <= 5) ? 1 : 0;
+  P.lim_1 = 1;
+  for (int i = 0; i < c->nv + 2; i++) P.lim_1 &= (p.limiter[i] == 1) ? 1 : 0;
   for (int s = 0; s < 4; s++)
     for (int i = 0; i < IMEXSW_MAX_VARS; i++) {
       P.bc_flag[s][i] = p.bc_flag[s][i];
@@ -1487,7 +1489,7 @@ void drop_graph(imexsw_ensemble* e) {
   if (e->graph) (void)hipGraphDestroy(e->graph);
   e->exec = nullptr;
   e->graph = nullptr;
-  e->graph_strip_h = 0;
+  e->graph_strip_h = -1;
 }
 
 // graph of graph_steps batched steps (kernels only: no memset nodes)

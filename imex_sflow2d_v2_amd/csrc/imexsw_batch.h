@@ -61,13 +61,15 @@ __global__ void __launch_bounds__(64 * kMaskGroup) kb_mask(const DevParams* __re
   append_group<kMaskGroup>(sink, t, rows_m);
 }
 
-// (tile, strip) items of all members, strip height fixed for the batch
+// (tile, strip) items of all members; strip_h 0: the height that strip_fit
+// finds for the step's listed rows
 template <int NS>
 __global__ void __launch_bounds__(64) kb_stencil(const DevParams* __restrict__ Ps,
                                                  const DevPtrs* __restrict__ Ds, BatchLists L,
                                                  int strip_h) {
-  const int per = kTileH / strip_h;
   const int n = (int)L.counts[0];
+  if (strip_h == 0) strip_h = strip_fit((int)L.counts[1], gridDim.x, kTileH);
+  const int per = kTileH / strip_h;
   for (int item = blockIdx.x; item < n * per; item += gridDim.x) {
     const int e = L.tiles[item / per];
     const int m = e >> kMemberShift, tile = e & kIdMask;

@@ -24,6 +24,9 @@ using imexsw::RkTableau;
 
 enum KernelId { K_MASK = 0, K_STENCIL, K_LOCAL, K_TOPO, K_DTPOLICY, K_POST, K_EROSION, K_NK };
 
+// default number of strips wanted in flight (imexsw_set_tuning)
+constexpr int kDefaultStrips = 2048;
+
 struct imexsw_ctx {
   imexsw_params p{};
   DevParams P{};
@@ -40,7 +43,7 @@ struct imexsw_ctx {
   int device = 0;   // the HIP device current at imexsw_create
   int strip_h = 16;         // tallest stencil strip (rows)
   int row_unit = 1;         // shortest stencil strip (rows)
-  int target_strips = 2048; // strips wanted in flight
+  int target_strips = kDefaultStrips; // strips wanted in flight
   // N_RK != 2: the tableau-driven stage pipeline and its stage planes
   bool general = false;
   RkTableau tab{};
@@ -94,11 +97,11 @@ struct imexsw_ensemble {
   unsigned long long* d_counts = nullptr;
   int total_tiles = 0;
   int n_cu = 256;
-  int strip_h = 8;
+  int strip_h = 0;  // 0: chosen each step on the device (strip_fit)
   int graph_steps = 25;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  int graph_strip_h = 0;
+  int graph_strip_h = -1;
   double last_ms = 0.0;
 };
 

@@ -181,6 +181,29 @@ __device__ __forceinline__ double shfl_d(double v, int src) {
   return __hiloint2double(hi, lo);
 }
 
+// a wavefront-uniform value in scalar registers
+__device__ __forceinline__ double uniform(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+__device__ __forceinline__ SrcTime uniform(const SrcTime& T) {
+  return SrcTime{(bool)__builtin_amdgcn_readfirstlane((int)T.off), uniform(T.tc), uniform(T.p15),
+                 uniform(T.p05)};
+}
+
+// v of the lane to the left / right (lanes 0 and 63 wrap around): whole-wave
+// DPP rotations, one VALU move per half instead of a trip through LDS
+__device__ __forceinline__ double lane_left(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x13c, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x13c, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane_right(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x134, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x134, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
 // ---------------------------------------------------------------------------
 // k_mask: check_solve (src/solver_2d.f90:666-857), one wavefront per work
 // tile and kMaskGroup tiles (stacked along y) per workgroup.  Lane l reads
@@ -489,30 +512,78 @@ __device__ __forceinline__ SrcInfo src_info(int b) {
   return S;
 }
 
+// What a cell's reconstruction needs of the radial source: its flags, and
+// the time factors and direction vector its boundary state is formed from
+// (where a reconstruction needs it; few wavefronts do)
+struct Ring {
+  SrcInfo S;
+  SrcTime T;
+  double v0, v1;
+};
+// component i of the boundary state of a ring cell (zero elsewhere),
+// src/solver_2d.f90:3879-3889
+template <int NS>
+__device__ __forceinline__ double ring_value(const DevParams& P, const Ring& r, int i) {
+  return (P.radial && r.S.src2 && r.S.dir) ? source_bdry<NS>(P, r.T, r.v0, r.v1, i) : 0.0;
+}
+
 __device__ __forceinline__ void qp2_uv(const double* qp, double& u, double& v) {
   // qp_to_qp2 (src/constitutive_2d.f90:2155-2179), velocity components
   if (qp[0] <= 0.0) {
     u = 0.0;
     v = 0.0;
   } else {
-    u = qp[1] / qp[0];
-    v = qp[2] / qp[0];
+    const Rcp r = rcp_of(qp[0]);
+    u = div_by(qp[1], r);
+    v = div_by(qp[2], r);
   }
 }
 
 // DIR 1: x (lo = west face value qrecW, hi = east qrecE); DIR 2: y (S, N).
 // c = own physical state, m / p = neighbours at index-1 / index+1 along DIR
 // (not read at a domain boundary), idx / n = position and extent along DIR,
-// other = position along the other direction, sb = source boundary state,
+// other = position along the other direction, ring = the cell's source data,
 // typo = the x_stencil(3) = y_stag(k+1) substitution of src/solver_2d.f90:
 // 3616 that reaches the x-slope of v.
+template <int DIR>
+__device__ __forceinline__ double stag_at(const DevParams& P, int i) {
+  return (DIR == 1) ? xstag(P, i) : ystag(P, i);
+}
+template <int DIR>
+__device__ __forceinline__ double comp_at(const DevParams& P, int i) {
+  return (DIR == 1) ? xcomp(P, i) : ycomp(P, i);
+}
+// the limited slope of variable i from its operands v0, c, v2 and the
+// reciprocals of the abscissa differences, which all variables share (rc: of
+// z2 - z0, for the limiters that use the centred difference)
+__device__ __forceinline__ double lim_slope(const DevParams& P, double v0, double c, double v2,
+                                            const Rcp& r0, const Rcp& r2, const Rcp& rc, int i) {
+  return limit_pick(P, div_by(v2 - c, r2), div_by(c - v0, r0),
+                    P.lim_c ? div_by(v2 - v0, rc) : 0.0, P.limiter[i]);
+}
+// the slopes of variables I0 .. I1-1 (all minmod: no branch between them)
+template <int I0, int I1>
+__device__ __forceinline__ void lim_slopes(const DevParams& P, const double* v0, const double* c,
+                                           const double* v2, const Rcp& r0, const Rcp& r2,
+                                           const Rcp& rc, double* slope) {
+  if (P.lim_1) {
+#pragma unroll
+    for (int i = I0; i < I1; i++)
+      slope[i] = minmod_(div_by(v2[i] - c[i], r2), div_by(c[i] - v0[i], r0));
+  } else {
+#pragma unroll
+    for (int i = I0; i < I1; i++) slope[i] = lim_slope(P, v0[i], c[i], v2[i], r0, r2, rc, i);
+  }
+}
+
+// the cells at a domain boundary, on the source ring and with `typo`
 template <int NS, int DIR>
-__device__ __forceinline__ void recon(const DevParams& P, const double* c,
-                                      const double* m, const double* p, int idx,
-                                      int n, int other, const SrcInfo S,
-                                      const double* sb, bool typo, double* lo,
-                                      double* hi) {
+__device__ __forceinline__ void recon_edge(const DevParams& P, const double* c,
+                                           const double* m, const double* p, int idx, int n,
+                                           int other, const Ring& ring, bool typo, double* lo,
+                                           double* hi) {
   constexpr int NV = 4 + NS;
+  const SrcInfo S = ring.S;
   const int side_lo = (DIR == 1) ? IMEXSW_W : IMEXSW_S;
   const int side_hi = (DIR == 1) ? IMEXSW_E : IMEXSW_N;
   const double one_by = (DIR == 1) ? P.one_by_dx : P.one_by_dy;
@@ -523,145 +594,148 @@ __device__ __forceinline__ void recon(const DevParams& P, const double* c,
   const bool srcb = (DIR == 1) && S.src2;
   const bool ovr_lo = (DIR == 1) ? (radial2 && !S.sE && S.sW) : (radial2 && S.sS);
   const bool ovr_hi = (DIR == 1) ? (radial2 && S.sE) : (radial2 && !S.sS && S.sN);
-  auto stag = [&](int i) { return (DIR == 1) ? xstag(P, i) : ystag(P, i); };
-  auto comp = [&](int i) { return (DIR == 1) ? xcomp(P, i) : ycomp(P, i); };
   // stencil abscissae left by the loop over the conservative variables
-  double z0, z2;
-  const double z1 = comp(idx);
+  double z0 = comp_at<DIR>(P, idx - 1), z2 = comp_at<DIR>(P, idx + 1);
+  const double z1 = comp_at<DIR>(P, idx);
   if (first) {
-    z0 = stag(0);
-    z2 = comp(idx + 1);
+    z0 = stag_at<DIR>(P, 0);
   } else if (last) {
-    z0 = comp(idx - 1);
-    z2 = stag(n);
+    z2 = stag_at<DIR>(P, n);
   } else {
-    z0 = ovr_lo ? stag(idx) : comp(idx - 1);
-    z2 = ovr_hi ? stag(idx + 1) : comp(idx + 1);
+    z0 = ovr_lo ? stag_at<DIR>(P, idx) : z0;
+    z2 = ovr_hi ? stag_at<DIR>(P, idx + 1) : z2;
   }
-  (void)other;
-  // the limiter's operands of every variable, then all their divisions
-  // (no branch between them), then the limiter and the boundary cases per
-  // variable: the values of limit_ on the same operands
-  double v0[NV], v2[NV], A[NV], B[NV], C[NV];
+  const Rcp r2 = rcp_of(z2 - z1), r0 = rcp_of(z1 - z0);
+  Rcp rc{1.0, 1.0};
+  if (P.lim_c) rc = rcp_of(z2 - z0);
+  const bool inner_lo = !first && !last && ovr_lo, inner_hi = !first && !last && ovr_hi;
+  const double cd = P.reconstr_coeff * d2;
+  const bool any_ring = P.radial && __any(ring.S.src2);
+  double v0[NV + 2], v2[NV + 2], slope[NV + 2];
 #pragma unroll
-  for (int i = 0; i < NV; i++) {
-    // the candidates in registers first: a choice between two addresses
-    // (of the argument block, or of two of the caller's arrays) would move
-    // the arrays to scratch memory
-    double blo = P.bc_value[side_lo][i], bhi = P.bc_value[side_hi][i];
-    double sbi = sb[i], mi = m[i], pi = p[i];
-    pin(blo);
-    pin(bhi);
-    pin(sbi);
-    pin(mi);
-    pin(pi);
-    if (first) {
-      v0[i] = srcb ? sbi : blo;
-      v2[i] = pi;
-    } else if (last) {
-      v0[i] = mi;
-      v2[i] = srcb ? sbi : bhi;
-    } else {
-      v0[i] = ovr_lo ? sbi : mi;
-      v2[i] = ovr_hi ? sbi : pi;
+  for (int i = 0; i < NV + 2; i++) {
+    v0[i] = m[i];
+    v2[i] = p[i];
+  }
+  if (any_ring) {
+#pragma unroll
+    for (int i = 0; i < NV + 2; i++) {
+      const double sb = ring_value<NS>(P, ring, i);
+      v0[i] = inner_lo ? sb : v0[i];
+      v2[i] = inner_hi ? sb : v2[i];
+    }
+  }
+  const bool any_end = __any(first || last);
+  if (any_end) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      const double sb = ring_value<NS>(P, ring, i);
+      if (first) v0[i] = srcb ? sb : P.bc_value[side_lo][i];
+      else if (last) v2[i] = srcb ? sb : P.bc_value[side_hi][i];
+    }
+  }
+  lim_slopes<0, NV>(P, v0, c, v2, r0, r2, rc, slope);
+  if (any_end && !srcb) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      const int fl = P.bc_flag[side_lo][i], fh = P.bc_flag[side_hi][i];
+      if (first && fl != 0)
+        slope[i] = (fl == 1) ? P.bc_value[side_lo][i] : (fl == 2) ? (p[i] - c[i]) * one_by : 0.0;
+      else if (!first && last && fh != 0)
+        slope[i] = (fh == 1) ? P.bc_value[side_hi][i] : (fh == 2) ? (c[i] - m[i]) * one_by : 0.0;
     }
   }
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    A[i] = (v2[i] - c[i]) / (z2 - z1);
-    B[i] = (c[i] - v0[i]) / (z1 - z0);
+    const double dq = cd * slope[i];
+    lo[i] = c[i] - dq;
+    hi[i] = c[i] + dq;
   }
+  // u and v with the limiters of hu and hv (:3496-3661), on the boundary from
+  // the face values of h, hu, hv just formed
+  double bu = 0.0, bw = 0.0;
+  if (any_end) {
 #pragma unroll
-  for (int i = 0; i < NV; i++) C[i] = 0.0;
-  if (P.lim_c) {
-#pragma unroll
-    for (int i = 0; i < NV; i++) C[i] = (v2[i] - v0[i]) / (z2 - z0);
-  }
-#pragma unroll
-  for (int i = 0; i < NV; i++) {
-    const double s1 = c[i];
-    const double lim_slope = limit_pick(P, A[i], B[i], C[i], P.limiter[i]);
-    double slope = lim_slope;
+    for (int i = 0; i < NV; i++) {
+      const double sb = ring_value<NS>(P, ring, i);
+      if (first) {
+        if (srcb) lo[i] = sb;
+        else if (P.bc_flag[side_lo][i] == 0) lo[i] = P.bc_value[side_lo][i];
+        else if (i == DIR) lo[i] = fmin(lo[i], 0.0);
+      }
+      if (last) {
+        if (srcb) hi[i] = sb;
+        else if (P.bc_flag[side_hi][i] == 0) hi[i] = P.bc_value[side_hi][i];
+        else if (i == DIR) hi[i] = fmax(hi[i], 0.0);
+      }
+    }
     if (first) {
-      const int f = P.bc_flag[side_lo][i];
-      const double bv = P.bc_value[side_lo][i];
-      if (!srcb && f != 0) slope = (f == 1) ? bv : (f == 2) ? (p[i] - s1) * one_by : 0.0;
+      qp2_uv(lo, bu, bw);
+      v0[NV] = bu;
+      v0[NV + 1] = bw;
     } else if (last) {
-      const int f = P.bc_flag[side_hi][i];
-      const double bv = P.bc_value[side_hi][i];
-      if (!srcb && f != 0) slope = (f == 1) ? bv : (f == 2) ? (s1 - m[i]) * one_by : 0.0;
-    }
-    const double dq = P.reconstr_coeff * d2 * slope;
-    lo[i] = s1 - dq;
-    hi[i] = s1 + dq;
-    if (first) {
-      const int f = P.bc_flag[side_lo][i];
-      if (srcb) lo[i] = sb[i];
-      else if (f == 0) lo[i] = P.bc_value[side_lo][i];
-      else if (i == DIR) lo[i] = fmin(lo[i], 0.0);
-    }
-    if (last) {
-      const int f = P.bc_flag[side_hi][i];
-      if (srcb) hi[i] = sb[i];
-      else if (f == 0) hi[i] = P.bc_value[side_hi][i];
-      else if (i == DIR) hi[i] = fmax(hi[i], 0.0);
+      qp2_uv(hi, bu, bw);
+      v2[NV] = bu;
+      v2[NV + 1] = bw;
     }
   }
-  // u and v with the limiters of hu and hv (:3496-3661), from the face
-  // values of h, hu, hv just formed when the cell is on the boundary
-  double ul = 0.0, wl = 0.0, uh = 0.0, wh = 0.0;
-  if (first) qp2_uv(lo, ul, wl);
-  if (last) qp2_uv(hi, uh, wh);
-  double u0[2], u2v[2], zz2[2], UA[2], UB[2], UC[2];
+  lim_slopes<NV, NV + 2>(P, v0, c, v2, r0, r2, rc, slope);
+  if (DIR == 1 && typo) {
+    // the substituted abscissa of the x-slope of v
+    constexpr int i = NV + 1;
+    const double zt = (!first && !last && radial2 && S.sE) ? stag_at<DIR>(P, idx + 1)
+                                                            : ystag(P, other + 1);
+    slope[i] = limit_pick(P, fdiv(v2[i] - c[i], zt - z1), div_by(c[i] - v0[i], r0),
+                          P.lim_c ? fdiv(v2[i] - v0[i], zt - z0) : 0.0, P.limiter[i]);
+  }
 #pragma unroll
-  for (int r = 0; r < 2; r++) {
-    const int i = NV + r;
-    zz2[r] = z2;
-    if (DIR == 1 && i == NV + 1 && typo)
-      zz2[r] = (!first && !last && radial2 && S.sE) ? stag(idx + 1) : ystag(P, other + 1);
-    double sbi = sb[i], mi = m[i], pi = p[i];
-    pin(sbi);
-    pin(mi);
-    pin(pi);
-    if (first) {
-      u0[r] = (r == 0) ? ul : wl;
-      u2v[r] = pi;
-    } else if (last) {
-      u0[r] = mi;
-      u2v[r] = (r == 0) ? uh : wh;
-    } else {
-      u0[r] = ovr_lo ? sbi : mi;
-      u2v[r] = ovr_hi ? sbi : pi;
+  for (int i = NV; i < NV + 2; i++) {
+    const double dq = cd * slope[i];
+    lo[i] = first ? (i == NV ? bu : bw) : c[i] - dq;
+    hi[i] = (!first && last) ? (i == NV ? bu : bw) : c[i] + dq;
+  }
+  if (any_ring) {
+#pragma unroll
+    for (int i = 0; i < NV + 2; i++) {
+      const double sb = ring_value<NS>(P, ring, i);
+      lo[i] = (inner_lo && !ovr_hi) ? sb : lo[i];
+      hi[i] = inner_hi ? sb : hi[i];
     }
   }
-#pragma unroll
-  for (int r = 0; r < 2; r++) {
-    UA[r] = (u2v[r] - c[NV + r]) / (zz2[r] - z1);
-    UB[r] = (c[NV + r] - u0[r]) / (z1 - z0);
-    UC[r] = 0.0;
+}
+
+// A wavefront without a lane at a boundary or on the ring takes the interior
+// form, free of the cases' selects; any other takes recon_edge, which gives an
+// interior lane the same values.
+template <int NS, int DIR>
+__device__ __forceinline__ void recon(const DevParams& P, const double* c,
+                                      const double* m, const double* p, int idx,
+                                      int n, int other, const Ring& ring,
+                                      bool typo, double* lo, double* hi) {
+  constexpr int NV = 4 + NS;
+  if (__any(idx == 0 || idx == n - 1 || (P.radial && ring.S.src2))) {
+    recon_edge<NS, DIR>(P, c, m, p, idx, n, other, ring, typo, lo, hi);
+    return;
   }
-  if (P.lim_c) {
+  const double z0 = comp_at<DIR>(P, idx - 1), z1 = comp_at<DIR>(P, idx),
+               z2 = comp_at<DIR>(P, idx + 1);
+  const Rcp r2 = rcp_of(z2 - z1), r0 = rcp_of(z1 - z0);
+  Rcp rc{1.0, 1.0};
+  if (P.lim_c) rc = rcp_of(z2 - z0);
+  const double cd = P.reconstr_coeff * ((DIR == 1) ? P.dx2 : P.dy2);
+  if (P.lim_1) {
 #pragma unroll
-    for (int r = 0; r < 2; r++) UC[r] = (u2v[r] - u0[r]) / (zz2[r] - z0);
-  }
+    for (int i = 0; i < NV + 2; i++) {
+      const double dq = cd * minmod_(div_by(p[i] - c[i], r2), div_by(c[i] - m[i], r0));
+      lo[i] = c[i] - dq;
+      hi[i] = c[i] + dq;
+    }
+  } else {
 #pragma unroll
-  for (int r = 0; r < 2; r++) {
-    const int i = NV + r;
-    const double s1 = c[i];
-    const double slope = limit_pick(P, UA[r], UB[r], UC[r], P.limiter[i]);
-    const double dq = P.reconstr_coeff * d2 * slope;
-    lo[i] = s1 - dq;
-    hi[i] = s1 + dq;
-    if (first) lo[i] = (r == 0) ? ul : wl;
-    else if (last) hi[i] = (r == 0) ? uh : wh;
-  }
-  if (!first && !last) {
-    if (ovr_hi) {
-#pragma unroll
-      for (int i = 0; i < NV + 2; i++) hi[i] = sb[i];
-    } else if (ovr_lo) {
-#pragma unroll
-      for (int i = 0; i < NV + 2; i++) lo[i] = sb[i];
+    for (int i = 0; i < NV + 2; i++) {
+      const double dq = cd * lim_slope(P, m[i], c[i], p[i], r0, r2, rc, i);
+      lo[i] = c[i] - dq;
+      hi[i] = c[i] + dq;
     }
   }
 }
@@ -700,22 +774,120 @@ __device__ __noinline__ void make_side_vp(const DevParams& P, const double* qp, 
   make_side_vp_body<NS, DIR>(P, qp, gc, bx, by, s);
 }
 
-// (VP: bx, by are the slope of the cell the state belongs to, read by the
-// profile flux coefficients)
-template <int NS, int DIR, bool VP = false>
-__device__ __forceinline__ void make_side(const DevParams& P, const double* qp,
-                                          double gc, Side<NS>& s, double bx = 0.0,
-                                          double by = 0.0) {
-  if (VP) {
-    make_side_vp<NS, DIR>(P, qp, gc, bx, by, &s);
-    return;
+// A face side without the profiles: its fluxes are its velocity times its
+// conservative values (and the pressure), so they are formed at the face
+// (expand) instead of being carried there.
+template <int NS>
+struct LeanSide {
+  double qc[4 + NS];
+  double vel, pt, vmin, vmax, zv;
+};
+
+// qp2qc, fluxes and speeds (imexsw_physics.h) with the mixture formed once,
+// without branches (a dry state's values selected): the same operations
+template <int NS, int DIR>
+__device__ __forceinline__ void make_side(const DevParams& P, const double* qp, double gc,
+                                          LeanSide<NS>& s, double = 0.0, double = 0.0) {
+  constexpr int NV = 4 + NS;
+  const bool wet = qp[0] > kEps;
+  const double h = qp[0], u = qp[NV], v = qp[NV + 1], T = qp[3];
+  double ars[NS > 0 ? NS : 1], at = 0.0, sar = 0.0;
+  const Rcp rh = rcp_of(h);
+#pragma unroll
+  for (int i = 0; i < NS; i++) {
+    const double al = P.alpha ? qp[4 + i] : div_by(qp[4 + i], rh);
+    at += al;
+    ars[i] = al * P.rho_s[i];
   }
-  qp2qc<NS>(P, qp, s.qc);
-  fluxes<NS, DIR>(P, s.qc, qp, gc, s.f);
-  speeds<NS, DIR>(P, qp, gc, s.vmin, s.vmax);
+#pragma unroll
+  for (int i = 0; i < NS; i++) sar += ars[i];
+  const double alphac = 1.0 - at;
+  const double rho_c = fdiv(alphac * fdiv(P.pres, P.sp_gas_const_a * T), alphac);
+  const double ac_rho = alphac * rho_c;
+  const double rho_m = ac_rho + sar;
+  const Rcp rr = rcp_of(rho_m);
+  const double inv_rhom = div_by(1.0, rr);
+  double rg = div_by(rho_m - P.rho_a_amb, rr) * P.grav;
+  const double xc = ac_rho * inv_rhom;
+  const double shc = (xc > kEps) ? fdiv(xc * P.sp_heat_a, xc) : P.sp_heat_a;
+  double dsh = 0.0, xs[NS > 0 ? NS : 1];
+#pragma unroll
+  for (int i = 0; i < NS; i++) {
+    xs[i] = ars[i] * inv_rhom;
+    dsh += xs[i] * P.sp_heat_s[i];
+  }
+  const double shm = dsh + xc * shc;
+  const double q0 = rho_m * h;
+  s.qc[0] = q0;
+  s.qc[1] = rho_m * qp[1];
+  s.qc[2] = rho_m * qp[2];
+  s.qc[3] = P.energy ? q0 * (shm * T + 0.5 * (u * u + v * v)) : q0 * shm * T;
+#pragma unroll
+  for (int i = 0; i < NS; i++) s.qc[4 + i] = xs[i] * q0;
+  s.vel = (DIR == 1) ? u : v;
+  s.pt = 0.5 * rho_m * gc * rg * (h * h);
+  if (!__all(wet)) {
+    // dry lanes
+#pragma unroll
+    for (int i = 0; i < NV; i++) s.qc[i] = wet ? s.qc[i] : 0.0;
+    s.pt = wet ? s.pt : 0.0;
+    rg = wet ? rg : 0.0;
+  }
+  const double rgh = rg * h;
+  const double cel = fsqrt((DIR == 1) ? rgh * gc : gc * rg * h);
+  s.vmin = (rgh < 0.0) ? s.vel : s.vel - cel;
+  s.vmax = (rgh < 0.0) ? s.vel : s.vel + cel;
   s.zv = (DIR == 1) ? qp[1] : s.qc[2];
 }
+// with the profiles (bx, by: the slope of the cell the state belongs to, read
+// by the profile flux coefficients)
+template <int NS, int DIR>
+__device__ __forceinline__ void make_side(const DevParams& P, const double* qp, double gc,
+                                          Side<NS>& s, double bx, double by) {
+  make_side_vp<NS, DIR>(P, qp, gc, bx, by, &s);
+}
+template <int NS, bool VP>
+struct side_of {
+  using type = LeanSide<NS>;
+};
+template <int NS>
+struct side_of<NS, true> {
+  using type = Side<NS>;
+};
 
+// the side with its fluxes
+template <int NS, int DIR>
+__device__ __forceinline__ void expand(const DevParams& P, const LeanSide<NS>& s, Side<NS>& o) {
+  constexpr int NV = 4 + NS;
+  double sf = 0.0;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    o.qc[i] = s.qc[i];
+    const double f = s.vel * s.qc[i];
+    o.f[i] = (i == DIR) ? f + s.pt : (i == 3 && P.energy) ? s.vel * (s.qc[3] + s.pt) : f;
+    if (i >= 4) sf += f;
+  }
+  // (the rounded quotient sf / f0 exceeds 1 exactly when sf exceeds f0 > 0)
+  if (o.f[0] > 0.0 && sf > o.f[0]) {
+    const Rcp rs = rcp_of(sf);
+#pragma unroll
+    for (int i = 4; i < NV; i++) o.f[i] = div_by(o.f[i], rs) * o.f[0];
+  }
+  o.vmin = s.vmin;
+  o.vmax = s.vmax;
+  o.zv = s.zv;
+}
+template <int NS, int DIR>
+__device__ __forceinline__ void expand(const DevParams&, const Side<NS>& s, Side<NS>& o) {
+  o = s;
+}
+
+template <int NS>
+__device__ __forceinline__ void zero_side(LeanSide<NS>& s) {
+#pragma unroll
+  for (int i = 0; i < 4 + NS; i++) s.qc[i] = 0.0;
+  s.vel = s.pt = s.vmin = s.vmax = s.zv = 0.0;
+}
 template <int NS>
 __device__ __forceinline__ void zero_side(Side<NS>& s) {
 #pragma unroll
@@ -726,21 +898,37 @@ __device__ __forceinline__ void zero_side(Side<NS>& s) {
   s.vmin = s.vmax = s.zv = 0.0;
 }
 
+// the side of the lane to the left
 template <int NS>
-__device__ __forceinline__ void shfl_side(const Side<NS>& in, Side<NS>& out, int src) {
+__device__ __forceinline__ void left_side(const Side<NS>& in, Side<NS>& out) {
 #pragma unroll
   for (int i = 0; i < 4 + NS; i++) {
-    out.f[i] = shfl_d(in.f[i], src);
-    out.qc[i] = shfl_d(in.qc[i], src);
+    out.f[i] = lane_left(in.f[i]);
+    out.qc[i] = lane_left(in.qc[i]);
   }
-  out.vmin = shfl_d(in.vmin, src);
-  out.vmax = shfl_d(in.vmax, src);
-  out.zv = shfl_d(in.zv, src);
+  out.vmin = lane_left(in.vmin);
+  out.vmax = lane_left(in.vmax);
+  out.zv = lane_left(in.zv);
+}
+template <int NS>
+__device__ __forceinline__ void left_side(const LeanSide<NS>& in, LeanSide<NS>& out) {
+#pragma unroll
+  for (int i = 0; i < 4 + NS; i++) out.qc[i] = lane_left(in.qc[i]);
+  out.vel = lane_left(in.vel);
+  out.pt = lane_left(in.pt);
+  out.vmin = lane_left(in.vmin);
+  out.vmax = lane_left(in.vmax);
+  out.zv = lane_left(in.zv);
 }
 
-template <int NS, int DIR>
-__device__ __forceinline__ double face_flux(const Side<NS>& L, const Side<NS>& R,
+// KT flux of the face between sides A (left / bottom) and B; returns the
+// largest wave speed
+template <int NS, int DIR, typename S>
+__device__ __forceinline__ double face_flux(const DevParams& P, const S& A, const S& B,
                                             double* H) {
+  Side<NS> L, R;
+  expand<NS, DIR>(P, A, L);
+  expand<NS, DIR>(P, B, R);
   const double aN = fmin(fmin(L.vmin, R.vmin), 0.0);
   const double aP = fmax(fmax(L.vmax, R.vmax), 0.0);
   kt_flux<NS, DIR>(L.f, R.f, L.qc, R.qc, aN, aP, L.zv, R.zv, H);
@@ -764,18 +952,6 @@ __device__ __forceinline__ void load_src(const DevParams& P, const DevPtrs& D, i
   b = on ? b : 0;
   v0 = on ? v0 : 0.0;
   v1 = on ? v1 : 0.0;
-}
-
-// boundary state of a ring cell (zero elsewhere), src/solver_2d.f90:3879-3889
-template <int NS>
-__device__ __forceinline__ void ring_state(const DevParams& P, const SrcInfo S,
-                                           const SrcTime& T, double v0, double v1,
-                                           double* sb) {
-  constexpr int NV = 4 + NS;
-#pragma unroll
-  for (int i = 0; i < NV + 2; i++) sb[i] = 0.0;
-  if (!(P.radial && S.src2 && S.dir)) return;
-  source_bdry<NS>(P, T, v0, v1, sb);
 }
 
 // ---------------------------------------------------------------------------
@@ -867,70 +1043,38 @@ __device__ __forceinline__ void load_row(const DevParams& P, const DevPtrs& D,
   }
 }
 
-// the two sides of the y face between rows k-1 (B, owner Sb) and k (T,
-// owner St), with the ring overrides of src/solver_2d.f90:3879-3889
-// (VP: pb, pt are the slopes (bx, by) of rows k-1 and k; the ring overrides
-// keep them by position, which matters only with slope correction, a
-// combination the library refuses)
-// A face side from one of two value sets (b when use_b), or a zero side
-// when `zero`: one make_side on the chosen values, zeroed afterwards.  The
-// same side as a make_side call per case; calls per case had left parts of
-// the side in scratch memory.
-template <int NS, int DIR, bool VP>
-__device__ __forceinline__ void side_of(const DevParams& P, const double* a, const double* b,
-                                        bool use_b, bool zero, double g, Side<NS>& s,
-                                        double bx, double by) {
-  constexpr int NV = 4 + NS;
-  double q[NV + 2];
-#pragma unroll
-  for (int i = 0; i < NV + 2; i++) {
-    double x = a[i], y = b[i];
-    pin(x);
-    pin(y);
-    q[i] = use_b ? y : x;
-  }
-  make_side<NS, DIR, VP>(P, q, g, s, bx, by);
-#pragma unroll
-  for (int i = 0; i < NV; i++) {
-    s.f[i] = zero ? 0.0 : s.f[i];
-    s.qc[i] = zero ? 0.0 : s.qc[i];
-  }
-  s.vmin = zero ? 0.0 : s.vmin;
-  s.vmax = zero ? 0.0 : s.vmax;
-  s.zv = zero ? 0.0 : s.zv;
-}
-
-// Bottom side of the y face between rows k-1 (hib, source data Sb) and k
-// (lot, St): hib, except next to a source cell (the ring's own value, or
-// none).
-template <int NS, bool VP = false>
-__device__ __forceinline__ void yface_bottom(const DevParams& P, const double* hib,
-                                             const double* lot, const SrcInfo Sb,
-                                             const SrcInfo St, int k, double g, Side<NS>& Bs,
-                                             const double* pb = nullptr) {
-  const double bx = VP ? pb[0] : 0.0, by = VP ? pb[1] : 0.0;
-  const bool zero = Sb.is_src && !(P.radial && St.src2 && St.sS && k < P.ny - 1);
-  side_of<NS, 2, VP>(P, hib, lot, Sb.is_src, zero, g, Bs, bx, by);
-}
-// Top side of the same face: lot, except next to a source cell.
-template <int NS, bool VP = false>
-__device__ __forceinline__ void yface_top(const DevParams& P, const double* hib,
-                                          const double* lot, const SrcInfo Sb,
-                                          const SrcInfo St, int k, double g, Side<NS>& Ts,
-                                          const double* pt = nullptr) {
-  const double bx = VP ? pt[0] : 0.0, by = VP ? pt[1] : 0.0;
-  const bool zero = St.is_src && !(P.radial && Sb.src2 && !Sb.sS && Sb.sN && k - 1 > 0);
-  side_of<NS, 2, VP>(P, hib, lot, !St.is_src, zero, g, Ts, bx, by);
-}
-template <int NS, bool VP = false>
+// the two sides of the y face between rows k-1 (B, owner Sb, value hib) and k
+// (T, owner St, value lot), 0 <= k <= ny: at a domain boundary both sides
+// carry the row's own value, next to a source cell the ring's value or none
+// (src/solver_2d.f90:3879-3889).  (VP: pb, pt are the slopes (bx, by) of rows
+// k-1 and k; the ring overrides keep them by position, which matters only
+// with slope correction, a combination the library refuses.)
+template <int NS, typename S>
 __device__ __forceinline__ void yface_sides(const DevParams& P, const double* hib,
                                             const double* lot, const SrcInfo Sb,
-                                            const SrcInfo St, int k, double g,
-                                            Side<NS>& Bs, Side<NS>& Ts,
-                                            const double* pb = nullptr,
-                                            const double* pt = nullptr) {
-  yface_bottom<NS, VP>(P, hib, lot, Sb, St, k, g, Bs, pb);
-  yface_top<NS, VP>(P, hib, lot, Sb, St, k, g, Ts, pt);
+                                            const SrcInfo St, int k, double g, S& Bs, S& Ts,
+                                            const double* pb, const double* pt) {
+  make_side<NS, 2>(P, hib, g, Bs, pb[0], pb[1]);
+  make_side<NS, 2>(P, lot, g, Ts, pt[0], pt[1]);
+  if (k == 0) {
+    if (St.is_src) zero_side<NS>(Ts);
+    Bs = Ts;
+  } else if (k == P.ny) {
+    if (Sb.is_src) zero_side<NS>(Bs);
+    Ts = Bs;
+  } else if (P.radial && __any(Sb.is_src || St.is_src)) {
+    // next to a source cell a side carries the other row's value (the side
+    // just made from it) or none
+    const S B = Bs, T = Ts;
+    if (Sb.is_src) {
+      if (St.src2 && St.sS && k < P.ny - 1) Bs = T;
+      else zero_side<NS>(Bs);
+    }
+    if (St.is_src) {
+      if (Sb.src2 && !Sb.sS && Sb.sN && k - 1 > 0) Ts = B;
+      else zero_side<NS>(Ts);
+    }
+  }
 }
 // the slope (bx, by) of cell (j, k) from a clamped address
 __device__ __forceinline__ void load_bp(const DevParams& P, const DevPtrs& D, int j, int k,
@@ -985,112 +1129,81 @@ __device__ __forceinline__ double load_gsy(const DevParams& P, const DevPtrs& D,
   return D.gsy ? v : 1.0;
 }
 
-template <int NS>
+// The x face fluxes of row k from its W sides and the E sides of the left
+// neighbours: the W face on every lane, the E face from the right neighbour.
+// The boundary faces carry the edge cell's own side on both sides: the W face
+// of column 0, and the E face of column nx-1, which is the W face of the halo
+// lane j == nx.  Every lane of the wavefront calls it.
+template <int NS, typename ST>
 __device__ __forceinline__ void x_face_fluxes(const DevParams& P, const SrcInfo S, int j,
-                                              const Side<NS>& Wself, const Side<NS>& Eself,
-                                              const Side<NS>& Eleft, double* HW, double* HE,
-                                              double& amaxW, double& amaxE);
-
-// x direction of row k: the W face flux on every lane, the E face by
-// shuffle from the right neighbour (a boundary face on the last column).
-// S is row k's source data, sb its ring state, qk its physical state.
-template <int NS, bool HASY, bool VP = false>
-__device__ __forceinline__ void x_fluxes(const DevParams& P, const SrcInfo S, const double* sb,
-                                         const double* qk, int j, int k, const RowData& R,
-                                         double* HW, double* HE, double& amaxW,
-                                         double& amaxE) {
+                                              const ST& Wself, const ST& Eleft, double* HW,
+                                              double* HE, double& amax) {
   constexpr int NV = 4 + NS;
-  const int lane = threadIdx.x & 63;
-  const bool injx = (j >= 0 && j < P.nx);
-  double qkm[NV + 2], qkp[NV + 2];
-#pragma unroll
-  for (int i = 0; i < NV + 2; i++) {
-    qkm[i] = shfl_d(qk[i], (lane + 63) & 63);
-    qkp[i] = shfl_d(qk[i], (lane + 1) & 63);
-  }
-  // after a north ring cell the x-slope of v uses y_stag(k+1) as its
-  // third abscissa (src/solver_2d.f90:3616)
-  const bool typo = HASY && injx && P.radial && S.src2 && k > 0 && k < P.ny - 1 &&
-                    !S.sS && S.sN;
-  Side<NS> Wself, Eself;
-  if (injx) {
-    double lo[NV + 2], hi[NV + 2];
-    recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, S, sb, typo, lo, hi);
-    if (S.is_src) {
-      zero_side<NS>(Wself);
-      zero_side<NS>(Eself);
-    } else {
-      make_side<NS, 1, VP>(P, lo, R.gW, Wself, R.bx, R.by);
-      make_side<NS, 1, VP>(P, hi, R.gE, Eself, R.bx, R.by);
+  ST Ls = Eleft, Rs = Wself;
+  if (P.radial && __any(S.is_src)) {
+    const int flags = (S.is_src ? 1 : 0) | (S.src2 ? 2 : 0) | (S.sE ? 4 : 0) | (S.sW ? 8 : 0);
+    const int flags_left = __shfl(flags, (threadIdx.x + 63) & 63, kWave);
+    const bool interior_me = (j > 0 && j < P.nx - 1);
+    const bool interior_left = (j - 1 > 0 && j - 1 < P.nx - 1);
+    if (flags_left & 1) {
+      if (S.src2 && !S.sE && S.sW && interior_me) Ls = Wself;
+      else zero_side<NS>(Ls);
     }
-  } else {
-    zero_side<NS>(Wself);
-    zero_side<NS>(Eself);
+    if (S.is_src) {
+      if ((flags_left & 2) && (flags_left & 4) && interior_left) Rs = Eleft;
+      else zero_side<NS>(Rs);
+    }
   }
-  Side<NS> Eleft;
-  shfl_side<NS>(Eself, Eleft, (lane + 63) & 63);
-  x_face_fluxes<NS>(P, S, j, Wself, Eself, Eleft, HW, HE, amaxW, amaxE);
-}
-
-// The x face fluxes of row k from its W and E sides (Eleft: the E side of
-// the left neighbour): the W face on every lane, the E face by shuffle from
-// the right neighbour (a boundary face on the last column).
-template <int NS>
-__device__ __forceinline__ void x_face_fluxes(const DevParams& P, const SrcInfo S, int j,
-                                              const Side<NS>& Wself, const Side<NS>& Eself,
-                                              const Side<NS>& Eleft, double* HW, double* HE,
-                                              double& amaxW, double& amaxE) {
-  constexpr int NV = 4 + NS;
-  const int lane = threadIdx.x & 63;
-  const int flags = (S.is_src ? 1 : 0) | (S.src2 ? 2 : 0) | (S.sE ? 4 : 0) | (S.sW ? 8 : 0);
-  const int flags_left = __shfl(flags, (lane + 63) & 63, kWave);
-  {
-    Side<NS> Ls, Rs;
+  if (__any(j == 0 || j == P.nx)) {
     if (j == 0) {
       Ls = Wself;
       Rs = Wself;
-    } else {
-      const bool interior_me = (j > 0 && j < P.nx - 1);
-      const bool interior_left = (j - 1 > 0 && j - 1 < P.nx - 1);
-      if (flags_left & 1) {
-        if (P.radial && S.src2 && !S.sE && S.sW && interior_me) Ls = Wself;
-        else zero_side<NS>(Ls);
-      } else {
-        Ls = Eleft;
-      }
-      if (S.is_src) {
-        if (P.radial && (flags_left & 2) && (flags_left & 4) && interior_left) Rs = Eleft;
-        else zero_side<NS>(Rs);
-      } else {
-        Rs = Wself;
-      }
-    }
-    amaxW = face_flux<NS, 1>(Ls, Rs, HW);
-  }
-  {
-    double HEs[NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++) HEs[i] = shfl_d(HW[i], (lane + 1) & 63);
-    double amaxEs = shfl_d(amaxW, (lane + 1) & 63);
-    if (j == P.nx - 1) {
-      amaxE = face_flux<NS, 1>(Eself, Eself, HE);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NV; i++) HE[i] = HEs[i];
-      amaxE = amaxEs;
+    } else if (j == P.nx) {
+      Ls = Eleft;
+      Rs = Eleft;
     }
   }
+  const double aW = face_flux<NS, 1>(P, Ls, Rs, HW);
+#pragma unroll
+  for (int i = 0; i < NV; i++) HE[i] = lane_right(HW[i]);
+  amax = fmax(aW, lane_right(aW));
 }
 
-// divergence, explicit terms and the residual D of one computed cell, and
-// its CFL time step folded into dtmin
+// x direction of row k: its source data, physical state qk and per-cell data
+template <int NS, bool HASY, bool VP = false>
+__device__ __forceinline__ void x_fluxes(const DevParams& P, const Ring& ring,
+                                         const double* qk, int j, int k, const RowData& R,
+                                         double* HW, double* HE, double& amax) {
+  constexpr int NV = 4 + NS;
+  const SrcInfo S = ring.S;
+  double qkm[NV + 2], qkp[NV + 2], lo[NV + 2], hi[NV + 2];
+#pragma unroll
+  for (int i = 0; i < NV + 2; i++) {
+    qkm[i] = lane_left(qk[i]);
+    qkp[i] = lane_right(qk[i]);
+  }
+  // after a north ring cell the x-slope of v uses y_stag(k+1) as its
+  // third abscissa (src/solver_2d.f90:3616)
+  const bool typo = HASY && j >= 0 && j < P.nx && P.radial && S.src2 && k > 0 &&
+                    k < P.ny - 1 && !S.sS && S.sN;
+  recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, ring, typo, lo, hi);
+  typename side_of<NS, VP>::type Wself, Eself, Eleft;
+  make_side<NS, 1>(P, lo, R.gW, Wself, R.bx, R.by);
+  make_side<NS, 1>(P, hi, R.gE, Eself, R.bx, R.by);
+  if (P.radial && S.is_src) {
+    zero_side<NS>(Wself);
+    zero_side<NS>(Eself);
+  }
+  left_side<NS>(Eself, Eleft);
+  x_face_fluxes<NS>(P, S, j, Wself, Eleft, HW, HE, amax);
+}
+
+// divergence, explicit terms and the residual D of one computed cell
 template <int NS, bool HASY>
 __device__ __forceinline__ void cell_update(const DevParams& P, const DevPtrs& D, size_t c,
                                             const double* qk, const RowData& R,
                                             const double* HW, const double* HE,
-                                            const double* HS, const double* HN, double amaxW,
-                                            double amaxE, double amaxS, double amaxN,
-                                            int compute_dt, double& dtmin,
+                                            const double* HS, const double* HN,
                                             const double* ex_in = nullptr) {
   constexpr int NV = 4 + NS;
   const size_t pl = plane(P);
@@ -1108,25 +1221,18 @@ __device__ __forceinline__ void cell_update(const DevParams& P, const DevPtrs& D
     if (HASY) dv = dv + (HN[i] - HS[i]) * P.one_by_dy;
     D.D[i * pl + c] = (0.0 + (dv - ex[i]) * 1.0) + (0.0 - 0.0) * 0.0;
   }
-  if (compute_dt) {
-    double ma = fmax(amaxW, amaxE);
-    const double dtx = (ma > 0.0) ? P.cfl * P.dx / ma : P.max_dt;
-    double dty = P.max_dt;
-    if (HASY) {
-      ma = fmax(amaxS, amaxN);
-      dty = (ma > 0.0) ? P.cfl * P.dy / ma : P.max_dt;
-    }
-    dtmin = fmin(dtmin, fmin(dtx, dty));
-  }
 }
 
-// wave minimum of the CFL time step, one atomic per wave (dt > 0: IEEE
-// order == integer order)
-__device__ __forceinline__ void dt_reduce(const DevPtrs& D, const DevParams& P, double dtmin) {
+// The CFL time step of a wavefront's cells from the largest face speed amax
+// of each lane's computed cells (dx = dy: cfl dx / a falls with a, so the
+// smallest quotient is the largest speed's), one atomic per wave (dt > 0:
+// IEEE order == integer order)
+__device__ __forceinline__ void dt_reduce(const DevPtrs& D, const DevParams& P, double amax) {
   const int lane = threadIdx.x & 63;
-  for (int off = 32; off > 0; off >>= 1) dtmin = fmin(dtmin, shfl_d(dtmin, (lane + off) & 63));
-  if (lane == 0 && dtmin < P.max_dt)
-    atomicMin(D.dt_bits, (unsigned long long)__double_as_longlong(dtmin));
+  for (int off = 32; off > 0; off >>= 1) amax = fmax(amax, shfl_d(amax, (lane + off) & 63));
+  const double dt = (amax > 0.0) ? fdiv(P.cfl * P.dx, amax) : P.max_dt;
+  if (lane == 0 && dt < P.max_dt)
+    atomicMin(D.dt_bits, (unsigned long long)__double_as_longlong(dt));
 }
 
 template <int NS, bool HASY, bool VP = false>
@@ -1153,13 +1259,34 @@ __device__ __forceinline__ int strip_height(const DevParams& P, unsigned long lo
   return strip_h;
 }
 
-// The stencil pass over the listed work tiles, cut into strips of strip_h
-// rows; workgroups take (tile, strip) items in turn until the list is
-// exhausted.  With one-row strips every item is a listed row.
+// Height of this step's strips with the default tuning: the power of two for
+// which the rounds of the resident wavefronts, each of (h + kStripOver) row
+// times, take least.  kStripOver is what a strip spends outside its rows: two
+// iterations of the y part, about one row's time together.
+constexpr int kStripOver = 1;
+__device__ __forceinline__ int strip_fit(int nrows, int slots, int max_strip) {
+  int best = 1, cost = 1 << 30;
+  for (int h = 1; h <= max_strip; h *= 2) {
+    const int t = ((nrows + h - 1) / h + slots - 1) / slots * (h + kStripOver);
+    if (t < cost) {
+      cost = t;
+      best = h;
+    }
+  }
+  return best;
+}
+
+// The stencil pass over the listed work tiles, cut into strips; workgroups
+// take strips in turn until the list is exhausted.  With one-row strips every
+// item is a listed row.  When every tile is listed the strips are cut from
+// whole tile columns instead, col_h rows each (chosen by the host so that
+// they fill the resident wavefronts evenly: 1000 x 1000 cells are 17 columns
+// of 60 strips of 17 rows, one round of 1020 on 1024 SIMDs, where 8-row
+// pieces of tiles made three rounds of 2142).
 template <int NS, bool HASY, bool VP = false>
 __global__ void __launch_bounds__(64) k_stencil(DevParams P, DevPtrs D, int unit,
                                                 int max_strip, int target_strips,
-                                                int compute_dt) {
+                                                int compute_dt, int col_h) {
   const int lane = threadIdx.x;
   // the step's scalars and list sizes in one round of loads
   double done = D.scal[S_DONE], t = D.scal[S_T];
@@ -1171,35 +1298,44 @@ __global__ void __launch_bounds__(64) k_stencil(DevParams P, DevPtrs D, int unit
   pin(ntiles);
   pin(nrows);
   if (done != 0.0) return;
-  const int strip_h = strip_height(P, w, unit, max_strip, target_strips);
   // the ring cells' time factors are the same for the whole step
-  const SrcTime T = P.radial ? src_time(P, t) : SrcTime{};
+  const SrcTime T = uniform(P.radial ? src_time(P, t) : SrcTime{});
   const int tiles_x = (P.nx + kStripW - 1) / kStripW;
-  if (strip_h == 1) {
-    for (int item = blockIdx.x; item < nrows; item += gridDim.x) {
-      const int row = D.row_list[item];
-      const int tile = row / kTileH;
-      const int k0 = (tile / tiles_x) * kTileH + row % kTileH;
-      stencil_strip<NS, HASY, VP>(P, D, T, (tile % tiles_x) * kStripW - 2 + lane, k0, k0 + 1,
-                                  false, compute_dt);
+  const bool cols = col_h > 0 && ntiles == tiles_x * ((P.ny + kTileH - 1) / kTileH);
+  const int strip_h = cols ? col_h
+                      : (col_h > 0) ? strip_fit(nrows, gridDim.x, max_strip)
+                                    : strip_height(P, w, unit, max_strip, target_strips);
+  // one-row strips: the listed rows; else the strips of the listed tiles
+  const bool by_row = !cols && strip_h == 1;
+  const int per = cols ? 1 : kTileH / strip_h;
+  const int items = cols ? tiles_x * ((P.ny + strip_h - 1) / strip_h)
+                    : by_row ? nrows : ntiles * per;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    int tx, k0;
+    if (cols) {
+      tx = item % tiles_x;
+      k0 = (item / tiles_x) * strip_h;
+    } else {
+      const int e = by_row ? D.row_list[item] : D.tile_list[item / per];
+      const int tile = by_row ? e / kTileH : e;
+      tx = tile % tiles_x;
+      k0 = (tile / tiles_x) * kTileH + (by_row ? e % kTileH : (item % per) * strip_h);
     }
-    return;
-  }
-  const int per = kTileH / strip_h;
-  for (int item = blockIdx.x; item < ntiles * per; item += gridDim.x) {
-    const int tile = D.tile_list[item / per];
-    const int tx = tile % tiles_x, tyy = tile / tiles_x;
-    const int k0 = tyy * kTileH + (item % per) * strip_h;
     if (k0 >= P.ny) continue;
-    const int k1 = min(k0 + strip_h, P.ny);
-    stencil_strip<NS, HASY, VP>(P, D, T, tx * kStripW - 2 + lane, k0, k1, true, compute_dt);
+    stencil_strip<NS, HASY, VP>(P, D, T, tx * kStripW - 2 + lane, k0, min(k0 + strip_h, P.ny),
+                                !by_row, compute_dt);
   }
 }
 
 // One strip: lane l owns column j = 60 * tile_x - 2 + l, rows k0 .. k1-1.
-// Every load of a row is issued one row ahead of its use (the raw states
-// three rows ahead), from clamped addresses and without a branch around it,
-// so that a strip pays the memory latency about once.
+// Iteration k reconstructs row k+1 along y, closes the N face of row k and
+// updates row k; it starts two rows below the strip, where only the first
+// parts run, so that every piece of the march exists once in the code.  (The
+// former march had the first face peeled off, one copy for one-row strips and
+// one for taller ones, and the boundary faces' own calls: 290 KB of code at
+// three classes, far beyond the instruction cache.)  Every load of a row is
+// issued one row ahead of its use, from clamped addresses and without a
+// branch around it, so that a strip pays the memory latency about once.
 template <int NS, bool HASY, bool VP>
 __device__ __forceinline__ void stencil_strip(const DevParams& P, const DevPtrs& D,
                                               const SrcTime& T, int j, int k0, int k1,
@@ -1216,158 +1352,107 @@ __device__ __forceinline__ void stencil_strip(const DevParams& P, const DevPtrs&
       for (int k = k0; k < k1; k++) any |= D.mask[cidx(P, j, k)] & M_COMPUTE;
     if (!__any(any)) return;
   }
-  const size_t pl = plane(P);
-  double dtmin = P.max_dt;
   const bool stored = VP && D.qpp;
-
-  double qm[NV + 2], qc[NV + 2], qn[NV + 2];  // rows k-1, k, k+1
-  double hiy[NV + 2];                          // N value of row k
-  double HS[NV];                               // y flux at the S face of row k
-  double amaxS = 0.0;
-  double rnext[NV + 2];  // raw values of row k+2, loaded one iteration ahead
-  // source data: row k (S, v0, v1) and row k+1 (raw byte bn, vectors), the
-  // slope correction of the S face of row k+1, and row k's per-cell data
-  int bc = 0, bn = 0;
-  double vc0 = 0.0, vc1 = 0.0, vn0 = 0.0, vn1 = 0.0, gn = 1.0;
-  RowData R;
+  double amax = 0.0;                    // of the computed cells
+  double qc[NV + 2], qn[NV + 2];        // rows k, k+1
+  double hiy[NV + 2];                   // N value of row k
+  double HS[NV], amaxS = 0.0;           // the S face of row k
+  double rnext[NV + 2];                 // raw values of row k+2
+  // source data: row k (S, vector) and row k+1 (raw byte bn, vector), and the
+  // slope correction of the N face of row k
   SrcInfo S{};
-  if (HASY) {
-    double qmm[NV + 2], sb[NV + 2], lo[NV + 2];
-    int bm;
-    double vm0, vm1, g0 = 1.0;
-    {
-      double r0[NV + 2], r1[NV + 2], r2[NV + 2], r3[NV + 2];
-      load_raw_v<NS, VP>(P, D, j, k0 - 2, r0);
-      load_raw_v<NS, VP>(P, D, j, k0 - 1, r1);
-      load_raw_v<NS, VP>(P, D, j, k0, r2);
-      load_raw_v<NS, VP>(P, D, j, k0 + 1, r3);
-      load_raw_v<NS, VP>(P, D, j, k0 + 2, rnext);
-      load_src(P, D, j, k0 - 1, bm, vm0, vm1);
-      load_src(P, D, j, k0, bc, vc0, vc1);
-      load_src(P, D, j, k0 + 1, bn, vn0, vn1);
-      g0 = load_gsy(P, D, j, k0);
-      gn = load_gsy(P, D, j, k0 + 1);
-      load_rowdata(P, D, j, k0, R);
-      finish_row<NS, VP>(P, j, k0 - 2, r0, qmm, stored);
-      finish_row<NS, VP>(P, j, k0 - 1, r1, qm, stored);
-      finish_row<NS, VP>(P, j, k0, r2, qc, stored);
-      finish_row<NS, VP>(P, j, k0 + 1, r3, qn, stored);
-    }
-    if (injx) S = src_info(bc);
-    Side<NS> Bs, Ts;
-    if (injx) {
-      ring_state<NS>(P, S, T, vc0, vc1, sb);
-      recon<NS, 2>(P, qc, qm, qn, k0, P.ny, j, S, sb, false, lo, hiy);
-      const double g = g0;
-      const double pk[2] = {R.bx, R.by};
-      if (k0 == 0) {
-        // boundary face: both sides carry the S value of row 0
-        if (S.is_src) zero_side<NS>(Ts); else make_side<NS, 2, VP>(P, lo, g, Ts, pk[0], pk[1]);
-        Bs = Ts;
-      } else {
-        const SrcInfo Sm = src_info(bm);
-        double sbm[NV + 2], lom[NV + 2], him[NV + 2], pm[2] = {0.0, 0.0};
-        if (VP) load_bp(P, D, j, k0 - 1, pm);
-        ring_state<NS>(P, Sm, T, vm0, vm1, sbm);
-        recon<NS, 2>(P, qm, qmm, qc, k0 - 1, P.ny, j, Sm, sbm, false, lom, him);
-        yface_sides<NS, VP>(P, him, lo, Sm, S, k0, g, Bs, Ts, pm, pk);
-      }
-    } else {
-      zero_side<NS>(Bs);
-      zero_side<NS>(Ts);
+  double vc0 = 0.0, vc1 = 0.0, vn0 = 0.0, vn1 = 0.0, gn = 1.0;
+  int bn = 0;
 #pragma unroll
-      for (int i = 0; i < NV + 2; i++) hiy[i] = 0.0;
-    }
-    amaxS = face_flux<NS, 2>(Bs, Ts, HS);
+  for (int i = 0; i < NV + 2; i++) hiy[i] = 0.0;
+#pragma unroll
+  for (int i = 0; i < NV; i++) HS[i] = 0.0;
+  int k = k0;
+  if (HASY) {
+    double r0[NV + 2], r1[NV + 2];
+    load_raw_v<NS, VP>(P, D, j, k0 - 2, r0);
+    load_raw_v<NS, VP>(P, D, j, k0 - 1, r1);
+    load_raw_v<NS, VP>(P, D, j, k0, rnext);
+    load_src(P, D, j, k0 - 1, bn, vn0, vn1);
+    finish_row<NS, VP>(P, j, k0 - 2, r0, qc, stored);
+    finish_row<NS, VP>(P, j, k0 - 1, r1, qn, stored);
+    k = k0 - 2;
   } else {
     load_row<NS, VP>(P, D, j, k0, qc);
+    int bc;
     load_src(P, D, j, k0, bc, vc0, vc1);
-    load_rowdata(P, D, j, k0, R);
-    if (injx) S = src_info(bc);
+    S = src_info(bc);
   }
 
-  for (int k = k0; k < k1; k++) {
-    const size_t c = injx ? cidx(P, j, k) : 0;
-    const bool more = k + 1 < k1;
-    // next row's per-cell data
-    RowData Rn;
-    if (more) load_rowdata(P, D, j, k + 1, Rn);
-    double sb[NV + 2];
-    if (injx) ring_state<NS>(P, S, T, vc0, vc1, sb);
-    else {
+#pragma unroll 1
+  for (; k < k1; k++) {
+    // ---------------- x faces and explicit terms of row k
+    const bool cell = k >= k0;
+    bool upd = false;
+    double dv[NV], ex[NV], amaxX = 0.0;
 #pragma unroll
-      for (int i = 0; i < NV + 2; i++) sb[i] = 0.0;
+    for (int i = 0; i < NV; i++) dv[i] = ex[i] = 0.0;
+    if (cell) {
+      RowData R;
+      load_rowdata(P, D, j, k, R);
+      double HW[NV], HE[NV];
+      x_fluxes<NS, HASY, VP>(P, Ring{S, T, vc0, vc1}, qc, j, k, R, HW, HE, amaxX);
+#pragma unroll
+      for (int i = 0; i < NV; i++) dv[i] = 0.0 + (HE[i] - HW[i]) * P.one_by_dx;
+      upd = own && (R.m & M_COMPUTE);
+      if (upd) expl_terms<NS>(P, R.bx, R.by, R.bxx, R.bxy, R.byy, R.gc, R.dg, qc, ex);
     }
-    // ---------------- y: N face of row k ----------------
-    double HN[NV];
-    double amaxN = 0.0;
-    SrcInfo Sn{};
-    int bnn = 0;
-    double vnn0 = 0.0, vnn1 = 0.0, gnn = 1.0;
+    const size_t pl = plane(P), c = cidx(P, j, k);
     if (HASY) {
-      double qnn[NV + 2], hin[NV + 2];
+      // ---------------- y: reconstruction of row k+1, the N face of row k
+      double qnn[NV + 2], lon[NV + 2], hin[NV + 2], HN[NV], amaxN = 0.0;
       finish_row<NS, VP>(P, j, k + 2, rnext, qnn, stored);
+      const bool more = k + 1 < k1;
+      SrcInfo Sn{};
+      if (injx && k + 1 >= 0 && k + 1 < P.ny) Sn = src_info(bn);
+      const Ring rn{Sn, T, vn0, vn1};
+      const double g = gn;
       if (more) {
         load_raw_v<NS, VP>(P, D, j, k + 3, rnext);  // next iteration's rows
-        load_src(P, D, j, k + 2, bnn, vnn0, vnn1);
-        gnn = load_gsy(P, D, j, k + 2);
+        load_src(P, D, j, k + 2, bn, vn0, vn1);
+        gn = load_gsy(P, D, j, k + 2);
       }
-      Side<NS> Bs, Ts;
-      const double pk[2] = {R.bx, R.by};
-      if (injx) {
-        if (k == P.ny - 1) {
-          const double g = gn;  // S face of row ny: the N boundary
-          if (S.is_src) zero_side<NS>(Bs); else make_side<NS, 2, VP>(P, hiy, g, Bs, pk[0], pk[1]);
-          Ts = Bs;
-#pragma unroll
-          for (int i = 0; i < NV + 2; i++) hin[i] = 0.0;
-        } else {
-          Sn = src_info(bn);
-          double sbn[NV + 2], lon[NV + 2];
-          ring_state<NS>(P, Sn, T, vn0, vn1, sbn);
-          recon<NS, 2>(P, qn, qc, qnn, k + 1, P.ny, j, Sn, sbn, false, lon, hin);
-          const double g = gn;
-          double pn[2] = {0.0, 0.0};
-          if (VP) load_bp(P, D, j, k + 1, pn);
-          yface_sides<NS, VP>(P, hiy, lon, S, Sn, k + 1, g, Bs, Ts, pk, pn);
+      recon<NS, 2>(P, qn, qc, qnn, k + 1, P.ny, j, rn, false, lon, hin);
+      if (k >= k0 - 1) {
+        double pk[2] = {0.0, 0.0}, pn[2] = {0.0, 0.0};
+        if (VP) {
+          load_bp(P, D, j, k, pk);
+          load_bp(P, D, j, k + 1, pn);
         }
-      } else {
-        zero_side<NS>(Bs);
-        zero_side<NS>(Ts);
-#pragma unroll
-        for (int i = 0; i < NV + 2; i++) hin[i] = 0.0;
+        typename side_of<NS, VP>::type Bs, Ts;
+        yface_sides<NS>(P, hiy, lon, S, Sn, k + 1, g, Bs, Ts, pk, pn);
+        amaxN = face_flux<NS, 2>(P, Bs, Ts, HN);
       }
-      amaxN = face_flux<NS, 2>(Bs, Ts, HN);
+      if (upd) {
+#pragma unroll
+        for (int i = 0; i < NV; i++)
+          D.D[i * pl + c] = 0.0 + ((dv[i] + (HN[i] - HS[i]) * P.one_by_dy) - ex[i]);
+        amax = fmax(amax, fmax(amaxX, fmax(amaxS, amaxN)));
+      }
 #pragma unroll
       for (int i = 0; i < NV + 2; i++) {
-        qm[i] = qc[i];
         qc[i] = qn[i];
         qn[i] = qnn[i];
         hiy[i] = hin[i];
       }
-    }
-    // physical state of row k: qm after the shift (2-D) or qc (1-D)
-    const double* qk = HASY ? qm : qc;
-    double HW[NV], HE[NV], amaxW, amaxE;
-    x_fluxes<NS, HASY, VP>(P, S, sb, qk, j, k, R, HW, HE, amaxW, amaxE);
-    if (own && (R.m & M_COMPUTE))
-      cell_update<NS, HASY>(P, D, c, qk, R, HW, HE, HS, HN, amaxW, amaxE, amaxS, amaxN,
-                            compute_dt, dtmin);
-    if (more) R = Rn;
-    if (HASY) {
 #pragma unroll
       for (int i = 0; i < NV; i++) HS[i] = HN[i];
       amaxS = amaxN;
       S = Sn;
-      vc0 = vn0;
-      vc1 = vn1;
-      bn = bnn;
-      vn0 = vnn0;
-      vn1 = vnn1;
-      gn = gnn;
+      vc0 = rn.v0;
+      vc1 = rn.v1;
+    } else if (upd) {
+#pragma unroll
+      for (int i = 0; i < NV; i++) D.D[i * pl + c] = 0.0 + (dv[i] - ex[i]);
+      amax = fmax(amax, amaxX);
     }
   }
-  if (compute_dt) dt_reduce(D, P, dtmin);
+  if (compute_dt) dt_reduce(D, P, amax);
 }
 
 // ---------------------------------------------------------------------------
@@ -1461,11 +1546,11 @@ __device__ __forceinline__ void vp_cell_sides(const DevParams& P, const DevPtrs&
   }
   // both reconstructions first: the neighbours' states are then dead while
   // the closures run
-  double sb[NV + 2], lox[NV + 2], hix[NV + 2], loy[NV + 2], hiy[NV + 2];
-  ring_state<NS>(P, S, T, v0, v1, sb);
+  double lox[NV + 2], hix[NV + 2], loy[NV + 2], hiy[NV + 2];
+  const Ring ring{S, T, v0, v1};
   const bool typo = P.radial && S.src2 && k > 0 && k < P.ny - 1 && !S.sS && S.sN;
-  recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, S, sb, typo, lox, hix);
-  recon<NS, 2>(P, qk, qm, qn, k, P.ny, j, S, sb, false, loy, hiy);
+  recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, ring, typo, lox, hix);
+  recon<NS, 2>(P, qk, qm, qn, k, P.ny, j, ring, false, loy, hiy);
   make_side_vp_body<NS, 1>(P, lox, R.gW, R.bx, R.by, &a);
   side_put<NS>(P, D, c, SD_W, a);
   make_side_vp_body<NS, 1>(P, hix, R.gE, R.bx, R.by, &b);
@@ -1536,7 +1621,7 @@ __device__ __forceinline__ void stencil_strip_vp(const DevParams& P, const DevPt
       for (int k = k0; k < k1; k++) any |= D.mask[cidx(P, j, k)] & M_COMPUTE;
     if (!__any(any)) return;
   }
-  double dtmin = P.max_dt;
+  double amax = 0.0;
   double HS[NV], amaxS = 0.0;
   int bc = 0;
   double v0, v1;
@@ -1560,7 +1645,7 @@ __device__ __forceinline__ void stencil_strip_vp(const DevParams& P, const DevPt
       side_get<NS>(P, D, j, k0, SD_S, Tn);
       vp_yface<NS>(P, Bn, Tn, src_info(bm), S, k0, Bs, Ts);
     }
-    amaxS = face_flux<NS, 2>(Bs, Ts, HS);
+    amaxS = face_flux<NS, 2>(P, Bs, Ts, HS);
   }
   for (int k = k0; k < k1; k++) {
     const size_t c = injx ? cidx(P, j, k) : 0;
@@ -1588,7 +1673,7 @@ __device__ __forceinline__ void stencil_strip_vp(const DevParams& P, const DevPt
         side_get<NS>(P, D, j, k + 1, SD_S, Tn);
         vp_yface<NS>(P, Bn, Tn, S, Sn, k + 1, Bs, Ts);
       }
-      amaxN = face_flux<NS, 2>(Bs, Ts, HN);
+      amaxN = face_flux<NS, 2>(P, Bs, Ts, HN);
     }
     // x faces of row k
     Side<NS> Wself, Eself, Eleft;
@@ -1599,18 +1684,19 @@ __device__ __forceinline__ void stencil_strip_vp(const DevParams& P, const DevPt
       zero_side<NS>(Wself);
       zero_side<NS>(Eself);
     }
-    shfl_side<NS>(Eself, Eleft, (lane + 63) & 63);
-    double HW[NV], HE[NV], amaxW, amaxE;
-    x_face_fluxes<NS>(P, S, j, Wself, Eself, Eleft, HW, HE, amaxW, amaxE);
-    if (own && (R.m & M_COMPUTE))
-      cell_update<NS, true>(P, D, c, qk, R, HW, HE, HS, HN, amaxW, amaxE, amaxS, amaxN,
-                            compute_dt, dtmin);
+    left_side<NS>(Eself, Eleft);
+    double HW[NV], HE[NV], amaxX;
+    x_face_fluxes<NS>(P, S, j, Wself, Eleft, HW, HE, amaxX);
+    if (own && (R.m & M_COMPUTE)) {
+      cell_update<NS, true>(P, D, c, qk, R, HW, HE, HS, HN);
+      amax = fmax(amax, fmax(amaxX, fmax(amaxS, amaxN)));
+    }
 #pragma unroll
     for (int i = 0; i < NV; i++) HS[i] = HN[i];
     amaxS = amaxN;
     S = Sn;
   }
-  if (compute_dt) dt_reduce(D, P, dtmin);
+  if (compute_dt) dt_reduce(D, P, amax);
 }
 
 // the strip items of k_stencil over the listed tiles, with the stored sides
@@ -1654,34 +1740,31 @@ __global__ void __launch_bounds__(64) k_stencil_vp(DevParams P, DevPtrs D, int u
 // the strip march.
 // ---------------------------------------------------------------------------
 template <int NS>
-__device__ __forceinline__ void side_store(double (*buf)[64], const Side<NS>& s, int lane) {
+__device__ __forceinline__ void side_store(double (*buf)[64], const LeanSide<NS>& s, int lane) {
 #pragma unroll
-  for (int i = 0; i < 4 + NS; i++) {
-    buf[i][lane] = s.f[i];
-    buf[4 + NS + i][lane] = s.qc[i];
-  }
-  buf[8 + 2 * NS][lane] = s.vmin;
-  buf[9 + 2 * NS][lane] = s.vmax;
-  buf[10 + 2 * NS][lane] = s.zv;
+  for (int i = 0; i < 4 + NS; i++) buf[i][lane] = s.qc[i];
+  buf[4 + NS][lane] = s.vel;
+  buf[5 + NS][lane] = s.pt;
+  buf[6 + NS][lane] = s.vmin;
+  buf[7 + NS][lane] = s.vmax;
+  buf[8 + NS][lane] = s.zv;
 }
 template <int NS>
-__device__ __forceinline__ void side_load(double (*buf)[64], Side<NS>& s, int lane) {
+__device__ __forceinline__ void side_load(double (*buf)[64], LeanSide<NS>& s, int lane) {
 #pragma unroll
-  for (int i = 0; i < 4 + NS; i++) {
-    s.f[i] = buf[i][lane];
-    s.qc[i] = buf[4 + NS + i][lane];
-  }
-  s.vmin = buf[8 + 2 * NS][lane];
-  s.vmax = buf[9 + 2 * NS][lane];
-  s.zv = buf[10 + 2 * NS][lane];
+  for (int i = 0; i < 4 + NS; i++) s.qc[i] = buf[i][lane];
+  s.vel = buf[4 + NS][lane];
+  s.pt = buf[5 + NS][lane];
+  s.vmin = buf[6 + NS][lane];
+  s.vmax = buf[7 + NS][lane];
+  s.zv = buf[8 + NS][lane];
 }
 
 // One listed row of k_stencil_rows (all six wavefronts of the workgroup).
 template <int NS>
 __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D, int row,
-                                            int tiles_x, double t, int compute_dt,
-                                            double& dtmin, double (*V)[NS + 6][64],
-                                            double (*SD)[2 * NS + 11][64]) {
+                                            int tiles_x, double t, double& amax, double (*V)[NS + 6][64],
+                                            double (*SD)[NS + 9][64]) {
   constexpr int NV = 4 + NS;
   constexpr int NQ = NV + 2;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1734,10 +1817,8 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
     if (need) {
       // a copy, not a reference: a reference chosen at run time would put
       // both structures in scratch memory
-      const SrcInfo Sr = (wv == 1) ? S : So;
-      double sb[NV + 2];
-      ring_state<NS>(P, Sr, T, (wv == 1) ? vc0 : vo0, (wv == 1) ? vc1 : vo1, sb);
-      recon<NS, 2>(P, qb, qa, qc, kr, P.ny, j, Sr, sb, false, lo, hi);
+      const Ring ring{(wv == 1) ? S : So, T, (wv == 1) ? vc0 : vo0, (wv == 1) ? vc1 : vo1};
+      recon<NS, 2>(P, qb, qa, qc, kr, P.ny, j, ring, false, lo, hi);
     } else {
 #pragma unroll
       for (int i = 0; i < NV + 2; i++) lo[i] = hi[i] = 0.0;
@@ -1758,16 +1839,15 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
   } else {
     finish_row<NS>(P, j, k, r1, qk);
     if (wv == 3) {
-      double sb[NV + 2], qkm[NV + 2], qkp[NV + 2], lo[NV + 2], hi[NV + 2];
+      double qkm[NV + 2], qkp[NV + 2], lo[NV + 2], hi[NV + 2];
 #pragma unroll
       for (int i = 0; i < NV + 2; i++) {
-        qkm[i] = shfl_d(qk[i], (lane + 63) & 63);
-        qkp[i] = shfl_d(qk[i], (lane + 1) & 63);
+        qkm[i] = lane_left(qk[i]);
+        qkp[i] = lane_right(qk[i]);
       }
       const bool typo = injx && P.radial && S.src2 && k > 0 && k < P.ny - 1 && !S.sS && S.sN;
       if (injx) {
-        ring_state<NS>(P, S, T, vc0, vc1, sb);
-        recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, S, sb, typo, lo, hi);
+        recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, Ring{S, T, vc0, vc1}, typo, lo, hi);
       } else {
 #pragma unroll
         for (int i = 0; i < NV + 2; i++) lo[i] = hi[i] = 0.0;
@@ -1783,7 +1863,7 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
   }
   __syncthreads();
   // ---- phase B
-  Side<NS> Wself;
+  LeanSide<NS> Wself;
   {
     double va[NQ], vb[NQ];
     const int ia = (wv < 2) ? 0 : (wv < 4) ? 2 : 4 + (wv - 4);
@@ -1793,7 +1873,7 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
 #pragma unroll
       for (int i = 0; i < NQ; i++) vb[i] = V[ia + 1][i][lane];
     }
-    Side<NS> sd;
+    LeanSide<NS> sd;
     if (wv < 4) {
       // y faces: S face of row k (w0 bottom = row k-1, w1 top = row k) and
       // N face (w2 bottom = row k, w3 top = row k+1).  The cases of
@@ -1829,14 +1909,7 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
         qs[i] = lot ? y : x;
       }
       make_side<NS, 2>(P, qs, g, sd);
-#pragma unroll
-      for (int i = 0; i < NV; i++) {
-        sd.f[i] = zero ? 0.0 : sd.f[i];
-        sd.qc[i] = zero ? 0.0 : sd.qc[i];
-      }
-      sd.vmin = zero ? 0.0 : sd.vmin;
-      sd.vmax = zero ? 0.0 : sd.vmax;
-      sd.zv = zero ? 0.0 : sd.zv;
+      if (zero) zero_side<NS>(sd);
       side_store<NS>(SD[wv], sd, lane);
     } else {
       // x faces: W side (w4, kept), E side (w5, to LDS)
@@ -1848,22 +1921,21 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
   }
   __syncthreads();
   // ---- phase C
-  double HW[NV], HE[NV], amaxW = 0.0, amaxE = 0.0;
+  double HW[NV], HE[NV], amaxX = 0.0;
   if (wv == 0 || wv == 2) {
-    Side<NS> Bs, Ts;
+    LeanSide<NS> Bs, Ts;
     side_load<NS>(SD[wv], Bs, lane);
     side_load<NS>(SD[wv + 1], Ts, lane);
     double H[NV];
-    const double a = face_flux<NS, 2>(Bs, Ts, H);
+    const double a = face_flux<NS, 2>(P, Bs, Ts, H);
     const int o = (wv == 0) ? 0 : 1;
 #pragma unroll
     for (int i = 0; i < NV; i++) V[o][i][lane] = H[i];
     V[o][NV][lane] = a;
   } else if (wv == 4) {
-    Side<NS> Eself, Eleft;
-    side_load<NS>(SD[4], Eself, lane);
+    LeanSide<NS> Eleft;
     side_load<NS>(SD[4], Eleft, (lane + 63) & 63);
-    x_face_fluxes<NS>(P, S, j, Wself, Eself, Eleft, HW, HE, amaxW, amaxE);
+    x_face_fluxes<NS>(P, S, j, Wself, Eleft, HW, HE, amaxX);
   }
   __syncthreads();
   // ---- phase D
@@ -1874,8 +1946,8 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
       HS[i] = V[0][i][lane];
       HN[i] = V[1][i][lane];
     }
-    cell_update<NS, true>(P, D, cidx(P, j, k), qk, R, HW, HE, HS, HN, amaxW, amaxE,
-                          V[0][NV][lane], V[1][NV][lane], compute_dt, dtmin, ex);
+    cell_update<NS, true>(P, D, cidx(P, j, k), qk, R, HW, HE, HS, HN, ex);
+    amax = fmax(amax, fmax(amaxX, fmax(V[0][NV][lane], V[1][NV][lane])));
   }
   __syncthreads();  // LDS free for the next row
 }
@@ -1885,7 +1957,7 @@ __global__ void __launch_bounds__(384) k_stencil_rows(DevParams P, DevPtrs D, in
   warm_kernargs<kArgBytes>();
   constexpr int NV = 4 + NS;
   constexpr int NQ = NV + 2;       // reconstructed values per side
-  constexpr int NSD = 2 * NV + 3;  // doubles per face side
+  constexpr int NSD = NV + 5;      // doubles per face side
   // phase A values (then the y fluxes of phase C), face sides
   __shared__ double V[6][NQ][64];
   __shared__ double SD[5][NSD][64];  // S bottom, S top, N bottom, N top, E of x
@@ -1900,14 +1972,14 @@ __global__ void __launch_bounds__(384) k_stencil_rows(DevParams P, DevPtrs D, in
   pin(row);
   if (done != 0.0 || (int)blockIdx.x >= nrows) return;
   const int tiles_x = (P.nx + kStripW - 1) / kStripW;
-  double dtmin = P.max_dt;
+  double amax = 0.0;
   // the workgroup's first row outside the loop over further rows: in a loop
   // the compiler hoists the row's uniform operands ahead of it, where, short
   // of scalar registers, it fetches the kernel arguments one at a time
-  stencil_row<NS>(P, D, row, tiles_x, t, compute_dt, dtmin, V, SD);
+  stencil_row<NS>(P, D, row, tiles_x, t, amax, V, SD);
   for (int item = blockIdx.x + gridDim.x; item < nrows; item += gridDim.x)
-    stencil_row<NS>(P, D, D.row_list[item], tiles_x, t, compute_dt, dtmin, V, SD);
-  if (wv == 4 && compute_dt) dt_reduce(D, P, dtmin);
+    stencil_row<NS>(P, D, D.row_list[item], tiles_x, t, amax, V, SD);
+  if (wv == 4 && compute_dt) dt_reduce(D, P, amax);
 }
 
 // ---------------------------------------------------------------------------

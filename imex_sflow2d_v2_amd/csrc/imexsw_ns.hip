@@ -10,6 +10,25 @@
 
 namespace imexsw {
 
+// Rows per whole-column strip (k_stencil) for `slots` resident wavefronts: the
+// height whose rounds take least, with the strip's own overhead; 0 with a
+// tuning other than the default, which asks for the tile strips it describes.
+static int column_height(const imexsw_ctx* c, int slots) {
+  if (c->P.ny < 2 || c->strip_h != kTileH || c->target_strips != kDefaultStrips) return 0;
+  const int tiles_x = (c->P.nx + kStripW - 1) / kStripW;
+  int best = 1;
+  long cost = -1;
+  for (int h = 1; h <= c->P.ny; h++) {
+    const long items = (long)tiles_x * ((c->P.ny + h - 1) / h);
+    const long t = (items + slots - 1) / slots * (h + kStripOver);
+    if (cost < 0 || t < cost) {
+      cost = t;
+      best = h;
+    }
+  }
+  return best;
+}
+
 template <int NS>
 void launch_stencil(imexsw_ctx* c, const DevPtrs& D, int compute_dt, bool rows) {
   // work items: (listed tile, strip) pairs, at most tiles * kTileH / row_unit
@@ -24,15 +43,16 @@ void launch_stencil(imexsw_ctx* c, const DevPtrs& D, int compute_dt, bool rows) 
   } else if (c->P.ny > 1) {
     static int res = 0;
     if (!res) res = resident_grid(k_stencil<NS, true>, 64, c->n_cu, 1 << 30);
-    hipLaunchKernelGGL((k_stencil<NS, true>), dim3(std::min(items, res)), dim3(64), 0,
-                       c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                       compute_dt);
+    const int grid = std::min(items, res);
+    hipLaunchKernelGGL((k_stencil<NS, true>), dim3(grid), dim3(64), 0, c->stream, c->P, D,
+                       c->row_unit, c->strip_h, c->target_strips, compute_dt,
+                       column_height(c, grid));
   } else {
     static int res = 0;
     if (!res) res = resident_grid(k_stencil<NS, false>, 64, c->n_cu, 1 << 30);
     hipLaunchKernelGGL((k_stencil<NS, false>), dim3(std::min(items, res)), dim3(64), 0,
                        c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                       compute_dt);
+                       compute_dt, 0);
   }
 }
 #if IMEXSW_PART == 3
@@ -53,12 +73,12 @@ void launch_stencil_vp(imexsw_ctx* c, const DevPtrs& D, int compute_dt, int item
     if (!res2) res2 = resident_grid(k_stencil<NS, true, true>, 64, c->n_cu, 1 << 30);
     hipLaunchKernelGGL((k_stencil<NS, true, true>), dim3(std::min(items, res2)), dim3(64), 0,
                        c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                       compute_dt);
+                       compute_dt, 0);
   } else {
     if (!res1) res1 = resident_grid(k_stencil<NS, false, true>, 64, c->n_cu, 1 << 30);
     hipLaunchKernelGGL((k_stencil<NS, false, true>), dim3(std::min(items, res1)), dim3(64), 0,
                        c->stream, c->P, D, c->row_unit, c->strip_h, c->target_strips,
-                       compute_dt);
+                       compute_dt, 0);
   }
 }
 #endif
@@ -178,7 +198,7 @@ void launch_assemble(imexsw_ctx* c, int policy) {
 template <int NS>
 void launch_batch_stencil(imexsw_ensemble* e) {
   const BatchLists L = batch_lists(e);
-  const int per = kTileH / e->strip_h;
+  const int per = e->strip_h ? kTileH / e->strip_h : kTileH;  // most strips per tile
   static int rs = 0;
   if (!rs) rs = resident_grid(kb_stencil<NS>, 64, e->n_cu, 1 << 30);
   hipLaunchKernelGGL((kb_stencil<NS>), dim3(std::min(e->total_tiles * per, rs)), dim3(64), 0,

@@ -32,6 +32,7 @@ struct DevParams {
   double cfl, max_dt, reconstr_coeff, theta;
   int limiter[IMEXSW_MAX_VARS + 2];
   int lim_c;  // some limiter (3, 4, 5) uses the centred difference
+  int lim_1;  // every variable's limiter is 1 (minmod)
   int bc_flag[4][IMEXSW_MAX_VARS];
   double bc_value[4][IMEXSW_MAX_VARS];
   // the side's condition on h keeps a dry neighbourhood dry: zero-gradient
@@ -113,13 +114,12 @@ __device__ __forceinline__ cpx csqrt_(cpx x) {
 // limiters (src/geometry_2d.f90:1555-1676)
 // ---------------------------------------------------------------------------
 // minmod(a,b) = 0.5*(sign a + sign b)*min(|a|,|b|); identical for all
-// finite arguments to the reference's division-based form.
+// finite arguments to the reference's division-based form (zero for a NaN).
 __device__ __forceinline__ double minmod_(double a, double b) {
-  double m = fmin(fabs(a), fabs(b));
-  if (!(m > 0.0)) return 0.0;
-  if (a > 0.0 && b > 0.0) return m;
-  if (a < 0.0 && b < 0.0) return -m;
-  return 0.0;
+  // the product's high word tells equal signs (also where it underflows: a
+  // zero keeps its sign) from opposite ones and from a NaN in one compare
+  const double m = copysign(fmin(fabs(a), fabs(b)), a);
+  return ((unsigned)__double2hiint(a * b) <= 0x7ff00000u) ? m : 0.0;
 }
 __device__ __forceinline__ double maxmod_(double a, double b) {
   if (fabs(a * b) <= 0.0) return 0.0;
@@ -128,26 +128,9 @@ __device__ __forceinline__ double maxmod_(double a, double b) {
   if (a < 0.0 && b < 0.0) return -m;
   return 0.0;
 }
-__device__ __forceinline__ double limit_(const DevParams& P, double v0, double v1,
-                                         double v2, double z0, double z1,
-                                         double z2, int lim) {
-  if (lim == 0) return 0.0;
-  double a = (v2 - v1) / (z2 - z1);
-  double b = (v1 - v0) / (z1 - z0);
-  switch (lim) {
-    case 1: return minmod_(a, b);
-    case 2: return maxmod_(minmod_(a, 2.0 * b), minmod_(2.0 * a, b));
-    case 6: return a;
-    case 7: return b;
-    default: break;
-  }
-  double c = (v2 - v0) / (z2 - z0);
-  if (lim == 3) return minmod_(c, P.theta * minmod_(a, b));
-  if (lim == 4) return minmod_(c, 2.0 * minmod_(a, b));
-  return c;  // 5: centred
-}
-// limit_ from its differences a, b and (when P.lim_c) c, already divided:
-// the same value, with the divisions of all variables of a reconstruction
+// The limiter `lim` from its differences a = (v2 - v1) / (z2 - z1), b =
+// (v1 - v0) / (z1 - z0) and (when P.lim_c) c = (v2 - v0) / (z2 - z0), already
+// divided, so that the divisions of all variables of a reconstruction are
 // issued together rather than one variable's after another's branches.
 __device__ __forceinline__ double limit_pick(const DevParams& P, double a, double b, double c,
                                              int lim) {
@@ -205,7 +188,7 @@ __device__ __forceinline__ double phys(const DevParams& P, const double* qj,
     qp[3] = P.T_ambient;
     return 0.0;
   }
-  double inv_qj1 = 1.0 / qj[0];
+  double inv_qj1 = fdiv(1.0, qj[0]);
   double xs[NS > 0 ? NS : 1];
   double sq = 0.0;
 #pragma unroll
@@ -217,7 +200,7 @@ __device__ __forceinline__ double phys(const DevParams& P, const double* qj,
 #pragma unroll
     for (int i = 0; i < NS; i++) sx += xs[i];
 #pragma unroll
-    for (int i = 0; i < NS; i++) xs[i] = xs[i] / sx;
+    for (int i = 0; i < NS; i++) xs[i] = fdiv(xs[i], sx);
   }
   double xs_tot = 0.0;
 #pragma unroll
@@ -231,38 +214,40 @@ __device__ __forceinline__ double phys(const DevParams& P, const double* qj,
   double T;
   if (qj[0] > P.eps_sing) {
     if (P.energy)
-      T = (qj[3] - 0.5 * (qj[1] * qj[1] + qj[2] * qj[2]) * inv_qj1) / (qj[0] * shm);
+      T = fdiv(qj[3] - 0.5 * (qj[1] * qj[1] + qj[2] * qj[2]) * inv_qj1, qj[0] * shm);
     else
-      T = qj[3] / (qj[0] * shm);
+      T = fdiv(qj[3], qj[0] * shm);
     if (T <= 0.0) T = P.T_ambient;
   } else {
     T = P.T_ambient;
   }
-  double rgc = (xc > kEps) ? ((xc - 0.0) * P.sp_gas_const_a + 0.0) / xc
+  double rgc = (xc > kEps) ? fdiv((xc - 0.0) * P.sp_gas_const_a + 0.0, xc)
                            : P.sp_gas_const_a;
   double inv_rho_c = rgc * T * P.inv_pres;
   double dinv = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) dinv += xs[i] * P.inv_rho_s[i];
   double inv_rhom = dinv + xc * inv_rho_c;
-  double rho_m = 1.0 / inv_rhom;
+  double rho_m = fdiv(1.0, inv_rhom);
   double h = qj[0] * inv_rhom;
   double u, v;
   if (VP) {
     double al[NS > 0 ? NS : 1];
 #pragma unroll
     for (int i = 0; i < NS; i++) al[i] = xs[i] * rho_m * P.inv_rho_s[i];
-    const double rho_c = P.pres / (rgc * T);
+    const double rho_c = fdiv(P.pres, rgc * T);
     const double ua = vp_velocity<NS>(P, h, qj[1], qj[2], rho_m, rho_c, al);
-    u = ua * qj[1] / (sqrt(qj[1] * qj[1] + qj[2] * qj[2]));
-    v = ua * qj[2] / (sqrt(qj[1] * qj[1] + qj[2] * qj[2]));
+    const Rcp rm = rcp_of(fsqrt(qj[1] * qj[1] + qj[2] * qj[2]));
+    u = div_by(ua * qj[1], rm);
+    v = div_by(ua * qj[2], rm);
   } else if (qj[0] > P.eps_sing) {
     u = qj[1] * inv_qj1;
     v = qj[2] * inv_qj1;
   } else {
     double q1sq = qj[0] * qj[0];
-    u = sqrt(2.0) * qj[0] * qj[1] / sqrt(q1sq * q1sq + P.eps_sing4);
-    v = sqrt(2.0) * qj[0] * qj[2] / sqrt(q1sq * q1sq + P.eps_sing4);
+    const Rcp rd = rcp_of(fsqrt(q1sq * q1sq + P.eps_sing4));
+    u = div_by(sqrt(2.0) * qj[0] * qj[1], rd);
+    v = div_by(sqrt(2.0) * qj[0] * qj[2], rd);
   }
   qp[0] = h;
   qp[1] = h * u;
@@ -310,21 +295,23 @@ __device__ __forceinline__ Mixt mixt(const DevParams& P, const double* qp) {
   }
   double r_h = qp[0], r_u = qp[NV], r_v = qp[NV + 1], r_T = qp[3];
   double al[NS > 0 ? NS : 1];
+  const Rcp rh = rcp_of(qp[0]);
 #pragma unroll
-  for (int i = 0; i < NS; i++) al[i] = P.alpha ? qp[4 + i] : qp[4 + i] / qp[0];
+  for (int i = 0; i < NS; i++) al[i] = P.alpha ? qp[4 + i] : div_by(qp[4 + i], rh);
   double at = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) at += al[i];
-  double rho_a = P.pres / (P.sp_gas_const_a * r_T);
-  double rho_c = ((1.0 - 0.0 - at - 0.0) * rho_a + 0.0) / (1.0 - 0.0 - at);
+  double rho_a = fdiv(P.pres, P.sp_gas_const_a * r_T);
+  double rho_c = fdiv((1.0 - 0.0 - at - 0.0) * rho_a + 0.0, 1.0 - 0.0 - at);
   double d = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) d += al[i] * P.rho_s[i];
   double rho_m = (1.0 - at) * rho_c + d;
-  double inv_rhom = 1.0 / rho_m;
-  double rg = (rho_m - P.rho_a_amb) / rho_m * P.grav;
+  const Rcp rr = rcp_of(rho_m);
+  double inv_rhom = div_by(1.0, rr);
+  double rg = div_by(rho_m - P.rho_a_amb, rr) * P.grav;
   double u2 = r_u * r_u + r_v * r_v;
-  m.ri = (u2 > 0.0) ? fmin(1.0e15, rg * r_h / u2) : 0.0;
+  m.ri = (u2 > 0.0) ? fmin(1.0e15, fdiv(rg * r_h, u2)) : 0.0;
   m.rho_m = rho_m;
   m.rho_c = rho_c;
   m.rg = rg;
@@ -337,7 +324,7 @@ __device__ __forceinline__ Mixt mixt(const DevParams& P, const double* qp) {
 #pragma unroll
     for (int i = 0; i < NS; i++) sxs += xs[i];
     double xc = 1.0 - sxs;
-    double c = (xc > kEps) ? ((xc - 0.0) * P.sp_heat_a + 0.0) / xc : P.sp_heat_a;
+    double c = (xc > kEps) ? fdiv((xc - 0.0) * P.sp_heat_a + 0.0, xc) : P.sp_heat_a;
     double dd = 0.0;
 #pragma unroll
     for (int i = 0; i < NS; i++) dd += xs[i] * P.sp_heat_s[i];
@@ -361,25 +348,26 @@ __device__ __forceinline__ void qp2qc(const DevParams& P, const double* qp,
   }
   double r_hu = qp[1], r_hv = qp[2], r_u = qp[NV], r_v = qp[NV + 1], r_T = qp[3];
   double ars[NS > 0 ? NS : 1], al[NS > 0 ? NS : 1], at = 0.0;
+  const Rcp rh = rcp_of(qp[0]);
 #pragma unroll
   for (int i = 0; i < NS; i++) {
-    al[i] = P.alpha ? qp[4 + i] : qp[4 + i] / qp[0];
+    al[i] = P.alpha ? qp[4 + i] : div_by(qp[4 + i], rh);
     at += al[i];
     ars[i] = al[i] * P.rho_s[i];
   }
-  double rho_a = P.pres / (P.sp_gas_const_a * r_T);
-  double rho_c = ((1.0 - 0.0 - at - 0.0) * rho_a + 0.0) / (1.0 - 0.0 - at);
+  double rho_a = fdiv(P.pres, P.sp_gas_const_a * r_T);
+  double rho_c = fdiv((1.0 - 0.0 - at - 0.0) * rho_a + 0.0, 1.0 - 0.0 - at);
   double alphac = 1.0 - at;
   double sar = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) sar += ars[i];
   double rho_m = alphac * rho_c + sar;
-  double inv_rhom = 1.0 / rho_m;
+  double inv_rhom = fdiv(1.0, rho_m);
   double xs[NS > 0 ? NS : 1];
 #pragma unroll
   for (int i = 0; i < NS; i++) xs[i] = ars[i] * inv_rhom;
   double xc = alphac * rho_c * inv_rhom;
-  double shc = (xc > kEps) ? ((xc - 0.0) * P.sp_heat_a + 0.0) / xc : P.sp_heat_a;
+  double shc = (xc > kEps) ? fdiv((xc - 0.0) * P.sp_heat_a + 0.0, xc) : P.sp_heat_a;
   double dsh = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) dsh += xs[i] * P.sp_heat_s[i];
@@ -419,7 +407,7 @@ __device__ __forceinline__ void speeds(const DevParams& P, const double* qp,
     vmin = vel;
     vmax = vel;
   } else {
-    double cel = (DIR == 1) ? sqrt(m.rg * r_h * gc) : sqrt(gc * m.rg * r_h);
+    double cel = (DIR == 1) ? fsqrt(m.rg * r_h * gc) : fsqrt(gc * m.rg * r_h);
     vmin = vel - cel;
     vmax = vel + cel;
   }
@@ -463,9 +451,11 @@ __device__ __forceinline__ void fluxes(const DevParams& P, const double* qc,
   double sf = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) sf += f[4 + i];
-  if ((f[0] > 0.0) && (sf / f[0] > 1.0)) {
+  // (the rounded quotient sf / f0 exceeds 1 exactly when sf exceeds f0 > 0)
+  if ((f[0] > 0.0) && (sf > f[0])) {
+    const Rcp rs = rcp_of(sf);
 #pragma unroll
-    for (int i = 0; i < NS; i++) f[4 + i] = f[4 + i] / sf * f[0];
+    for (int i = 0; i < NS; i++) f[4 + i] = div_by(f[4 + i], rs) * f[0];
   }
 }
 
@@ -481,27 +471,39 @@ __device__ __forceinline__ void kt_flux(const double* fL, const double* fR,
                                         double zvR, double* H) {
   constexpr int NV = 4 + NS;
   const bool same = (aN == aP);
+  // every variable is divided by aP - aN: one reciprocal (speeds below
+  // 1e-290, whose fluxes vanish, are kept off the reciprocal's range)
+  const double den = aP - aN;
+  const Rcp rd = rcp_of(den > 1.0e-290 ? den : 1.0);
+  const double aa = div_by(aP * aN, rd);
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    double avg = same ? 0.0 : (aP * fL[i] - aN * fR[i]) / (aP - aN);
-    H[i] = same ? 0.0 : avg + (aP * aN) / (aP - aN) * (qR[i] - qL[i]);
+    const double avg = div_by(aP * fL[i] - aN * fR[i], rd);
+    H[i] = same ? 0.0 : avg + aa * (qR[i] - qL[i]);
   }
   double s = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) s += H[4 + i];
+  // s / H0 >= 1 (DIR 1) or > 1 (DIR 2): the rounded quotient compares with 1
+  // as s compares with H0
+  const bool zcap = H[0] == 0.0 && s != 0.0 && signbit(s) == signbit(H[0]);
   if (DIR == 1) {
-    if (s / H[0] >= 1.0) {
+    const bool cap = H[0] > 0.0 ? s >= H[0] : H[0] < 0.0 ? s <= H[0] : zcap;
+    if (cap) {
+      const Rcp rH = rcp_of(H[0]);
       double sr = 0.0;
 #pragma unroll
-      for (int i = 0; i < NS; i++) sr += H[4 + i] / H[0];
+      for (int i = 0; i < NS; i++) sr += div_by(H[4 + i], rH);
+      const Rcp rs = rcp_of(sr);
 #pragma unroll
-      for (int i = 0; i < NS; i++) H[4 + i] = H[4 + i] / sr;
+      for (int i = 0; i < NS; i++) H[4 + i] = div_by(H[4 + i], rs);
     }
   } else {
-    if (s / H[0] > 1.0) {
-      double r = s / H[0];
+    const bool cap = H[0] > 0.0 ? s > H[0] : H[0] < 0.0 ? s < H[0] : zcap;
+    if (cap) {
+      const Rcp r = rcp_of(fdiv(s, H[0]));
 #pragma unroll
-      for (int i = 0; i < NS; i++) H[4 + i] = H[4 + i] / r;
+      for (int i = 0; i < NS; i++) H[4 + i] = div_by(H[4 + i], r);
     }
   }
   if (zvL == 0.0 && zvR == 0.0) {
@@ -547,14 +549,15 @@ __device__ __forceinline__ void semi_impl(const DevParams& P, double Bx, double 
   double r_h = qp[0], r_u = qp[NV], r_v = qp[NV + 1];
   Mixt m = mixt<NS, false>(P, qp);
   double r_w = P.slope ? r_u * Bx + r_v * By : 0.0;
-  double mod_vel = sqrt(r_u * r_u + r_v * r_v + r_w * r_w);
+  double mod_vel = fsqrt(r_u * r_u + r_v * r_v + r_w * r_w);
   if (P.rheo_model == 1 && mod_vel > 0.0) {
+    const Rcp rv = rcp_of(mod_vel);
     double cft = P.curv ? Bxx * (r_u * r_u) + 2.0 * Bxy * r_u * r_v + Byy * (r_v * r_v)
                         : 0.0;
-    double tt = P.mu * m.rho_m * (m.rg + cft) * r_h * sqrt(gc);
+    double tt = P.mu * m.rho_m * (m.rg + cft) * r_h * fsqrt(gc);
     tt = fmax(0.0, tt);
-    s1 = 0.0 - tt * r_u / mod_vel;
-    s2 = 0.0 - tt * r_v / mod_vel;
+    s1 = 0.0 - div_by(tt * r_u, rv);
+    s2 = 0.0 - div_by(tt * r_v, rv);
   }
 }
 
@@ -832,26 +835,20 @@ __device__ __forceinline__ SrcTime src_time(const DevParams& P, double time) {
   return r;
 }
 
+// component i of the boundary state of a ring cell with direction vector
+// (vx, vy)
 template <int NS>
-__device__ __forceinline__ void source_bdry(const DevParams& P, const SrcTime& T, double vx,
-                                            double vy, double* sb) {
+__device__ __forceinline__ double source_bdry(const DevParams& P, const SrcTime& T, double vx,
+                                              double vy, int i) {
   constexpr int NV = 4 + NS;
-  if (T.off) {
-#pragma unroll
-    for (int i = 0; i < NV + 2; i++) sb[i] = 0.0;
-    sb[3] = P.T_source;
-    return;
-  }
-  const double tc = T.tc;
-  sb[0] = tc * P.h_source;
-  sb[1] = T.p15 * P.h_source * P.vel_source * vx;
-  sb[2] = T.p15 * P.h_source * P.vel_source * vy;
-  sb[3] = P.T_source;
-#pragma unroll
-  for (int i = 0; i < NS; i++)
-    sb[4 + i] = P.alpha ? P.alphas_source[i] : tc * P.h_source * P.alphas_source[i];
-  sb[NV] = T.p05 * P.vel_source * vx;
-  sb[NV + 1] = T.p05 * P.vel_source * vy;
+  if (i == 3) return P.T_source;
+  if (T.off) return 0.0;
+  if (i == 0) return T.tc * P.h_source;
+  if (i == 1) return T.p15 * P.h_source * P.vel_source * vx;
+  if (i == 2) return T.p15 * P.h_source * P.vel_source * vy;
+  if (i == NV) return T.p05 * P.vel_source * vx;
+  if (i == NV + 1) return T.p05 * P.vel_source * vy;
+  return P.alpha ? P.alphas_source[i - 4] : T.tc * P.h_source * P.alphas_source[i - 4];
 }
 
 }  // namespace imexsw

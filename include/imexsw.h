@@ -415,8 +415,10 @@ const char *imexsw_ensemble_last_error(const imexsw_ensemble *ens);
  * check_solve, downloads, stats).  Owned by the ensemble. */
 imexsw_ctx *imexsw_ensemble_member(imexsw_ensemble *ens, int32_t i);
 
-/* Stencil strip height for all members (4, 8 or 16 rows) and the number of
- * time steps per captured graph (1..1000).  Results do not depend on these. */
+/* Stencil strip height for all members (4, 8 or 16 rows; until it is set, or
+ * found by the autotuner, each step's is fitted to its listed rows) and the
+ * number of time steps per captured graph (1..1000).  Results do not depend on
+ * these. */
 int imexsw_ensemble_set_tuning(imexsw_ensemble *ens, int strip_rows, int graph_steps);
 
 /* Run nsteps batched steps of the main loop for every member (the dt policy
