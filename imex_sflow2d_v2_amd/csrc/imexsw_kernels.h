@@ -2136,9 +2136,9 @@ __device__ __forceinline__ void assembly_checks(const DevParams& P, const DevPtr
 #pragma unroll
   for (int i = 0; i < NS; i++) ssol += q[4 + i];
   if (ssol > q[0]) {
-    if (((ssol - q[0]) / q[0] < 1.0e-10) || (q[0] < kEps)) {
+    if ((fdiv(ssol - q[0], q[0]) < 1.0e-10) || (q[0] < kEps)) {
 #pragma unroll
-      for (int i = 0; i < NS; i++) q[4 + i] = q[4 + i] / ssol * q[0];
+      for (int i = 0; i < NS; i++) q[4 + i] = fdiv(q[4 + i], ssol) * q[0];
       cur = false;
     } else {
       if (counts) atomicAdd(&e[C_SUMS - C_NEWTON_CELLS], 1ull);
@@ -2330,7 +2330,7 @@ __device__ __forceinline__ void local_cell(const DevParams& P, const DevPtrs& D,
     for (int i = 0; i < NS; i++) ssol += q[4 + i];
     if (ssol > q[0] && q[0] < 1.0e-10) {
 #pragma unroll
-      for (int i = 0; i < NS; i++) q[4 + i] = q[4 + i] / ssol * q[0];
+      for (int i = 0; i < NS; i++) q[4 + i] = fdiv(q[4 + i], ssol) * q[0];
     }
     double rg = 0.0;
     if (q[0] > 0.0) {
@@ -2365,7 +2365,7 @@ __device__ __forceinline__ void local_cell(const DevParams& P, const DevPtrs& D,
     if (!(qp_cur && pd_cur)) pd = phys_or_dry<NS, VP>(P, q, qp);
     if (q[0] > 0.0) {
       D.hmax[c] = fmax(hm, qp[0]);
-      const double mv = sqrt(qp[NV] * qp[NV] + qp[NV + 1] * qp[NV + 1]);
+      const double mv = fsqrt(qp[NV] * qp[NV] + qp[NV + 1] * qp[NV + 1]);
       if (qp[0] > 0.001) {
         D.pdynmax[c] = fmax(pm, pd);
         D.modvel[c] = fmax(mvel, mv);

@@ -51,6 +51,14 @@ __device__ __forceinline__ double div_by(double a, const Rcp& d) {
 }
 __device__ __forceinline__ double fdiv(double a, double b) { return div_by(a, rcp_of(b)); }
 
+// a / b for b and the quotient well inside the exponent range and a likewise
+// or +0: no special case to fix up
+__device__ __forceinline__ double quot_n(double a, double b) {
+  const Rcp d = rcp_of(b);
+  const double q = a * d.r;
+  return __builtin_fma(__builtin_fma(-b, q, a), d.r, q);
+}
+
 // sqrt(x) without the scaling of arguments below 2^-767 (the same bits above
 // it, and for zero, infinity and NaN)
 __device__ __forceinline__ double fsqrt(double x) {
@@ -64,20 +72,15 @@ __device__ __forceinline__ double fsqrt(double x) {
   return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0, +infinity
 }
 
-// The special cases are selected after the fact rather than branched
-// around, so that the straight-line code of independent calls can overlap.
-__device__ __forceinline__ double det_log(double x) {
-  // x > 0, finite
-  const int64_t bits0 = __double_as_longlong(x);
-  const bool sub = ((bits0 >> 52) & 0x7ff) == 0;  // subnormal: scale by 2^54
-  const double xs = sub ? x * 18014398509481984.0 : x;
-  const int64_t bits = __double_as_longlong(xs);
-  int e = (int)((bits >> 52) & 0x7ff) - (sub ? 54 : 0) - 1022;  // x = m * 2^e, m in [0.5, 1)
+// log(x), x > 0, normal and finite: x = m 2^e, m in [sqrt(1/2), sqrt(2))
+__device__ __forceinline__ double det_log_n(double x, int de0 = 0) {
+  const int64_t bits = __double_as_longlong(x);
+  int e = (int)((bits >> 52) & 0x7ff) - 1022 + de0;  // m in [0.5, 1)
   double m = __longlong_as_double((bits & 0x000fffffffffffffLL) | 0x3fe0000000000000LL);
   const bool lo = m < 0.70710678118654752440;
   m = lo ? m * 2.0 : m;
   e -= lo ? 1 : 0;
-  const double s = (m - 1.0) / (m + 1.0);
+  const double s = quot_n(m - 1.0, m + 1.0);
   const double s2 = s * s;
   // 1/3 + s2/5 + ... + s2^10/23 by Estrin's scheme (depth 7, not 20)
   const double x2 = s2 * s2, x4 = x2 * x2, x8 = x4 * x4;
@@ -90,13 +93,20 @@ __device__ __forceinline__ double det_log(double x) {
   const double de = (double)e;
   return (de * kLn2Hi + logm) + de * kLn2Lo;
 }
+// The special cases are selected after the fact rather than branched
+// around, so that the straight-line code of independent calls can overlap.
+__device__ __forceinline__ double det_log(double x) {
+  // x > 0, finite; subnormal: scaled by 2^54
+  const bool sub = ((__double_as_longlong(x) >> 52) & 0x7ff) == 0;
+  return det_log_n(sub ? x * 18014398509481984.0 : x, sub ? -54 : 0);
+}
 
-__device__ __forceinline__ double det_exp(double y) {
-  const bool hi = y > 709.0, lo = y < -745.0;
-  const double yc = (hi || lo) ? 0.0 : y;
-  const double n = rint(yc * kInvLn2);
-  const double r = (yc - n * kLn2Hi) - n * kLn2Lo;
-  // sum of r^k / k!, k = 0..14, by Estrin's scheme (depth 8, not 28)
+// 2^n e^r, n = rint(y / ln 2): the sum of r^k / k!, k = 0..14, by Estrin's
+// scheme (depth 8, not 28), scaled exactly (one rounding below the normal
+// range) by the exponent
+__device__ __forceinline__ double det_exp_core(double y) {
+  const double n = rint(y * kInvLn2);
+  const double r = (y - n * kLn2Hi) - n * kLn2Lo;
   const double r2 = r * r, r4 = r2 * r2, r8 = r4 * r4;
   const double a0 = 1.0 + r, a1 = 0.5 + 1.0 / 6.0 * r;
   const double a2 = 1.0 / 24.0 + 1.0 / 120.0 * r, a3 = 1.0 / 720.0 + 1.0 / 5040.0 * r;
@@ -106,13 +116,11 @@ __device__ __forceinline__ double det_exp(double y) {
   const double b0 = a0 + a1 * r2, b1 = a2 + a3 * r2, b2 = a4 + a5 * r2;
   const double b3 = a6 + 1.0 / 87178291200.0 * r2;
   const double p = (b0 + b1 * r4) + (b2 + b3 * r4) * r8;
-  // scale by 2^n in two steps to stay in range near the limits
-  const int ni = (int)n;
-  const int n1 = ni / 2, n2 = ni - n1;
-  const double s1 = __longlong_as_double((int64_t)(1023 + n1) << 52);
-  const double s2 = __longlong_as_double((int64_t)(1023 + n2) << 52);
-  const double v = (p * s1) * s2;
-  return hi ? __longlong_as_double(0x7ff0000000000000LL) : lo ? 0.0 : v;
+  return __builtin_amdgcn_ldexp(p, (int)n);
+}
+__device__ __forceinline__ double det_exp(double y) {
+  const double v = det_exp_core(y);
+  return y > 709.0 ? __longlong_as_double(0x7ff0000000000000LL) : y < -745.0 ? 0.0 : v;
 }
 
 // x**y for x >= 0 (the reference only raises non-negative quantities)

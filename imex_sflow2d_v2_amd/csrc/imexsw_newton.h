@@ -576,10 +576,10 @@ __device__ __forceinline__ bool predictor(const DevParams& P, const double* q0,
     q_si[1] = 0.0;
     q_si[2] = 0.0;
   } else {
-    double m = sqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]);
-    double den = sqrt(f2 * f2 + f3 * f3);
-    q_si[1] = m * f2 / den;
-    q_si[2] = m * f3 / den;
+    double m = fsqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]);
+    const Rcp den = rcp_of(fsqrt(f2 * f2 + f3 * f3));
+    q_si[1] = div_by(m * f2, den);
+    q_si[2] = div_by(m * f3, den);
   }
   return true;
 }
@@ -609,9 +609,11 @@ __device__ __forceinline__ int stage2(const DevParams& P, const double* q0,
     return 0;
   }
   double Rj[NV];
+  const Rcp rdt = rcp_of(dt * 1.0);
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    double si = (q_si[i] - q_fv[i]) / (dt * 1.0);
+    // (only the momenta differ from q_fv)
+    const double si = (i == 1 || i == 2) ? div_by(q_si[i] - q_fv[i], rdt) : 0.0;
     Rj[i] = (D[i] - 0.0) - 1.0 * si;
     q[i] = q_si[i];
   }
@@ -679,10 +681,10 @@ __device__ __forceinline__ int stage2(const DevParams& P, const double* q0,
     q[1] = 0.0;
     q[2] = 0.0;
   } else {
-    double m = sqrt(q[1] * q[1] + q[2] * q[2]);
-    double den = sqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]);
-    q[1] = m * q_si[1] / den;
-    q[2] = m * q_si[2] / den;
+    double m = fsqrt(q[1] * q[1] + q[2] * q[2]);
+    const Rcp den = rcp_of(fsqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]));
+    q[1] = div_by(m * q_si[1], den);
+    q[2] = div_by(m * q_si[2], den);
   }
   return no.iters;
 }
@@ -712,13 +714,14 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
   const double alpha_max = 0.6, hind_exp = 4.65;
   double r_h = qp[0], r_u = qp[NV], r_v = qp[NV + 1];
   double al[NS > 0 ? NS : 1], at = 0.0;
+  const Rcp rh = rcp_of(qp[0]), rdt = rcp_of(dt);
 #pragma unroll
-  for (int i = 0; i < NS; i++) al[i] = P.alpha ? qp[4 + i] : qp[4 + i] / qp[0];
+  for (int i = 0; i < NS; i++) al[i] = P.alpha ? qp[4 + i] : div_by(qp[4 + i], rh);
 #pragma unroll
   for (int i = 0; i < NS; i++) at += al[i];
   double r_w = P.slope ? r_u * Bx + r_v * By : 0.0;
   double mv2 = r_u * r_u + r_v * r_v + r_w * r_w;
-  double mv = sqrt(mv2);
+  double mv = fsqrt(mv2);
   if (P.erosion_coeff > 0.0) {
     double te = P.erosion_coeff * mv * r_h * (1.0 - at);
     double tse = te * (1.0 - P.erodible_porosity);
@@ -726,16 +729,16 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
     for (int i = 0; i < NS; i++) er[i] = P.erodible_fract[i] * tse;
   }
 #pragma unroll
-  for (int i = 0; i < NS; i++) er[i] = fmax(0.0, fmin(er[i], erodible[i] / dt));
+  for (int i = 0; i < NS; i++) er[i] = fmax(0.0, fmin(er[i], div_by(erodible[i], rdt)));
   double tse = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) tse += er[i];
-  double te = tse / (1.0 - P.erodible_porosity);
+  double te = fdiv(tse, 1.0 - P.erodible_porosity);
   double cont_erosion = te * P.erodible_porosity;
   if (at <= P.alphastot_min) return;
   double r_T = qp[3];
   Mixt m = mixt<NS, true>(P, qp);
-  double inv_kin_visc = 1.0 / P.kin_visc_c;
+  double inv_kin_visc = fdiv(1.0, P.kin_visc_c);
   // bottom over mean concentration with the profiles (:4676-4683)
   double dcf[NS > 0 ? NS : 1];
 #pragma unroll
@@ -743,7 +746,7 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
   if (VP && P.bottom_conc) vp_dep_coeffs<NS>(P, r_h, mv, m.rho_c, dcf);
   if (P.settling) {
     // hindered settling factor, the same for every class
-    const double hind = det_pow(1.0 - fmin(1.0, at / alpha_max), hind_exp);
+    const double hind = det_pow(1.0 - fmin(1.0, fdiv(at, alpha_max)), hind_exp);
     double svs[NS > 0 ? NS : 1];
     if (LANES > 1) {
       constexpr int NSL = (NS + LANES - 1) / LANES;
@@ -783,7 +786,7 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
                                                           inv_kin_visc);
         double d = al[i] * sv * dcf[i];
         d = d * hind;
-        dep[i] = fmin(d, r_h * al[i] / dt);
+        dep[i] = fmin(d, div_by(r_h * al[i], rdt));
       }
     }
   }
@@ -794,13 +797,13 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
   double sal = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) sal += al[i];
-  cl = fmin(cl, r_h * fmax(0.0, P.max_packing - sal) / dt);
-  cl = fmin(cl, (r_h * (1.0 - sal) - P.coeff_porosity * (r_h * sal - dt * sdep)) / dt);
+  cl = fmin(cl, div_by(r_h * fmax(0.0, P.max_packing - sal), rdt));
+  cl = fmin(cl, div_by(r_h * (1.0 - sal) - P.coeff_porosity * (r_h * sal - dt * sdep), rdt));
   double T_erodible = P.erod_dep ? r_T : P.T_erodible;
   double air = 0.0;
   if (P.entrain && (r_h > 0.0) && (m.ri > 0.0)) {
-    double ec = 0.075 / sqrt(1.0 + 718.0 * det_pow(m.ri, 2.4));
-    air = ec * sqrt(mv2);
+    double ec = fdiv(0.075, fsqrt(1.0 + 718.0 * det_pow(m.ri, 2.4)));
+    air = ec * fsqrt(mv2);
   }
   double dep_tot = 0.0, ers_tot = 0.0, rdep = 0.0, rers = 0.0, sdc = 0.0, sec = 0.0;
 #pragma unroll
@@ -828,7 +831,7 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
             P.T_ambient * P.sp_heat_a * P.rho_a_amb * air;
 #pragma unroll
   for (int i = 0; i < NS; i++) eq[4 + i] = P.rho_s[i] * (er[i] - dep[i]);
-  topo = (dep_tot - ers_tot) / (1.0 - P.erodible_porosity);
+  topo = fdiv(dep_tot - ers_tot, 1.0 - P.erodible_porosity);
 }
 
 }  // namespace imexsw
