@@ -305,11 +305,17 @@ void drop_ctx_graph(imexsw_ctx* c) {
   }
 }
 
-// Sparse steps when the stencil strips would be one row high (the
-// strip-height rule of k_stencil applied to w computed cells), with N_RK = 2
-// and no harvest (the harvest runs in the dense stage kernel).
+// Sparse steps with few computed cells, N_RK = 2 and no harvest (the harvest
+// runs in the dense stage kernel).  The sparse form spends four lanes on a
+// cell and six wavefronts on a row to shorten one cell's chain, the dense form
+// has twice its latency and a quarter of its work: with the default tuning the
+// line is at 24576 cells (step times, three classes: 10.9k cells 148 us sparse,
+// 171 dense; 16.8k 183 / 171; 42k 325 / 206; two classes: 17k 123 / 135, 27k
+// 148 / 137).  With another tuning it is where its strips become one row high.
+constexpr unsigned long long kSparseCells = 24576;
 bool want_sparse(const imexsw_ctx* c, unsigned long long w) {
   if (c->general || c->D.harvest || c->P.ny < 2) return false;
+  if (c->strip_h == kTileH && c->target_strips == kDefaultStrips) return w < kSparseCells;
   return c->strip_h < 2 ||
          w / (unsigned long long)(kStripW * 2) < (unsigned long long)c->target_strips;
 }
