@@ -7,12 +7,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "imexsw_ctx.h"
@@ -441,8 +443,34 @@ void fill_tableau(int nrk, RkTableau& T) {
   T.stiff = (d1 == 0.0 && d2 == 0.0) ? 1 : 0;
 }
 
-int set_scalar(imexsw_ctx* c, int slot, double v) {
-  HIPCHK(c, hipMemcpyAsync(c->D.scal + slot, &v, sizeof(double), hipMemcpyHostToDevice, c->stream));
+// device-side inputs of a host-called procedure, set by one launch
+struct Put {
+  HostSet h{};
+  Put& scal(int slot, double v) {
+    h.slot[h.n] = slot;
+    h.value[h.n++] = v;
+    return *this;
+  }
+  Put& dt_bits() {
+    h.dt_bits = 1;
+    return *this;
+  }
+  Put& lists() {
+    h.lists = 1;
+    return *this;
+  }
+};
+int put(imexsw_ctx* c, const Put& p) {
+  hipLaunchKernelGGL(k_host_set<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D, p.h);
+  return check_launch(c, "k_host_set");
+}
+
+// the active-cell count and the CFL minimum, written by the device into pinned
+// host memory; waits for the stream
+int get_results(imexsw_ctx* c) {
+  if (!c->h_res) HIPCHK(c, hipHostMalloc((void**)&c->h_res, 2 * sizeof(unsigned long long)));
+  hipLaunchKernelGGL(k_host_get<>, dim3(1), dim3(64), 0, c->stream, c->D, c->h_res);
+  if (check_launch(c, "k_host_get")) return -1;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -463,14 +491,147 @@ int ensure_stage(imexsw_ctx* c, size_t bytes) {
   return 0;
 }
 
+// Pinned memory that large downloads pass through: two chunks for the process,
+// held while contexts exist and used by one download at a time (another that
+// overlaps it copies directly).
+constexpr size_t kPinChunk = (size_t)4 << 20;
+constexpr size_t kPinMin = (size_t)256 << 10;  // downloads below it are copied directly
+struct PinPool {
+  std::mutex mu;       // the chunks
+  std::mutex count_mu; // users
+  int users = 0;
+  char* mem = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  int device = -1;
+};
+PinPool g_pin;
+
+void pin_acquire() {
+  std::lock_guard<std::mutex> lk(g_pin.count_mu);
+  g_pin.users++;
+}
+void pin_drop() {
+  for (hipEvent_t& e : g_pin.ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
+  if (g_pin.mem) (void)hipHostFree(g_pin.mem);
+  g_pin.mem = nullptr;
+  g_pin.device = -1;
+}
+void pin_release() {
+  std::lock_guard<std::mutex> lk(g_pin.count_mu);
+  if (--g_pin.users > 0) return;
+  std::lock_guard<std::mutex> lk2(g_pin.mu);
+  pin_drop();
+}
+
+// The chunks of one download: chunk i of the device memory arrives in half
+// i % 2 of the pinned memory, and the caller and its helpers copy a slice each
+// to the host array.
+struct ChunkCopy {
+  char* host;
+  const char* pin;
+  size_t bytes, chunks;
+  int parts;
+  std::atomic<size_t> ready{0};  // chunks that have arrived
+  std::atomic<size_t> done[2];   // slices copied out of each half, in all
+  std::atomic<bool> stop{false};
+  void slice(size_t i, int part) {
+    const size_t at = i * kPinChunk, len = std::min(kPinChunk, bytes - at);
+    const size_t per = (len / parts + 4095) / 4096 * 4096;
+    const size_t o = std::min(len, per * part);
+    const size_t n = (part == parts - 1) ? len - o : std::min(per, len - o);
+    if (n) std::memcpy(host + at + o, pin + (i & 1) * kPinChunk + o, n);
+    done[i & 1].fetch_add(1, std::memory_order_release);
+  }
+  void help(int part) {
+    for (size_t i = 0; i < chunks; i++) {
+      while (ready.load(std::memory_order_acquire) <= i) {
+        if (stop.load(std::memory_order_acquire)) return;
+        std::this_thread::yield();
+      }
+      slice(i, part);
+    }
+  }
+};
+
+// Device memory to a host array, after the stream's work.  A copy into
+// pageable memory runs at 17 GB/s, and at 10 GB/s into an array whose pages are
+// touched for the first time, as an output array's are; through pinned chunks
+// the transfer overlaps the copy out of them, which several threads make for a
+// large array (they fault its pages side by side).
+int copy_to_host(imexsw_ctx* c, void* host, const void* dev, size_t bytes) {
+  std::unique_lock<std::mutex> lk(g_pin.mu, std::defer_lock);
+  if (bytes < kPinMin || !lk.try_lock()) {
+    HIPCHK(c, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  if (g_pin.device != c->device) pin_drop();
+  if (!g_pin.mem) {
+    HIPCHK(c, hipHostMalloc((void**)&g_pin.mem, 2 * kPinChunk));
+    g_pin.device = c->device;
+    for (hipEvent_t& e : g_pin.ev) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  ChunkCopy w;
+  w.host = static_cast<char*>(host);
+  w.pin = g_pin.mem;
+  w.bytes = bytes;
+  w.chunks = (bytes + kPinChunk - 1) / kPinChunk;
+  w.done[0] = w.done[1] = 0;
+  // one thread for every 4 MiB, at most 8
+  w.parts = (int)std::min<size_t>(8, std::max<size_t>(1, bytes / kPinChunk));
+  std::vector<std::thread> helpers;
+  int started = 1;
+  try {
+    helpers.reserve(w.parts);
+    // (the slices are fixed before the first helper runs: a helper that
+    // cannot be started leaves its slices to the caller)
+    for (int p = 1; p < w.parts; p++, started++) helpers.emplace_back([&w, p] { w.help(p); });
+  } catch (...) {
+  }
+  const char* d = static_cast<const char*>(dev);
+  auto send = [&](size_t i) -> hipError_t {
+    const size_t at = i * kPinChunk;
+    hipError_t e = hipMemcpyAsync(g_pin.mem + (i & 1) * kPinChunk, d + at,
+                                  std::min(kPinChunk, bytes - at), hipMemcpyDeviceToHost,
+                                  c->stream);
+    return e == hipSuccess ? hipEventRecord(g_pin.ev[i & 1], c->stream) : e;
+  };
+  hipError_t err = send(0);
+  if (err == hipSuccess && w.chunks > 1) err = send(1);
+  for (size_t i = 0; err == hipSuccess && i < w.chunks; i++) {
+    err = hipEventSynchronize(g_pin.ev[i & 1]);
+    if (err != hipSuccess) break;
+    w.ready.store(i + 1, std::memory_order_release);
+    w.slice(i, 0);
+    for (int p = started; p < w.parts; p++) w.slice(i, p);
+    if (i + 2 < w.chunks) {
+      // the half is free once every slice of this chunk is out of it
+      const size_t want = (size_t)w.parts * (i / 2 + 1);
+      while (w.done[i & 1].load(std::memory_order_acquire) < want) std::this_thread::yield();
+      err = send(i + 2);
+    }
+  }
+  if (err != hipSuccess) w.stop.store(true, std::memory_order_release);
+  for (std::thread& t : helpers) t.join();
+  if (err != hipSuccess) {
+    (void)hipStreamSynchronize(c->stream);
+    return fail(c, "download: %s", hipGetErrorString(err));
+  }
+  return 0;
+}
+
 // host (nvar, nx, ny) Fortran array -> nvar device planes
-int upload_aos(imexsw_ctx* c, const double* host, int nvar, double* dst) {
+// (wait: for the copy and the conversion)
+int upload_aos(imexsw_ctx* c, const double* host, int nvar, double* dst, bool wait = true) {
   const size_t n = (size_t)nvar * c->P.nx * c->P.ny;
   if (ensure_stage(c, n * sizeof(double))) return -1;
   HIPCHK(c, hipMemcpyAsync(c->stage, host, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL(k_aos_to_planes<>, c->grid_tiles, dim3(256), 0, c->stream, c->P, c->stage, nvar, dst);
   if (check_launch(c, "k_aos_to_planes")) return -1;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (wait) HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
 
@@ -480,23 +641,34 @@ int download_aos(imexsw_ctx* c, const double* src, int nvar, double* host) {
   hipLaunchKernelGGL(k_planes_to_aos<>, c->grid_tiles, dim3(256), 0, c->stream, c->P, src, nvar,
                      c->stage, 0, c->P.ny);
   if (check_launch(c, "k_planes_to_aos")) return -1;
-  HIPCHK(c, hipMemcpyAsync(host, c->stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  return 0;
+  return copy_to_host(c, host, c->stage, n * sizeof(double));
 }
 
 // host (nx, ny) Fortran plane <-> device plane with pitch
 template <typename T>
-int upload_plane(imexsw_ctx* c, const T* host, T* dst, int w, int h, size_t dpitch_elems) {
-  HIPCHK(c, hipMemcpy2DAsync(dst, dpitch_elems * sizeof(T), host, (size_t)w * sizeof(T),
-                             (size_t)w * sizeof(T), h, hipMemcpyHostToDevice, c->stream));
+int upload_plane(imexsw_ctx* c, const T* host, T* dst) {
+  const size_t n = (size_t)c->P.nx * c->P.ny;
+  if (ensure_stage(c, n * sizeof(T))) return -1;
+  T* st = reinterpret_cast<T*>(c->stage);
+  HIPCHK(c, hipMemcpyAsync(st, host, n * sizeof(T), hipMemcpyHostToDevice, c->stream));
+  hipLaunchKernelGGL(k_plane_unpack<T>, c->grid_tiles, dim3(256), 0, c->stream, c->P, st, dst);
+  if (check_launch(c, "k_plane_unpack")) return -1;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
 template <typename T>
-int download_plane(imexsw_ctx* c, const T* src, T* host, int w, int h, size_t spitch_elems) {
-  HIPCHK(c, hipMemcpy2DAsync(host, (size_t)w * sizeof(T), src, spitch_elems * sizeof(T),
-                             (size_t)w * sizeof(T), h, hipMemcpyDeviceToHost, c->stream));
+int download_plane(imexsw_ctx* c, const T* src, T* host) {
+  const size_t n = (size_t)c->P.nx * c->P.ny;
+  if (ensure_stage(c, n * sizeof(T))) return -1;
+  T* st = reinterpret_cast<T*>(c->stage);
+  hipLaunchKernelGGL(k_plane_pack<T>, c->grid_tiles, dim3(256), 0, c->stream, c->P, src, st);
+  if (check_launch(c, "k_plane_pack")) return -1;
+  return copy_to_host(c, host, st, n * sizeof(T));
+}
+// the staggered planes (set-up only): w x h values, pitch d
+int upload_staggered(imexsw_ctx* c, const double* host, double* dst, int w, int h, size_t d) {
+  HIPCHK(c, hipMemcpy2DAsync(dst, d * sizeof(double), host, (size_t)w * sizeof(double),
+                             (size_t)w * sizeof(double), h, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -557,6 +729,7 @@ int imexsw_create(const imexsw_params* params, imexsw_ctx** out) {
     if (p.limiter[i] < 0 || p.limiter[i] > 7) return fail(nullptr, "limiter out of range");
 
   imexsw_ctx* c = new imexsw_ctx();
+  pin_acquire();
   c->p = p;
   c->ns = p.n_solid;
   c->nv = 4 + p.n_solid;
@@ -663,6 +836,7 @@ int imexsw_create(const imexsw_params* params, imexsw_ctx** out) {
 
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     fail(nullptr, "hipStreamCreate failed");
+    pin_release();
     delete c;
     return -1;
   }
@@ -767,25 +941,27 @@ void imexsw_destroy(imexsw_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   if (c->h_cnt) (void)hipHostFree(c->h_cnt);
   if (c->h_done) (void)hipHostFree(c->h_done);
+  if (c->h_res) (void)hipHostFree(c->h_res);
   if (c->D.harvest) (void)hipFree(c->D.harvest);
   for (void* p : c->allocs) (void)hipFree(p);
   if (c->stage) (void)hipFree(c->stage);
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  pin_release();
   delete c;
 }
 
 int imexsw_set_topography(imexsw_ctx* c, const double* B_cent, const uint8_t* nodata) {
   if (!c || !B_cent) return fail(c, "null argument");
   const DevParams& P = c->P;
-  if (upload_plane(c, B_cent, c->D.B, P.nx, P.ny, P.pitch)) return -1;
+  if (upload_plane(c, B_cent, c->D.B)) return -1;
   if (nodata) {
     uint8_t* nd = nullptr;
     if (!c->D.nodata) {
       if (dalloc(c, &nd, c->plane)) return -1;
       c->D.nodata = nd;
     }
-    if (upload_plane(c, nodata, const_cast<uint8_t*>(c->D.nodata), P.nx, P.ny, P.pitch)) return -1;
+    if (upload_plane(c, nodata, const_cast<uint8_t*>(c->D.nodata))) return -1;
   }
   if (run_topo(c, 0)) return -1;
   c->d_valid = false;
@@ -800,19 +976,19 @@ int imexsw_set_geometry(imexsw_ctx* c, const double* B_cent, const double* Bx,
   if (!c || !B_cent) return fail(c, "null argument");
   const DevParams& P = c->P;
   DevPtrs& D = c->D;
-  if (upload_plane(c, B_cent, D.B, P.nx, P.ny, P.pitch)) return -1;
-  if (Bx && upload_plane(c, Bx, D.Bx, P.nx, P.ny, P.pitch)) return -1;
-  if (By && upload_plane(c, By, D.By, P.nx, P.ny, P.pitch)) return -1;
+  if (upload_plane(c, B_cent, D.B)) return -1;
+  if (Bx && upload_plane(c, Bx, D.Bx)) return -1;
+  if (By && upload_plane(c, By, D.By)) return -1;
   if (D.Bxx) {
-    if (Bxx && upload_plane(c, Bxx, D.Bxx, P.nx, P.ny, P.pitch)) return -1;
-    if (Bxy && upload_plane(c, Bxy, D.Bxy, P.nx, P.ny, P.pitch)) return -1;
-    if (Byy && upload_plane(c, Byy, D.Byy, P.nx, P.ny, P.pitch)) return -1;
+    if (Bxx && upload_plane(c, Bxx, D.Bxx)) return -1;
+    if (Bxy && upload_plane(c, Bxy, D.Bxy)) return -1;
+    if (Byy && upload_plane(c, Byy, D.Byy)) return -1;
   }
   if (D.gcoef) {
-    if (gcoef && upload_plane(c, gcoef, D.gcoef, P.nx, P.ny, P.pitch)) return -1;
-    if (dgdx && upload_plane(c, dgdx, D.dgdx, P.nx, P.ny, P.pitch)) return -1;
-    if (gsx && upload_plane(c, gsx, D.gsx, P.nx + 1, P.ny, P.pitch + 1)) return -1;
-    if (gsy && upload_plane(c, gsy, D.gsy, P.nx, P.ny + 1, P.pitch)) return -1;
+    if (gcoef && upload_plane(c, gcoef, D.gcoef)) return -1;
+    if (dgdx && upload_plane(c, dgdx, D.dgdx)) return -1;
+    if (gsx && upload_staggered(c, gsx, D.gsx, P.nx + 1, P.ny, P.pitch + 1)) return -1;
+    if (gsy && upload_staggered(c, gsy, D.gsy, P.nx, P.ny + 1, P.pitch)) return -1;
   }
   if (nodata) {
     uint8_t* nd = nullptr;
@@ -820,7 +996,7 @@ int imexsw_set_geometry(imexsw_ctx* c, const double* B_cent, const double* Bx,
       if (dalloc(c, &nd, c->plane)) return -1;
       D.nodata = nd;
     }
-    if (upload_plane(c, nodata, const_cast<uint8_t*>(D.nodata), P.nx, P.ny, P.pitch)) return -1;
+    if (upload_plane(c, nodata, const_cast<uint8_t*>(D.nodata))) return -1;
   }
   c->d_valid = false;
   return 0;
@@ -861,7 +1037,7 @@ int imexsw_set_source(imexsw_ctx* c, const int32_t* source_cell, const uint8_t* 
     D.sinfo = si;
     D.sring = sr;
   }
-  if (upload_plane(c, info.data(), const_cast<uint8_t*>(D.sinfo), P.nx, P.ny, P.pitch)) return -1;
+  if (upload_plane(c, info.data(), const_cast<uint8_t*>(D.sinfo))) return -1;
   if (upload_aos(c, ring.data(), 2, const_cast<double*>(D.sring))) return -1;
   HIPCHK(c, hipMemsetAsync(D.tile_dirty, 1, (size_t)c->n_tiles, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -871,7 +1047,7 @@ int imexsw_set_source(imexsw_ctx* c, const int32_t* source_cell, const uint8_t* 
 
 int imexsw_upload_q(imexsw_ctx* c, const double* q) {
   if (!c || !q) return fail(c, "null argument");
-  if (upload_aos(c, q, c->nv, c->D.q)) return -1;
+  if (upload_aos(c, q, c->nv, c->D.q, false)) return -1;
   hipLaunchKernelGGL(k_sflag<>, c->grid_tiles, dim3(256), 0, c->stream, c->P, c->D);
   if (check_launch(c, "k_sflag")) return -1;
   if (c->D.qpp) {
@@ -898,34 +1074,23 @@ int imexsw_upload_erosion(imexsw_ctx* c, const double* erodible, const double* d
   if (erodible && upload_aos(c, erodible, c->ns, c->D.erodible)) return -1;
   for (int i = 0; i < c->ns; i++) {
     const size_t off = (size_t)i * P.nx * P.ny;
-    if (deposit && upload_plane(c, deposit + off, c->D.deposit + i * c->plane, P.nx, P.ny, P.pitch)) return -1;
-    if (erosion && upload_plane(c, erosion + off, c->D.erosion + i * c->plane, P.nx, P.ny, P.pitch)) return -1;
+    if (deposit && upload_plane(c, deposit + off, c->D.deposit + i * c->plane)) return -1;
+    if (erosion && upload_plane(c, erosion + off, c->D.erosion + i * c->plane)) return -1;
   }
   return 0;
 }
 
 int imexsw_check_solve(imexsw_ctx* c, int solve_all, double t, int32_t* solve_cells) {
   if (!c) return fail(c, "null argument");
-  if (set_scalar(c, S_T, t)) return -1;
-  if (set_scalar(c, S_DONE, 0.0)) return -1;
-  HIPCHK(c, hipMemsetAsync(c->D.counters + C_COMPUTE_CELLS * kSlots, 0,
-                           kSlots * sizeof(unsigned long long), c->stream));
-  HIPCHK(c, hipMemsetAsync(c->D.counters + C_TILES * kSlots, 0,
-                           2 * kSlots * sizeof(unsigned long long), c->stream));  // tiles, rows
-  HIPCHK(c, hipMemsetAsync(c->D.counters + C_CELLS * kSlots, 0,
-                           kSlots * sizeof(unsigned long long), c->stream));
+  if (put(c, Put().scal(S_T, t).scal(S_DONE, 0.0).lists())) return -1;
   if (run_mask(c, solve_all)) return -1;
   // the mask now reflects this call's solve_all: the next step's mask
   // scans every tile again
   HIPCHK(c, hipMemsetAsync(c->D.tile_dirty, 1, (size_t)c->n_tiles, c->stream));
   c->d_valid = false;
   if (solve_cells) {
-    unsigned long long v[kSlots], n = 0;
-    HIPCHK(c, hipMemcpyAsync(v, c->D.counters + C_SOLVE_CELLS * kSlots, sizeof v,
-                             hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < kSlots; i++) n += v[i];
-    *solve_cells = (int32_t)n;
+    if (get_results(c)) return -1;
+    *solve_cells = (int32_t)c->h_res[0];
   }
   return 0;
 }
@@ -934,15 +1099,11 @@ int imexsw_timestep(imexsw_ctx* c, double* dt) {
   if (!c || !dt) return fail(c, "null argument");
   // the procedures called one at a time run whatever state imexsw_advance
   // stopped in
-  if (set_scalar(c, S_DONE, 0.0)) return -1;
-  const unsigned long long init = (unsigned long long)(*(const long long*)&c->P.max_dt);
-  HIPCHK(c, hipMemcpyAsync(c->D.dt_bits, &init, sizeof init, hipMemcpyHostToDevice, c->stream));
+  if (put(c, Put().scal(S_DONE, 0.0).dt_bits())) return -1;
   if (run_stencil(c, c->P.cfl != -1.0)) return -1;
-  unsigned long long bits = 0;
-  HIPCHK(c, hipMemcpyAsync(&bits, c->D.dt_bits, sizeof bits, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (get_results(c)) return -1;
   double v;
-  std::memcpy(&v, &bits, sizeof v);
+  std::memcpy(&v, &c->h_res[1], sizeof v);
   *dt = (c->P.cfl != -1.0) ? v : c->P.max_dt;
   return 0;
 }
@@ -950,7 +1111,7 @@ int imexsw_timestep(imexsw_ctx* c, double* dt) {
 int imexsw_rk_step(imexsw_ctx* c, double t, double dt) {
   if (!c) return fail(c, "null argument");
   if (!(dt > 0.0)) return fail(c, "dt must be positive");
-  if (set_scalar(c, S_T, t) || set_scalar(c, S_DT, dt) || set_scalar(c, S_DONE, 0.0)) return -1;
+  if (put(c, Put().scal(S_T, t).scal(S_DT, dt).scal(S_DONE, 0.0))) return -1;
   if (c->general) {
     if (init_stages(c)) return -1;
     if (!c->d_valid && run_stencil(c, 0)) return -1;
@@ -966,7 +1127,7 @@ int imexsw_rk_step(imexsw_ctx* c, double t, double dt) {
 
 int imexsw_erosion_deposition(imexsw_ctx* c, double dt) {
   if (!c) return fail(c, "null argument");
-  if (set_scalar(c, S_DT, dt) || set_scalar(c, S_DONE, 0.0)) return -1;
+  if (put(c, Put().scal(S_DT, dt).scal(S_DONE, 0.0))) return -1;
   if (run_local(c, OP_EROSION, K_EROSION)) return -1;
   c->d_valid = false;
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -983,7 +1144,7 @@ int imexsw_topography_reconstruction(imexsw_ctx* c) {
 
 int imexsw_post_step(imexsw_ctx* c, double sums[4]) {
   if (!c) return fail(c, "null argument");
-  if (set_scalar(c, S_DONE, 0.0)) return -1;
+  if (put(c, Put().scal(S_DONE, 0.0))) return -1;
   if (sums)
     HIPCHK(c, hipMemsetAsync(c->D.tile_sums, 0, 4 * (size_t)c->n_tiles * kTileH * sizeof(double),
                              c->stream));
@@ -1120,16 +1281,15 @@ int imexsw_download(imexsw_ctx* c, double* q, double* qp, double* hmax, double* 
     NS_SWITCH(c->ns, CALL)
 #undef CALL
     if (check_launch(c, "k_qp_out")) return -1;
-    HIPCHK(c, hipMemcpyAsync(qp, c->stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (copy_to_host(c, qp, c->stage, n * sizeof(double))) return -1;
   }
-  if (hmax && download_plane(c, c->D.hmax, hmax, P.nx, P.ny, P.pitch)) return -1;
-  if (pdynmax && download_plane(c, c->D.pdynmax, pdynmax, P.nx, P.ny, P.pitch)) return -1;
-  if (mod_vel_max && download_plane(c, c->D.modvel, mod_vel_max, P.nx, P.ny, P.pitch)) return -1;
+  if (hmax && download_plane(c, c->D.hmax, hmax)) return -1;
+  if (pdynmax && download_plane(c, c->D.pdynmax, pdynmax)) return -1;
+  if (mod_vel_max && download_plane(c, c->D.modvel, mod_vel_max)) return -1;
   const int nl = P.n_thk * P.n_pdyn;
   if (vuln && nl > 0) {
     std::vector<uint32_t> bits((size_t)P.nx * P.ny);
-    if (download_plane(c, c->D.vuln, bits.data(), P.nx, P.ny, P.pitch)) return -1;
+    if (download_plane(c, c->D.vuln, bits.data())) return -1;
     for (size_t cc = 0; cc < bits.size(); cc++)
       for (int i = 0; i < nl; i++) vuln[cc * nl + i] = (bits[cc] >> i) & 1u;
   }
@@ -1180,17 +1340,17 @@ int imexsw_download_erosion(imexsw_ctx* c, double* erodible, double* deposit, do
     if (erodible && download_aos(c, c->D.erodible, c->ns, erodible)) return -1;
     for (int i = 0; i < c->ns; i++) {
       const size_t off = (size_t)i * P.nx * P.ny;
-      if (deposit && download_plane(c, c->D.deposit + i * c->plane, deposit + off, P.nx, P.ny, P.pitch)) return -1;
-      if (erosion && download_plane(c, c->D.erosion + i * c->plane, erosion + off, P.nx, P.ny, P.pitch)) return -1;
+      if (deposit && download_plane(c, c->D.deposit + i * c->plane, deposit + off)) return -1;
+      if (erosion && download_plane(c, c->D.erosion + i * c->plane, erosion + off)) return -1;
     }
   }
-  if (B_cent && download_plane(c, c->D.B, B_cent, P.nx, P.ny, P.pitch)) return -1;
+  if (B_cent && download_plane(c, c->D.B, B_cent)) return -1;
   return 0;
 }
 
 int imexsw_download_mask(imexsw_ctx* c, uint8_t* mask) {
   if (!c || !mask) return fail(c, "null argument");
-  if (download_plane(c, c->D.mask, mask, c->P.nx, c->P.ny, c->P.pitch)) return -1;
+  if (download_plane(c, c->D.mask, mask)) return -1;
   const size_t n = (size_t)c->P.nx * c->P.ny;
   for (size_t i = 0; i < n; i++) mask[i] &= M_ACTIVE;  // solve_mask only
   return 0;

@@ -68,6 +68,7 @@ struct imexsw_ctx {
   int64_t sparse_steps = 0;
   unsigned long long* h_cnt = nullptr;  // pinned: 2 x kSlots computed-cell counters
   double* h_done = nullptr;             // pinned: 2 copies of the run's done flag
+  unsigned long long* h_res = nullptr;  // pinned: active cells, CFL minimum
   hipEvent_t cnt_ev[2] = {nullptr, nullptr};
   // captured kGraphSteps-step graphs of imexsw_advance (dense, sparse) and
   // what they captured

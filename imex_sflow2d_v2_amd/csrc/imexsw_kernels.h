@@ -2770,6 +2770,53 @@ __global__ void k_aos_to_planes(DevParams P, const double* __restrict__ src, int
   for (int i = 0; i < nvar; i++) dst[i * pl + cidx(P, j, k)] = src[s + i];
 }
 
+// one plane <-> contiguous rows of nx values (a 2-D copy to or from pageable
+// host memory goes row by row, 8 us each: 1.2 ms for a plane of 200 x 151)
+template <typename T>
+__global__ void k_plane_pack(DevParams P, const T* __restrict__ src, T* __restrict__ dst) {
+  const int j = blockIdx.x * kTileX + (threadIdx.x & 63);
+  const int k = blockIdx.y * kTileY + (threadIdx.x >> 6);
+  if (j < P.nx && k < P.ny) dst[(size_t)k * P.nx + j] = src[cidx(P, j, k)];
+}
+template <typename T>
+__global__ void k_plane_unpack(DevParams P, const T* __restrict__ src, T* __restrict__ dst) {
+  const int j = blockIdx.x * kTileX + (threadIdx.x & 63);
+  const int k = blockIdx.y * kTileY + (threadIdx.x >> 6);
+  if (j < P.nx && k < P.ny) dst[cidx(P, j, k)] = src[(size_t)k * P.nx + j];
+}
+
+// What a host-called procedure sets before its kernels, in one launch of 64
+// threads: scalars, the CFL accumulator, the mask's counters and lists.
+struct HostSet {
+  int n;            // scalars
+  int slot[4];
+  double value[4];
+  int dt_bits, lists;
+};
+template <int = 0>
+__global__ void k_host_set(DevParams P, DevPtrs D, HostSet h) {
+  const int i = threadIdx.x;
+  if (i < h.n) D.scal[h.slot[i]] = h.value[i];
+  if (h.dt_bits && i == 0) *D.dt_bits = (unsigned long long)__double_as_longlong(P.max_dt);
+  if (h.lists) {
+    *ctr(D, C_COMPUTE_CELLS, i) = 0;
+    *ctr(D, C_TILES, i) = 0;
+    *ctr(D, C_ROWS, i) = 0;
+    *ctr(D, C_CELLS, i) = 0;
+  }
+}
+// What such a procedure returns, written to host memory: the active cells and
+// the CFL minimum.
+template <int = 0>
+__global__ void k_host_get(DevPtrs D, unsigned long long* out) {
+  unsigned long long n = *ctr(D, C_SOLVE_CELLS, threadIdx.x);
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+  if (threadIdx.x == 0) {
+    out[0] = n;
+    out[1] = *D.dt_bits;
+  }
+}
+
 // state flags of the current state (after an upload)
 template <int = 0>
 __global__ void k_sflag(DevParams P, DevPtrs D) {
