@@ -205,12 +205,13 @@ int run_mask_general(imexsw_ctx* c, int solve_all) {
 
 // partial: rescan only the dirty tiles (the step loop)
 int run_mask(imexsw_ctx* c, int solve_all, int partial = 0) {
-  if (c->general) return run_mask_general(c, solve_all);
+  // two dilations are k_mask's whatever the path
+  if (c->general && c->P.nrk != 2) return run_mask_general(c, solve_all);
   {
     Timed tm(c, K_MASK);
     const dim3 grid(c->grid_mask.x, (c->grid_mask.y + kMaskGroup - 1) / kMaskGroup);
     hipLaunchKernelGGL(k_mask<>, grid, dim3(64 * kMaskGroup), 0, c->stream, c->P, c->D,
-                       solve_all, partial);
+                       solve_all, partial, c->general ? 1 : 0);
   }
   return check_launch(c, "k_mask");
 }
@@ -241,7 +242,8 @@ int run_topo(imexsw_ctx* c, int sparse) {
 // assembly.  policy: dt from the time-step policy, else the scalar dt.
 int run_stages(imexsw_ctx* c, int policy) {
   const RkTableau& T = c->tab;
-  for (int st = 0; st < T.nrk; st++) {
+  // N_RK = 2: one launch for the second stage and the assembly
+  for (int st = (T.nrk == 2) ? 1 : 0; st < T.nrk; st++) {
     {
       Timed tm(c, K_LOCAL);
 #define CALL(N) launch_stage<N>(c, st, policy)
@@ -252,6 +254,7 @@ int run_stages(imexsw_ctx* c, int policy) {
     const bool same_as_cfl_pass = st == 0 && T.a_dirk[0][0] == 0.0;
     if (T.omega_tilde[st] > 0.0 && !same_as_cfl_pass && run_stencil(c, 0, false, st)) return -1;
   }
+  if (T.nrk == 2) return 0;
   {
     Timed tm(c, K_LOCAL);
 #define CALL(N) launch_assemble<N>(c, policy)
@@ -263,6 +266,7 @@ int run_stages(imexsw_ctx* c, int policy) {
 
 // every stage state starts as q (what inactive cells keep)
 int init_stages(imexsw_ctx* c) {
+  if (c->tab.nrk == 2) return 0;  // no stage state is read back
   const int grid = (int)std::min<size_t>((c->plane * c->nv + 255) / 256, (size_t)c->n_cu * 8);
   hipLaunchKernelGGL(kg_stage_init<>, dim3(grid), dim3(256), 0, c->stream, c->P, c->D.scal,
                      c->D.q, c->G.qrk, c->tab.nrk);
@@ -276,11 +280,11 @@ int init_stages(imexsw_ctx* c) {
 int enqueue_step(imexsw_ctx* c, bool commit_prev) {
   {
     Timed tm(c, K_DTPOLICY);
-    hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(1), 0, c->stream, c->P, c->D,
+    hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D,
                        commit_prev ? 1 : 0, 1);
   }
   if (c->general) {
-    if (run_mask(c, 0) || init_stages(c)) return -1;
+    if (run_mask(c, 0, 1) || init_stages(c)) return -1;
     if (run_stencil(c, c->P.cfl != -1.0)) return -1;
     if (run_stages(c, 1)) return -1;
     if (run_local(c, OP_EROSION | OP_POST | OP_POLICY, K_LOCAL)) return -1;
@@ -294,7 +298,7 @@ int enqueue_step(imexsw_ctx* c, bool commit_prev) {
   return check_launch(c, "k_step_begin");
 }
 int end_steps(imexsw_ctx* c) {
-  hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(1), 0, c->stream, c->P, c->D, 1, 0);
+  hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D, 1, 0);
   return check_launch(c, "k_step_begin");
 }
 
@@ -882,15 +886,17 @@ int imexsw_create(const imexsw_params* params, imexsw_ctx** out) {
     // the tableau-driven stage pipeline (N_RK != 2, and every N_RK with
     // the profile closures or rheology models 6 and 8): stage states,
     // residuals and implicit terms of every stage, two byte planes for the
-    // mask dilation
+    // mask dilation; with N_RK = 2 the first stage's residual alone
     c->general = true;
     fill_tableau(p.n_rk, c->tab);
-    const size_t sp = (size_t)c->nv * pl * p.n_rk;
-    rc |= dalloc(c, &c->G.qrk, sp);
-    rc |= dalloc(c, &c->G.Dx, sp);
-    rc |= dalloc(c, &c->G.Im, sp);
-    rc |= dalloc(c, &c->G.ma, pl);
-    rc |= dalloc(c, &c->G.mb, pl);
+    const size_t sp = (size_t)c->nv * pl;
+    rc |= dalloc(c, &c->G.Dx, p.n_rk == 2 ? sp : sp * p.n_rk);
+    if (p.n_rk != 2) {
+      rc |= dalloc(c, &c->G.qrk, sp * p.n_rk);
+      rc |= dalloc(c, &c->G.Im, sp * p.n_rk);
+      rc |= dalloc(c, &c->G.ma, pl);
+      rc |= dalloc(c, &c->G.mb, pl);
+    }
   }
   rc |= dalloc(c, &D.tile_sums, 4 * (size_t)c->n_tiles * kTileH);
   rc |= dalloc(c, &D.tile_flag, (size_t)c->n_tiles);

@@ -262,9 +262,11 @@ __device__ __forceinline__ unsigned lane_read(unsigned v, int src) {
 // bytes and counts (nothing within reach changed state since its last scan,
 // so neither can have changed, and it has no cell to compute).  The
 // active-cell counter is a running total kept by per-tile differences.
+// `all`: every active cell is computed (the tableau-driven path).
 __device__ __forceinline__ unsigned mask_tile(const DevParams& P, const DevPtrs& D, int tx,
                                               int tyy, int tiles_x, int solve_all,
-                                              bool clean, unsigned* comp_out = nullptr) {
+                                              bool clean, bool all,
+                                              unsigned* comp_out = nullptr) {
   constexpr int LH = kTileH + 4;
   const int lane = threadIdx.x & 63;
   const int tile = tyy * tiles_x + tx;
@@ -339,7 +341,7 @@ __device__ __forceinline__ unsigned mask_tile(const DevParams& P, const DevPtrs&
   }
   const unsigned rows16 = ((1u << kTileH) - 1u) << 2;
   act &= rows16;
-  const unsigned comp = act & busy;
+  const unsigned comp = all ? act : act & busy;
   if (own) {
 #pragma unroll
     for (int rr = 0; rr < kTileH; rr++) {
@@ -449,7 +451,7 @@ __device__ __forceinline__ void append_group(const ListSink& L, int tile, unsign
 // grid (tiles_x, ceil(tiles_y / kMaskGroup)), kMaskGroup wavefronts
 template <int = 0>
 __global__ void __launch_bounds__(64 * kMaskGroup) k_mask(DevParams P, DevPtrs D,
-                                                          int solve_all, int partial) {
+                                                          int solve_all, int partial, int all) {
   const int tiles_x = (P.nx + kStripW - 1) / kStripW;
   const int tiles_y = (P.ny + kTileH - 1) / kTileH;
   const int w = threadIdx.x >> 6;
@@ -484,9 +486,10 @@ __global__ void __launch_bounds__(64 * kMaskGroup) k_mask(DevParams P, DevPtrs D
   const int tyy = blockIdx.y * kMaskGroup + w;
   unsigned rows_m = 0, comp = 0;
   if (tyy < tiles_y)
-    rows_m = mask_tile(P, D, blockIdx.x, tyy, tiles_x, solve_all, clean, &comp);
+    rows_m = mask_tile(P, D, blockIdx.x, tyy, tiles_x, solve_all, clean, all, &comp);
   const int j = blockIdx.x * kStripW - 2 + (int)(threadIdx.x & 63);
-  append_group<kMaskGroup>(own_sink(D), tyy * tiles_x + blockIdx.x, rows_m, comp,
+  // (the tableau-driven path has no use for the cell list)
+  append_group<kMaskGroup>(own_sink(D), tyy * tiles_x + blockIdx.x, rows_m, all ? 0u : comp,
                            (int)cidx(P, max(j, 0), tyy * kTileH), (int)P.pitch,
                            (long long)P.nx * P.ny);
 }
@@ -2068,14 +2071,61 @@ __device__ __forceinline__ void reset_member(const DevParams& P, const DevPtrs& 
 // Between two steps of imexsw_advance: commit the previous step (its time
 // step policy, t = t + dt, counters) when `commit`, then reset the per-step
 // counters for the next one.  With commit and without reset: the end of the
-// last step.
+// last step.  One wavefront, a counter slot per lane: the same as
+// dtpolicy_member, advance_member and reset_member with every load in one
+// round (one thread walking the slots took 4.5 us).
 template <int = 0>
-__global__ void k_step_begin(DevParams P, DevPtrs D, int commit, int reset) {
+__global__ void __launch_bounds__(64) k_step_begin(DevParams P, DevPtrs D, int commit,
+                                                   int reset) {
+  const int lane = threadIdx.x;
+  double done = D.scal[S_DONE];
+  unsigned long long n = *ctr(D, C_SOLVE_CELLS, lane), nc = *ctr(D, C_COMPUTE_CELLS, lane);
+  unsigned long long c0 = *ctr(D, C_STEPS, 0), c1 = *ctr(D, C_ACTIVE_UPD, 0),
+                     c2 = *ctr(D, C_COMPUTE_UPD, 0);
+  double t = D.scal[S_T], dt_old = D.scal[S_DT_OLD];
+  const StepDt r = step_dt(P, D);
+  pin(done);
+  pin(n);
+  pin(nc);
+  pin(t);
+  pin(dt_old);
+  if (done != 0.0) return;
   if (commit) {
-    dtpolicy_member(P, D);
-    advance_member(D);
+    if (r.done) {
+      if (lane == 0) D.scal[S_DONE] = 1.0;
+      return;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      n += __shfl_xor(n, off, 64);
+      nc += __shfl_xor(nc, off, 64);
+    }
+    const double t1 = t + r.dt;
+    // the run stops once t reaches the output time (t_output, snapped to t_end
+    // by the policy), where the reference's loop writes its output
+    const bool stop = t1 >= r.t_out;
+    if (lane == 0) {
+      D.scal[S_DT_CFL] = r.dt_cfl;
+      D.scal[S_DT_OLD_OLD] = dt_old;
+      D.scal[S_DT_OLD] = r.dt;
+      D.scal[S_DT] = r.dt;
+      D.scal[S_T_OUT] = r.t_out;
+      D.scal[S_T] = t1;
+      *ctr(D, C_STEPS, 0) = c0 + 1;
+      *ctr(D, C_ACTIVE_UPD, 0) = c1 + n;
+      *ctr(D, C_COMPUTE_UPD, 0) = c2 + nc;
+      if (stop) D.scal[S_DONE] = 1.0;
+    }
+    if (stop) return;
   }
-  if (reset) reset_member(P, D);
+  if (reset) {
+    *ctr(D, C_COMPUTE_CELLS, lane) = 0;
+    if (lane == 0) {
+      *D.dt_bits = (unsigned long long)__double_as_longlong(P.max_dt);
+      *ctr(D, C_TILES, 0) = 0;
+      *ctr(D, C_ROWS, 0) = 0;
+      *ctr(D, C_CELLS, 0) = 0;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------

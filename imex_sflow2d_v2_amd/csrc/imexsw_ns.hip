@@ -168,18 +168,28 @@ void launch_convert(const DevParams& P, hipStream_t s, int n_cu, long long n, co
                        out, mode);
 }
 
-template <int NS, bool VP>
-void launch_stage_v(imexsw_ctx* c, int st, int policy) {
+template <int NS, bool VP, int RM, bool LAST>
+void launch_stage_k(imexsw_ctx* c, int st, int policy) {
   const int items = (c->n_tiles * kTileH + 3) / 4;
   static int res = 0;
-  if (!res) res = resident_grid(kg_stage<NS, VP>, 256, c->n_cu, 1 << 30);
-  hipLaunchKernelGGL((kg_stage<NS, VP>), dim3(std::min(items, res)), dim3(256), 0, c->stream,
-                     c->P, c->D, c->G, c->tab, st, policy);
+  if (!res) res = resident_grid(kg_stage<NS, VP, RM, LAST>, 256, c->n_cu, 1 << 30);
+  hipLaunchKernelGGL((kg_stage<NS, VP, RM, LAST>), dim3(std::min(items, res)), dim3(256), 0,
+                     c->stream, c->P, c->D, c->G, c->tab, st, policy);
+}
+template <int NS, bool VP, int RM>
+void launch_stage_m(imexsw_ctx* c, int st, int policy) {
+  if (c->tab.nrk == 2) launch_stage_k<NS, VP, RM, true>(c, st, policy);
+  else launch_stage_k<NS, VP, RM, false>(c, st, policy);
 }
 template <int NS>
 void launch_stage(imexsw_ctx* c, int st, int policy) {
-  if (c->P.vp) launch_stage_v<NS, true>(c, st, policy);
-  else launch_stage_v<NS, false>(c, st, policy);
+  const int rm = c->P.rheo ? c->P.rheo_model : 1;
+  // (the profiles come with model 8 or without rheology)
+  if (c->P.vp && rm == 8) launch_stage_m<NS, true, 8>(c, st, policy);
+  else if (c->P.vp) launch_stage_m<NS, true, 1>(c, st, policy);
+  else if (rm == 8) launch_stage_m<NS, false, 8>(c, st, policy);
+  else if (rm == 6) launch_stage_m<NS, false, 6>(c, st, policy);
+  else launch_stage_m<NS, false, 1>(c, st, policy);
 }
 template <int NS, bool VP>
 void launch_assemble_v(imexsw_ctx* c, int policy) {

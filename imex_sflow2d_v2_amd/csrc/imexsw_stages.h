@@ -150,10 +150,10 @@ __device__ __forceinline__ void integrate_friction(const DevParams& P, double* q
   phys<NS, VP>(P, qj, qp);
   const double r_h = qp[0];
   double r_u = qp[NV], r_v = qp[NV + 1];
-  const double mvh = sqrt(r_u * r_u + r_v * r_v);
-  const double mv = 1.0 / (1.0 / mvh + P.ff / r_h * dt);
-  r_u = r_u * (mv / mvh);
-  r_v = r_v * (mv / mvh);
+  const Rcp mvh = rcp_of(fsqrt(r_u * r_u + r_v * r_v));
+  const double mv = fdiv(1.0, div_by(1.0, mvh) + fdiv(P.ff, r_h) * dt);
+  r_u = r_u * div_by(mv, mvh);
+  r_v = r_v * div_by(mv, mvh);
   qp[1] = r_h * r_u;
   qp[2] = r_h * r_v;
   qp[NV] = r_u;
@@ -168,7 +168,8 @@ __device__ __forceinline__ void integrate_friction(const DevParams& P, double* q
 // summed over the stages before this one, in stage order from 0.0 (row i_RK
 // of the tableau without its diagonal); out: the stage state and NH + SI_NH
 // of the stage.  Returns the Newton iteration count (0: no Newton).
-template <int NS, bool VP = false>
+// RM: the rheology model compiled in, 1 (or no rheology), 6 or 8.
+template <int NS, bool VP, int RM>
 __device__ __forceinline__ int stage_cell(const DevParams& P, const double* q0,
                                           const double* s1p, const double* s2p,
                                           double a_diag, double dt, double Bx, double By,
@@ -194,9 +195,10 @@ __device__ __forceinline__ int stage_cell(const DevParams& P, const double* q0,
   // rheology model 1 alone has: it is formed only for them
   int iters = 0;
   if (a_diag != 0.0) {
+    const Rcp rda = rcp_of(dt * a_diag);
     if (q_fv[0] > 0.0) {
       double s1 = 0.0, s2 = 0.0;
-      if (P.rheo && P.rheo_model == 1) {
+      if (RM == 1 && P.rheo && P.rheo_model == 1) {
         phys<NS, VP>(P, q_fv, qp);
         semi_impl<NS>(P, Bx, By, Bxx, Bxy, Byy, gc, qp, s1, s2);
       }
@@ -213,26 +215,25 @@ __device__ __forceinline__ int stage_cell(const DevParams& P, const double* q0,
         q_si[1] = 0.0;
         q_si[2] = 0.0;
       } else {
-        const double m = sqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]);
-        const double den = sqrt(f2 * f2 + f3 * f3);
-        q_si[1] = m * f2 / den;
-        q_si[2] = m * f3 / den;
+        const double m = fsqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]);
+        const Rcp den = rcp_of(fsqrt(f2 * f2 + f3 * f3));
+        q_si[1] = div_by(m * f2, den);
+        q_si[2] = div_by(m * f3, den);
       }
 #pragma unroll
       for (int i = 0; i < NV; i++) {
-        si_nh[i] = (q_si[i] - q_fv[i]) / (dt * a_diag);
+        si_nh[i] = div_by(q_si[i] - q_fv[i], rda);
         q_guess[i] = q_si[i];
         Rj[i] = Rj[i] - a_diag * si_nh[i];
       }
       // rheology model 8: solve_rk_step integrates the friction in closed
       // form and returns (src/solver_2d.f90:1734-1739)
-      const bool fric8 = P.rheo && P.rheo_model == 8;
+      constexpr bool fric8 = RM == 8;
       if (fric8) {
         integrate_friction<NS, VP>(P, q_guess, dt);
       } else {
-        const NewtonOut no = (P.rheo && P.rheo_model == 6)
-                                 ? solve_rk_step<NS, 6>(P, q_guess, q0, Rj, a_diag, dt, Bx, By)
-                                 : solve_rk_step<NS>(P, q_guess, q0, Rj, a_diag, dt, Bx, By);
+        const NewtonOut no =
+            solve_rk_step<NS, RM == 6 ? 6 : 1>(P, q_guess, q0, Rj, a_diag, dt, Bx, By);
         iters = no.iters;
         nonconv = !no.conv;
         ls_evals = no.ls_evals;
@@ -250,10 +251,10 @@ __device__ __forceinline__ int stage_cell(const DevParams& P, const double* q0,
         q_guess[1] = 0.0;
         q_guess[2] = 0.0;
       } else {
-        const double m = sqrt(q_guess[1] * q_guess[1] + q_guess[2] * q_guess[2]);
-        const double den = sqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]);
-        q_guess[1] = m * q_si[1] / den;
-        q_guess[2] = m * q_si[2] / den;
+        const double m = fsqrt(q_guess[1] * q_guess[1] + q_guess[2] * q_guess[2]);
+        const Rcp den = rcp_of(fsqrt(q_si[1] * q_si[1] + q_si[2] * q_si[2]));
+        q_guess[1] = div_by(m * q_si[1], den);
+        q_guess[2] = div_by(m * q_si[2], den);
       }
     } else {
 #pragma unroll
@@ -264,7 +265,7 @@ __device__ __forceinline__ int stage_cell(const DevParams& P, const double* q0,
     }
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-      const double nh = (q_guess[i] - q_si[i]) / (dt * a_diag);
+      const double nh = div_by(q_guess[i] - q_si[i], rda);
       im_out[i] = nh + si_nh[i];
     }
   } else {
@@ -285,9 +286,45 @@ struct StageCounters {
   int imax;
 };
 
-template <int NS, bool VP = false>
-__global__ void __launch_bounds__(256) kg_stage(DevParams P, DevPtrs D, RkPtrs G, RkTableau T,
-                                                int st, int policy) {
+// The assembled state q of cell c: its checks, then the state, its flags and
+// (profiles) its physical variables stored for the erosion pass.
+template <int NS, bool VP>
+__device__ __forceinline__ void assemble_cell(const DevParams& P, const DevPtrs& D, size_t c,
+                                              double* q, unsigned long long* cnt) {
+  constexpr int NV = 4 + NS;
+  const size_t pl = plane(P);
+  double qp[NV + 2];
+  bool cur = true;
+  assembly_checks<NS, VP>(P, D, c, q, qp, cnt, true, &cur);
+  bool zero = true;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    D.q[i * pl + c] = q[i];
+    zero = zero && (q[i] == 0.0);
+  }
+  D.sflag[c] = state_flags(q[0], zero);
+  if (VP && D.qpp) {
+    // the physical variables of the assembled state, for the erosion pass
+    if (!cur) phys_or_dry<NS, VP>(P, q, qp);
+#pragma unroll
+    for (int i = 0; i < NV + 2; i++) D.qpp[i * pl + c] = qp[i];
+  }
+}
+
+// RM as in stage_cell, one kernel each: with the Newton solves of models 1 and
+// 6 and the closed form of model 8 in one kernel, every model ran at the
+// registers of the largest.  LAST (N_RK = 2): the stage is the second and last
+// of the stiffly accurate two-stage tableau, whose first is explicit (its state
+// is q^n, its implicit terms are zero): the stage's state is assembled in place
+// and nothing of it is stored.  Bound by each cell's serial FP64 chain, at 256
+// registers a lane (two waves a SIMD; 301 x 203 cells, N_RK = 3, Newton solves:
+// 64 us a stage, 68 without the bound, and with three waves it spills).  N_RK = 2,
+// 100 x 68 cells, model 6: a step's two stages, assembly, stage copies and mask
+// chain 60 us, as one launch and one mask 26; 500 x 386 with profiles and model
+// 8: 750 us for stages and assembly, 630 as one launch.
+template <int NS, bool VP, int RM, bool LAST>
+__global__ void __launch_bounds__(256, 2) kg_stage(DevParams P, DevPtrs D, RkPtrs G, RkTableau T,
+                                                   int st, int policy) {
   constexpr int NV = 4 + NS;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   __shared__ unsigned long long cnt[4][kLocalEvents];
@@ -314,6 +351,7 @@ __global__ void __launch_bounds__(256) kg_stage(DevParams P, DevPtrs D, RkPtrs G
   for (int it = blockIdx.x * 4 + w; live && it < nrows; it += gridDim.x * 4) {
     const int row = D.row_list[it];
     const int tile = row / kTileH;
+    if (LAST && lane == 0) mark_dirty(P, D, tile);
     const int j = (tile % tiles_x) * kStripW - 2 + lane;
     const int k = (tile / tiles_x) * kTileH + row % kTileH;
     if (!(lane >= 2 && lane < 2 + kStripW && j < P.nx && k < P.ny)) continue;
@@ -327,7 +365,12 @@ __global__ void __launch_bounds__(256) kg_stage(DevParams P, DevPtrs D, RkPtrs G
       s2[i] = 0.0;
     }
     // the earlier stages' terms with row st of the tableau, in stage order
-    for (int r = 0; r < st; r++) {
+    // (LAST: one stage of weight 1, without implicit terms)
+    if (LAST) {
+#pragma unroll
+      for (int i = 0; i < NV; i++) s1[i] = 0.0 + G.Dx[i * pl + c];
+    }
+    for (int r = 0; !LAST && r < st; r++) {
       const double at = T.a_tilde[st][r], ad = T.a_dirk[st][r];
 #pragma unroll
       for (int i = 0; i < NV; i++) {
@@ -338,10 +381,11 @@ __global__ void __launch_bounds__(256) kg_stage(DevParams P, DevPtrs D, RkPtrs G
     const double bxx = D.Bxx ? D.Bxx[c] : 0.0, bxy = D.Bxy ? D.Bxy[c] : 0.0,
                  byy = D.Byy ? D.Byy[c] : 0.0, gc = D.gcoef ? D.gcoef[c] : 1.0;
     int nonconv, ls;
-    const int its = stage_cell<NS, VP>(P, q0, s1, s2, a_diag, dt, D.Bx[c], D.By[c], bxx, bxy,
+    const int its = stage_cell<NS, VP, RM>(P, q0, s1, s2, a_diag, dt, D.Bx[c], D.By[c], bxx, bxy,
                                        byy, gc, qr, im, nonconv, ls);
+    if (LAST) assemble_cell<NS, VP>(P, D, c, qr, cnt[w]);
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
+    for (int i = 0; !LAST && i < NV; i++) {
       G.qrk[st * sp + i * pl + c] = qr[i];
       G.Im[st * sp + i * pl + c] = im[i];
       // a stage without a flux evaluation keeps zero terms (:1298-1335)
@@ -404,7 +448,7 @@ __global__ void __launch_bounds__(256) kg_assemble(DevParams P, DevPtrs D, RkPtr
     if (!(lane >= 2 && lane < 2 + kStripW && j < P.nx && k < P.ny)) continue;
     const size_t c = cidx(P, j, k);
     if (!(D.mask[c] & M_COMPUTE)) continue;
-    double q[NV], qp[NV + 2];
+    double q[NV];
 #pragma unroll
     for (int i = 0; i < NV; i++) {
       double s1 = 0.0, s2 = 0.0;
@@ -413,21 +457,7 @@ __global__ void __launch_bounds__(256) kg_assemble(DevParams P, DevPtrs D, RkPtr
       for (int r = 0; r < T.nrk; r++) s2 = s2 + G.Im[r * sp + i * pl + c] * T.omega[r];
       q[i] = T.stiff ? G.qrk[(T.nrk - 1) * sp + i * pl + c] : D.q[i * pl + c] - dt * (s1 - s2);
     }
-    bool cur = true;
-    assembly_checks<NS, VP>(P, D, c, q, qp, cnt[w], true, &cur);
-    bool zero = true;
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      D.q[i * pl + c] = q[i];
-      zero = zero && (q[i] == 0.0);
-    }
-    D.sflag[c] = state_flags(q[0], zero);
-    if (VP && D.qpp) {
-      // the physical variables of the assembled state, for the erosion pass
-      if (!cur) phys_or_dry<NS, VP>(P, q, qp);
-#pragma unroll
-      for (int i = 0; i < NV + 2; i++) D.qpp[i * pl + c] = qp[i];
-    }
+    assemble_cell<NS, VP>(P, D, c, q, cnt[w]);
   }
   __syncthreads();
   if (threadIdx.x == 0) {
