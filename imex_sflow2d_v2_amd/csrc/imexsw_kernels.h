@@ -754,16 +754,26 @@ struct Side {
 // A face side with the profile closures, kept out of line: the stencil
 // march has six call sites, and inlined at all of them the closures' sums
 // took the march to 512 registers and 3.5 KB of spills per lane.  The
-// side's h0 and settling speeds are shared by its momentum and its flux
+// side's sums are formed in one pass for its momentum and its flux
 // coefficients (the carrier density of both is mixt_var's).
+template <int NS>
+__device__ __forceinline__ void vp_side_state(const DevParams& P, const double* qp, double bx,
+                                              double by, VpState<NS>& S) {
+  constexpr int NV = 4 + NS;
+  const double u = qp[NV], v = qp[NV + 1];
+  const double w = P.slope ? u * bx + v * by : 0.0;
+  vp_state<NS, true>(P, u * u + v * v, w * w, S);
+}
 template <int NS, int DIR>
 __device__ __forceinline__ void make_side_vp_body(const DevParams& P, const double* qp,
                                                   double gc, double bx, double by,
                                                   Side<NS>* s) {
   if (qp[0] > kEps) {
-    const VpPre<NS> pre = vp_pre<NS>(P, qp[0], mixt<NS, false>(P, qp).rho_c);
-    qp2qc<NS, true>(P, qp, s->qc, &pre);
-    fluxes<NS, DIR, true>(P, s->qc, qp, gc, s->f, bx, by, &pre);
+    VpState<NS> S;
+    vp_pre<NS>(P, qp[0], mixt<NS, false>(P, qp).rho_c, S);
+    vp_side_state<NS>(P, qp, bx, by, S);
+    qp2qc<NS, true>(P, qp, s->qc, &S);
+    fluxes<NS, DIR, true>(P, s->qc, qp, gc, s->f, bx, by, &S);
   } else {
     qp2qc<NS, true>(P, qp, s->qc);
     fluxes<NS, DIR, true>(P, s->qc, qp, gc, s->f, bx, by);
@@ -1464,8 +1474,8 @@ __device__ __forceinline__ void stencil_strip(const DevParams& P, const DevPtrs&
 // and E values of the x reconstruction, its S and N values of the y
 // reconstruction, with the slope correction of that face and the cell's own
 // bed slope): k_vp_sides forms them for every cell of the listed tiles and
-// a one-cell ring around them, with the profile closures inlined and no
-// march around them, and the strip march (stencil_strip_vp) reads them.
+// those that a ring of one cell around them needs, with the profile closures
+// inlined and no march around them, and the strip march (stencil_strip_vp) reads them.
 // The ring overrides pick the other cell's side of the face, which is the
 // side formed from the same state (the slope the closures read differs only
 // with slope correction, a combination refused with a radial source).
@@ -1519,55 +1529,89 @@ __device__ __forceinline__ void qpp_get(const DevParams& P, const DevPtrs& D, in
   }
 }
 
-// the four sides of cell (j, k), with the operands the strip march gives
-// make_side (zero sides for a source-interior cell, whose own sides no face
-// uses)
-template <int NS>
+// the two sides of cell (j, k) in direction DIR, with the operands the strip
+// march gives make_side (zero sides for a source-interior cell, whose own
+// sides no face uses)
+template <int NS, int DIR>
 __device__ __forceinline__ void vp_cell_sides(const DevParams& P, const DevPtrs& D,
                                               const SrcTime& T, int j, int k) {
-  constexpr int NV = 4 + NS;
+  constexpr int NV = 4 + NS, DX = (DIR == 1), DY = (DIR == 2);
   const size_t c = cidx(P, j, k);
-  double qk[NV + 2], qkm[NV + 2], qkp[NV + 2], qm[NV + 2], qn[NV + 2];
+  double qk[NV + 2], qm[NV + 2], qn[NV + 2], r[2][NV + 2];
   qpp_get<NS>(P, D, j, k, qk);
-  qpp_get<NS>(P, D, j - 1, k, qkm);
-  qpp_get<NS>(P, D, j + 1, k, qkp);
-  qpp_get<NS>(P, D, j, k - 1, qm);
-  qpp_get<NS>(P, D, j, k + 1, qn);
+  qpp_get<NS>(P, D, j - DX, k - DY, qm);
+  qpp_get<NS>(P, D, j + DX, k + DY, qn);
   int bc;
   double v0, v1;
   load_src(P, D, j, k, bc, v0, v1);
   RowData R;
   load_rowdata(P, D, j, k, R);
-  const double gS = load_gsy(P, D, j, k), gN = load_gsy(P, D, j, k + 1);
+  const double g0 = DX ? R.gW : load_gsy(P, D, j, k);
+  const double g1 = DX ? R.gE : load_gsy(P, D, j, k + 1);
   const SrcInfo S = src_info(bc);
-  Side<NS> a, b;
+  Side<NS> a;
   if (S.is_src) {
     zero_side<NS>(a);
 #pragma unroll
-    for (int s = 0; s < 4; s++) side_put<NS>(P, D, c, s, a);
+    for (int s = 0; s < 2; s++) side_put<NS>(P, D, c, (DX ? SD_W : SD_S) + s, a);
     return;
   }
-  // both reconstructions first: the neighbours' states are then dead while
-  // the closures run
-  double lox[NV + 2], hix[NV + 2], loy[NV + 2], hiy[NV + 2];
+  // both values first: the neighbours' states are then dead while the closures
+  // run, which are one piece of code for the two
   const Ring ring{S, T, v0, v1};
-  const bool typo = P.radial && S.src2 && k > 0 && k < P.ny - 1 && !S.sS && S.sN;
-  recon<NS, 1>(P, qk, qkm, qkp, j, P.nx, k, ring, typo, lox, hix);
-  recon<NS, 2>(P, qk, qm, qn, k, P.ny, j, ring, false, loy, hiy);
-  make_side_vp_body<NS, 1>(P, lox, R.gW, R.bx, R.by, &a);
-  side_put<NS>(P, D, c, SD_W, a);
-  make_side_vp_body<NS, 1>(P, hix, R.gE, R.bx, R.by, &b);
-  side_put<NS>(P, D, c, SD_E, b);
-  make_side_vp_body<NS, 2>(P, loy, gS, R.bx, R.by, &a);
-  side_put<NS>(P, D, c, SD_S, a);
-  make_side_vp_body<NS, 2>(P, hiy, gN, R.bx, R.by, &b);
-  side_put<NS>(P, D, c, SD_N, b);
+  const bool typo = DX && P.radial && S.src2 && k > 0 && k < P.ny - 1 && !S.sS && S.sN;
+  recon<NS, DIR>(P, qk, qm, qn, DX ? j : k, DX ? P.nx : P.ny, DX ? k : j, ring, typo, r[0], r[1]);
+#pragma nounroll
+  for (int s = 0; s < 2; s++) {
+    double q[NV + 2];
+#pragma unroll
+    for (int i = 0; i < NV + 2; i++) q[i] = s ? r[1][i] : r[0][i];
+    make_side_vp_body<NS, DIR>(P, q, s ? g1 : g0, R.bx, R.by, &a);
+    side_put<NS>(P, D, c, (DX ? SD_W : SD_S) + s, a);
+  }
 }
 
-// one workgroup per listed tile in turn: the tile's cells and the ring of
-// cells around it
+// One wavefront per item: a listed tile's cells, 64 at a time, in one of the
+// two directions, then the cells beyond its edges in unlisted tiles (those in
+// listed ones are formed there).  Bound by the issue of the closures' FP64
+// exponentials and logarithms (62% of the cycles), so what counts is an even load
+// and sums shared by a side's momentum and fluxes: 500 x 386, two classes, 20
+// points: 756 us with a workgroup per tile (225 tiles), the ring formed twice and
+// two passes over the points, 444 like this, 418 without the exponential's range
+// selects.  Three waves a SIMD (168 registers, 244 bytes spilled) 418, two 440.
+constexpr int kSideCells = (kStripW * kTileH + 63) / 64;
+constexpr int kSideX = kSideCells + (2 * kTileH + 63) / 64;
+constexpr int kSideY = kSideCells + (2 * kStripW + 63) / 64;
+template <int NS, int DIR>
+__device__ __forceinline__ void vp_sides_item(const DevParams& P, const DevPtrs& D,
+                                              const SrcTime& T, int tile, int part) {
+  const int tiles_x = (P.nx + kStripW - 1) / kStripW;
+  const int tx = tile % tiles_x, ty = tile / tiles_x;
+  const int x0 = tx * kStripW, y0 = ty * kTileH;
+  const int tw = min(kStripW, P.nx - x0), th = min(kTileH, P.ny - y0);
+  int j, k;
+  if (part < kSideCells) {
+    const int e = part * 64 + (int)threadIdx.x;
+    if (e >= tw * th) return;
+    j = x0 + e % tw;
+    k = y0 + e / tw;
+  } else {
+    // DIR 1: the columns left and right of the tile; 2: the rows below and above
+    const int n = (DIR == 1) ? th : tw;
+    int e = (part - kSideCells) * 64 + (int)threadIdx.x;
+    if (e >= 2 * n) return;
+    const bool far = e >= n;
+    if (far) e -= n;
+    j = (DIR == 1) ? (far ? x0 + tw : x0 - 1) : x0 + e;
+    k = (DIR == 1) ? y0 + e : (far ? y0 + th : y0 - 1);
+    if (j < 0 || j >= P.nx || k < 0 || k >= P.ny) return;
+    const int step = (DIR == 1) ? 1 : tiles_x;
+    if (D.tile_flag[far ? tile + step : tile - step]) return;
+  }
+  vp_cell_sides<NS, DIR>(P, D, T, j, k);
+}
 template <int NS>
-__global__ void __launch_bounds__(256, 2) k_vp_sides(DevParams P, DevPtrs D) {
+__global__ void __launch_bounds__(64, 3) k_vp_sides(DevParams P, DevPtrs D) {
   double done = D.scal[S_DONE], t = D.scal[S_T];
   int ntiles = (int)*ctr(D, C_TILES, 0);
   pin(done);
@@ -1575,15 +1619,10 @@ __global__ void __launch_bounds__(256, 2) k_vp_sides(DevParams P, DevPtrs D) {
   pin(ntiles);
   if (done != 0.0) return;
   const SrcTime T = P.radial ? src_time(P, t) : SrcTime{};
-  const int tiles_x = (P.nx + kStripW - 1) / kStripW;
-  constexpr int W = kStripW + 2, H = kTileH + 2;
-  for (int item = blockIdx.x; item < ntiles; item += gridDim.x) {
-    const int tile = D.tile_list[item];
-    const int x0 = (tile % tiles_x) * kStripW - 1, y0 = (tile / tiles_x) * kTileH - 1;
-    for (int e = threadIdx.x; e < W * H; e += blockDim.x) {
-      const int j = x0 + e % W, k = y0 + e / W;
-      if (j >= 0 && j < P.nx && k >= 0 && k < P.ny) vp_cell_sides<NS>(P, D, T, j, k);
-    }
+  for (int item = blockIdx.x; item < ntiles * (kSideX + kSideY); item += gridDim.x) {
+    const int tile = D.tile_list[item / (kSideX + kSideY)], part = item % (kSideX + kSideY);
+    if (part < kSideX) vp_sides_item<NS, 1>(P, D, T, tile, part);
+    else vp_sides_item<NS, 2>(P, D, T, tile, part - kSideX);
   }
 }
 
@@ -2973,8 +3012,10 @@ __global__ void k_convert(DevParams P, long long n, const double* __restrict__ i
       for (int i = 0; i < NV; i++) r[i] = 1.0;
       if (VP && qp[0] > kEps) {
         const Mixt m = mixt<NS, false>(P, qp);
-        vp_flux_coeffs<NS>(P, qp, bx[e], by[e], vp_pre<NS>(P, qp[0], m.rho_c), m.rho_c, m.rho_m,
-                           r);
+        VpState<NS> S;
+        vp_pre<NS>(P, qp[0], m.rho_c, S);
+        vp_side_state<NS>(P, qp, bx[e], by[e], S);
+        vp_flux_coeffs<NS>(P, qp, bx[e], by[e], S, m.rho_c, m.rho_m, r);
       }
     }
 #pragma unroll

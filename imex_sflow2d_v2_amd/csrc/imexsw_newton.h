@@ -743,7 +743,8 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
   double dcf[NS > 0 ? NS : 1];
 #pragma unroll
   for (int i = 0; i < NS; i++) dcf[i] = 1.0;
-  if (VP && P.bottom_conc) vp_dep_coeffs<NS>(P, r_h, mv, m.rho_c, dcf);
+  double svp[NS > 0 ? NS : 1];
+  if (VP && P.bottom_conc) vp_dep_coeffs<NS>(P, r_h, mv, m.rho_c, dcf, svp);
   if (P.settling) {
     // hindered settling factor, the same for every class
     const double hind = det_pow(1.0 - fmin(1.0, fdiv(at, alpha_max)), hind_exp);
@@ -782,8 +783,10 @@ __device__ __forceinline__ void mass_exchange(const DevParams& P, const double* 
     for (int i = 0; i < NS; i++) {
       if (al[i] > 0.0) {
         const double sv = (LANES > 1) ? svs[i]
-                                      : settling_velocity(P, P.diam_s[i], P.rho_s[i], m.rho_c,
-                                                          inv_kin_visc);
+                          : (VP && P.bottom_conc)
+                              ? svp[i]
+                              : settling_velocity(P, P.diam_s[i], P.rho_s[i], m.rho_c,
+                                                  inv_kin_visc);
         double d = al[i] * sv * dcf[i];
         d = d * hind;
         dep[i] = fmin(d, div_by(r_h * al[i], rdt));

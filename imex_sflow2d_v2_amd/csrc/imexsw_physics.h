@@ -345,10 +345,10 @@ __device__ __forceinline__ Mixt mixt(const DevParams& P, const double* qp) {
 }
 
 // qp_to_qc (src/constitutive_2d.f90:1709-2140, no liquid; VP: the profile
-// momentum, with the state's h0 and settling speeds from pre when given)
+// momentum, with the state's sums from vs when given)
 template <int NS, bool VP = false>
 __device__ __forceinline__ void qp2qc(const DevParams& P, const double* qp,
-                                      double* qc, const VpPre<NS>* pre = nullptr) {
+                                      double* qc, const VpState<NS>* vs = nullptr) {
   constexpr int NV = 4 + NS;
   double r_h = qp[0];
   if (!(r_h > kEps)) {
@@ -388,8 +388,14 @@ __device__ __forceinline__ void qp2qc(const DevParams& P, const double* qp,
     double ra[NS > 0 ? NS : 1];
 #pragma unroll
     for (int i = 0; i < NS; i++) ra[i] = (at > 1.0) ? al[i] / at : (at < 0.0) ? 0.0 : al[i];
-    const VpPre<NS> pr = pre ? *pre : vp_pre<NS>(P, r_h, rho_c);
-    vp_momentum<NS>(P, r_h, r_u, r_v, pr, rho_c, ra, qc[1], qc[2]);
+    if (vs) {
+      vp_momentum<NS>(P, r_h, r_u, r_v, *vs, rho_c, ra, qc[1], qc[2]);
+    } else {
+      VpState<NS> S;
+      vp_pre<NS>(P, r_h, rho_c, S);
+      vp_state<NS, false>(P, r_u * r_u + r_v * r_v, 0.0, S);
+      vp_momentum<NS>(P, r_h, r_u, r_v, S, rho_c, ra, qc[1], qc[2]);
+    }
   } else {
     qc[1] = rho_m * r_hu;
     qc[2] = rho_m * r_hv;
@@ -429,7 +435,7 @@ template <int NS, int DIR, bool VP = false>
 __device__ __forceinline__ void fluxes(const DevParams& P, const double* qc,
                                        const double* qp, double gc, double* f,
                                        double Bx = 0.0, double By = 0.0,
-                                       const VpPre<NS>* pre = nullptr) {
+                                       const VpState<NS>* vs = nullptr) {
   constexpr int NV = 4 + NS;
   if (!(qp[0] > kEps)) {
 #pragma unroll
@@ -442,8 +448,7 @@ __device__ __forceinline__ void fluxes(const DevParams& P, const double* qc,
 #pragma unroll
   for (int i = 0; i < NV; i++) sc[i] = 1.0;
   if (VP) {
-    const VpPre<NS> pr = pre ? *pre : vp_pre<NS>(P, r_h, m.rho_c);
-    vp_flux_coeffs<NS>(P, qp, Bx, By, pr, m.rho_c, m.rho_m, sc);
+    vp_flux_coeffs<NS>(P, qp, Bx, By, *vs, m.rho_c, m.rho_m, sc);
   }
   double vel = (DIR == 1) ? r_u : r_v;
   double pt = 0.5 * m.rho_m * gc * m.rg * (r_h * r_h);
