@@ -109,7 +109,14 @@ __global__ void __launch_bounds__(256) kb_local(const DevParams* __restrict__ Ps
     for (int i = lane; i < kLocalEvents; i += 64) cnt[w][i] = 0;
     __builtin_amdgcn_wave_barrier();
     int imax = 0;
-    local_row<NS, PH>(P, D, e & kIdMask, D.scal[S_DT], ops, cnt[w], imax);
+    const int tiles_x = (P.nx + kStripW - 1) / kStripW;
+    const int row = e & kIdMask, tile = row / kTileH;
+    const int j = (tile % tiles_x) * kStripW - 2 + lane;
+    const int k = (tile / tiles_x) * kTileH + row % kTileH;
+    double sums[4] = {0.0, 0.0, 0.0, 0.0};  // not formed: ops holds no OP_SUMS
+    if (lane >= 2 && lane < 2 + kStripW && j < P.nx && k < P.ny)
+      local_cell<NS, PH>(P, D, cidx(P, j, k), D.scal[S_DT], ops & ~(int)OP_SUMS, cnt[w], imax,
+                         sums[0], sums[1], sums[2], sums[3]);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
     if (lane < kLocalEvents && cnt[w][lane])

@@ -488,8 +488,9 @@ __global__ void __launch_bounds__(64 * kMaskGroup) k_mask(DevParams P, DevPtrs D
   if (tyy < tiles_y)
     rows_m = mask_tile(P, D, blockIdx.x, tyy, tiles_x, solve_all, clean, all, &comp);
   const int j = blockIdx.x * kStripW - 2 + (int)(threadIdx.x & 63);
-  // (the tableau-driven path has no use for the cell list)
-  append_group<kMaskGroup>(own_sink(D), tyy * tiles_x + blockIdx.x, rows_m, all ? 0u : comp,
+  // (of the tableau-driven path only the profiles' kernels read the cell list)
+  append_group<kMaskGroup>(own_sink(D), tyy * tiles_x + blockIdx.x, rows_m,
+                           (all && !P.vp) ? 0u : comp,
                            (int)cidx(P, max(j, 0), tyy * kTileH), (int)P.pitch,
                            (long long)P.nx * P.ny);
 }
@@ -2497,28 +2498,62 @@ __device__ __forceinline__ void mark_dirty(const DevParams& P, const DevPtrs& D,
     }
 }
 
-// One tile row (60 cells, one per lane 2..61) of k_local; per-row partial
-// sums go to tile_sums[4 * row ..] when OP_SUMS.
-template <int NS, int PH, bool VP = false>
-__device__ __forceinline__ void local_row(const DevParams& P, const DevPtrs& D, int row,
-                                          double dt, int ops, unsigned long long* e,
-                                          int& imax) {
+// The plane index of the lane's cell in work item `item` of the step, -1 for
+// none, and the cell's tile and its neighbours marked for the next mask when
+// `mark`.  CELLS: 64 entries of the list of cells to compute, which holds a
+// tile's cells row by row (n: its length; every lane of the wavefront calls);
+// else the item'th listed tile row, 60 cells on lanes 2..61.
+// The profiles' kernels take cells: their lanes all take the same time, so full
+// wavefronts are what counts (500 x 386: stage 456 -> 382 us, erosion 284 ->
+// 220; its last column of tiles is 20 cells wide).  The others take rows: where
+// Newton counts differ from cell to cell a fuller wavefront waits for more of
+// them (512 x 512 incline 118 us by rows, 153 by cells; 301 x 203 68 / 70),
+// and the erosion part is no better for it (1000 x 1000: 188 / 200).
+template <bool CELLS>
+__device__ __forceinline__ int item_cell(const DevParams& P, const DevPtrs& D, int item, int n,
+                                         bool mark) {
   const int lane = threadIdx.x & 63;
   const int tiles_x = (P.nx + kStripW - 1) / kStripW;
-  const int tile = row / kTileH;
+  if (CELLS) {
+    const int idx = item * kWave + lane;
+    const int c = idx < n ? D.cell_list[idx] : -1;
+    const int k = c / (int)P.pitch, j = c - k * (int)P.pitch;
+    const int tile = (c < 0) ? -1 : (k / kTileH) * tiles_x + j / kStripW;
+    const int before = __shfl_up(tile, 1, 64);
+    if (mark && tile >= 0 && (lane == 0 || before != tile)) mark_dirty(P, D, tile);
+    return c;
+  }
+  const int row = D.row_list[item], tile = row / kTileH;
+  if (mark && lane == 0) mark_dirty(P, D, tile);
   const int j = (tile % tiles_x) * kStripW - 2 + lane;
   const int k = (tile / tiles_x) * kTileH + row % kTileH;
   const bool own = lane >= 2 && lane < 2 + kStripW && j < P.nx && k < P.ny;
+  return own ? (int)cidx(P, j, k) : -1;
+}
+// number of items of the step
+template <bool CELLS>
+__device__ __forceinline__ int item_count(const DevParams& P, int n) {
+  return CELLS ? (min(n, P.nx * P.ny) + kWave - 1) / kWave : n;
+}
+
+// One item of k_local; with OP_SUMS a tile row, whose partial sums go to
+// tile_sums[4 * row ..].
+template <int NS, int PH, bool CELLS, bool VP>
+__device__ __forceinline__ void local_item(const DevParams& P, const DevPtrs& D, int item,
+                                           int n, double dt, int ops, unsigned long long* e,
+                                           int& imax) {
+  const int c = item_cell<CELLS>(P, D, item, n, true);
   double s_mass = 0.0, s_vol = 0.0, s_area = 0.0, s_sol = 0.0;
-  if (own)
-    local_cell<NS, PH, VP>(P, D, cidx(P, j, k), dt, ops, e, imax, s_mass, s_vol, s_area, s_sol);
-  if (PH == 1 && (ops & OP_SUMS)) {
+  if (c >= 0)
+    local_cell<NS, PH, VP>(P, D, (size_t)c, dt, ops, e, imax, s_mass, s_vol, s_area, s_sol);
+  if (PH == 1 && !CELLS && (ops & OP_SUMS)) {
+    const int row = D.row_list[item];
     double v4[4] = {s_mass, s_vol, s_area, s_sol};
 #pragma unroll
     for (int m = 0; m < 4; m++) {
       double v = v4[m];
-      for (int off = 32; off > 0; off >>= 1) v += shfl_d(v, lane ^ off);
-      if (lane == 0) D.tile_sums[4 * (size_t)row + m] = v;
+      for (int off = 32; off > 0; off >>= 1) v += shfl_d(v, (threadIdx.x & 63) ^ off);
+      if ((threadIdx.x & 63) == 0) D.tile_sums[4 * (size_t)row + m] = v;
     }
   }
 }
@@ -2633,13 +2668,14 @@ __global__ void __launch_bounds__(64) k_mlp_guess(DevParams P, DevPtrs D, MlpDev
   }
 }
 
-// One wavefront per listed tile row (per row part for PH 3); the four
-// wavefronts of a workgroup take rows in turn until the list is exhausted.
+// One wavefront per item (item_cell; kCellsPerWave listed cells for PH 3 and
+// 4); the four wavefronts of a workgroup take items in turn until the list is
+// exhausted.  CELLS: with the profiles, but for the sums.
 // The plain stage update and the erosion part are held to two workgroups
 // per CU (the register budget of two waves per SIMD): on a wet grid the
 // second wave hides the first's latency (13% faster stage update measured
 // at 2048^2, no change on sparse steps).
-template <int NS, int PH, bool VP = false>
+template <int NS, int PH, bool VP = false, bool CELLS = false>
 __global__ void __launch_bounds__(256, (!VP && (PH == 0 || PH == 1)) ? 2 : 1)
     k_local(DevParams P, DevPtrs D, int ops) {
   warm_kernargs<kArgBytes>();
@@ -2658,7 +2694,8 @@ __global__ void __launch_bounds__(256, (!VP && (PH == 0 || PH == 1)) ? 2 : 1)
     c_first = D.cell_list[idx];
   }
   // the list size, issued ahead of the step's scalars (one round of loads)
-  unsigned long long nl_raw = (PH >= 3) ? *ctr(D, C_CELLS, 0) : *ctr(D, C_ROWS, 0);
+  constexpr bool cells = CELLS || PH >= 3;
+  unsigned long long nl_raw = cells ? *ctr(D, C_CELLS, 0) : *ctr(D, C_ROWS, 0);
   bool live;
   double dt;
   if (ops & OP_POLICY) {
@@ -2670,17 +2707,15 @@ __global__ void __launch_bounds__(256, (!VP && (PH == 0 || PH == 1)) ? 2 : 1)
     dt = D.scal[S_DT];
   }
   pin(nl_raw);
-  // PH 3, 4: items of kCellsPerWave listed cells; else listed tile rows
-  const int nlist = (PH >= 3) ? (int)min(nl_raw, (unsigned long long)P.nx * P.ny) : (int)nl_raw;
-  const int items = (PH >= 3) ? (nlist + kCellsPerWave - 1) / kCellsPerWave : nlist;
+  const int nlist = cells ? (int)min(nl_raw, (unsigned long long)P.nx * P.ny) : (int)nl_raw;
+  const int items = (PH >= 3) ? (nlist + kCellsPerWave - 1) / kCellsPerWave
+                              : item_count<CELLS>(P, nlist);
   for (int it = blockIdx.x * 4 + w; live && it < items; it += gridDim.x * 4) {
-    if (PH >= 3) {
+    if (PH >= 3)
       local_cells<NS, (PH >= 3 ? PH : 3)>(P, D, it, nlist, dt, ops, cnt[w], imax,
                                            (it == (int)blockIdx.x * 4 + w) ? c_first : -1);
-    } else {
-      if (lane == 0) mark_dirty(P, D, D.row_list[it] / kTileH);
-      local_row<NS, PH, VP>(P, D, D.row_list[it], dt, ops, cnt[w], imax);
-    }
+    else
+      local_item<NS, PH, CELLS, VP>(P, D, it, nlist, dt, ops, cnt[w], imax);
   }
   for (int off = 32; off > 0; off >>= 1) imax = max(imax, __shfl_xor(imax, off, 64));
   if (lane == 0) itmax[w] = imax;

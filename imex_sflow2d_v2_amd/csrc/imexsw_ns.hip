@@ -29,6 +29,14 @@ static int column_height(const imexsw_ctx* c, int slots) {
   return best;
 }
 
+// Workgroups of four wavefronts for every item of item_cell: cells 64 to a
+// wavefront, or tile rows
+[[maybe_unused]] static int item_groups(const imexsw_ctx* c, bool cells) {
+  const long long n = cells ? ((long long)c->P.nx * c->P.ny + kWave - 1) / kWave
+                            : (long long)c->n_tiles * kTileH;
+  return (int)std::min<long long>((n + 3) / 4, 1 << 30);
+}
+
 template <int NS>
 void launch_stencil(imexsw_ctx* c, const DevPtrs& D, int compute_dt, bool rows) {
   // work items: (listed tile, strip) pairs, at most tiles * kTileH / row_unit
@@ -84,8 +92,7 @@ void launch_stencil_vp(imexsw_ctx* c, const DevPtrs& D, int compute_dt, int item
 #endif
 template <int NS>
 void launch_local(imexsw_ctx* c, int ops, bool fused) {
-  // work items: listed tile rows, four per workgroup
-  const int items = (c->n_tiles * kTileH + 3) / 4;
+  const int items = item_groups(c, false);
   // a Newton starting point for the stage update: the learned one (its
   // guesses computed first, into the guess planes) or the closed form
   int start = 0;
@@ -129,10 +136,16 @@ void launch_local(imexsw_ctx* c, int ops, bool fused) {
                          c->P, c->D, rk);
   }
   if ((ops & (OP_EROSION | OP_POST | OP_SUMS)) && c->P.vp) {
-    static int res1v = 0;
+    static int res1v = 0, res1c = 0;
     if (!res1v) res1v = resident_grid(k_local<NS, 1, true>, 256, c->n_cu, 1 << 30);
-    hipLaunchKernelGGL((k_local<NS, 1, true>), dim3(std::min(items, res1v)), dim3(256), 0,
-                       c->stream, c->P, c->D, ops & ~(int)OP_RK);
+    if (!res1c) res1c = resident_grid(k_local<NS, 1, true, true>, 256, c->n_cu, 1 << 30);
+    if (ops & OP_SUMS)
+      hipLaunchKernelGGL((k_local<NS, 1, true>), dim3(std::min(items, res1v)), dim3(256), 0,
+                         c->stream, c->P, c->D, ops & ~(int)OP_RK);
+    else
+      hipLaunchKernelGGL((k_local<NS, 1, true, true>),
+                         dim3(std::min(item_groups(c, true), res1c)), dim3(256), 0, c->stream,
+                         c->P, c->D, ops & ~(int)OP_RK);
   } else if (ops & (OP_EROSION | OP_POST | OP_SUMS)) {
     hipLaunchKernelGGL((k_local<NS, 1>), dim3(std::min(items, res1)), dim3(256), 0, c->stream,
                        c->P, c->D, ops & ~(int)OP_RK);
@@ -170,7 +183,7 @@ void launch_convert(const DevParams& P, hipStream_t s, int n_cu, long long n, co
 
 template <int NS, bool VP, int RM, bool LAST>
 void launch_stage_k(imexsw_ctx* c, int st, int policy) {
-  const int items = (c->n_tiles * kTileH + 3) / 4;
+  const int items = item_groups(c, VP);
   static int res = 0;
   if (!res) res = resident_grid(kg_stage<NS, VP, RM, LAST>, 256, c->n_cu, 1 << 30);
   hipLaunchKernelGGL((kg_stage<NS, VP, RM, LAST>), dim3(std::min(items, res)), dim3(256), 0,
@@ -193,7 +206,7 @@ void launch_stage(imexsw_ctx* c, int st, int policy) {
 }
 template <int NS, bool VP>
 void launch_assemble_v(imexsw_ctx* c, int policy) {
-  const int items = (c->n_tiles * kTileH + 3) / 4;
+  const int items = item_groups(c, VP);
   static int res = 0;
   if (!res) res = resident_grid(kg_assemble<NS, VP>, 256, c->n_cu, 1 << 30);
   hipLaunchKernelGGL((kg_assemble<NS, VP>), dim3(std::min(items, res)), dim3(256), 0, c->stream,

@@ -117,7 +117,8 @@ __device__ __forceinline__ double vp_h0(const DevParams& P, double r_h) {
 // workgroup (at most kVpLanes), the rest are formed again.  40 KB a workgroup:
 // four fit a CU, one more than the registers allow.  500 x 386, model 8, two
 // conversions a cell: stage kernel 630 us with every logarithm formed each time,
-// 487 from LDS, 458 with the points unrolled and without range selects.
+// 487 from LDS, 458 with the points unrolled and without range selects, 380 with
+// full wavefronts (item_cell).
 constexpr int kVpCache = 20, kVpLanes = 256;
 
 // point m of the rule on [0, h0]: z, weight and log(b z + 1)

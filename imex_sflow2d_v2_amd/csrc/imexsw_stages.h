@@ -82,7 +82,7 @@ __global__ void kg_mask_dilate(DevParams P, const double* scal, const uint8_t* a
 
 // The source interior leaves the mask; mask bytes (every active cell is
 // computed), active and computed counts, and the tiles and tile rows with
-// an active cell appended to the work lists.  One wavefront per work tile,
+// an active cell, and the cells, appended to the work lists.  One wavefront per work tile,
 // kMaskGroup tiles per workgroup, the lane layout of k_mask.
 template <int = 0>
 __global__ void __launch_bounds__(64 * kMaskGroup) kg_mask_final(DevParams P, DevPtrs D,
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(64 * kMaskGroup) kg_mask_final(DevParams P, De
   const int tile = tyy * tiles_x + blockIdx.x;
   const int j = blockIdx.x * kStripW - 2 + lane;
   const bool own = tyy < tiles_y && lane >= 2 && lane < 2 + kStripW && j < P.nx;
-  unsigned rows_m = 0;
+  unsigned rows_m = 0, comp = 0;
   int count = 0;
   if (own) {
     for (int rr = 0; rr < kTileH; rr++) {
@@ -111,6 +111,7 @@ __global__ void __launch_bounds__(64 * kMaskGroup) kg_mask_final(DevParams P, De
       }
     }
   }
+  comp = rows_m;
   for (int off = 32; off > 0; off >>= 1) {
     count += __shfl_xor(count, off, 64);
     rows_m |= (unsigned)__shfl_xor((int)rows_m, off, 64);
@@ -123,7 +124,9 @@ __global__ void __launch_bounds__(64 * kMaskGroup) kg_mask_final(DevParams P, De
     if (count) atomicAdd(ctr(D, C_COMPUTE_CELLS, tile), (unsigned long long)count);
     D.tile_flag[tile] = rows_m ? 1 : 0;
   }
-  append_group<kMaskGroup>(own_sink(D), tile, tyy < tiles_y ? rows_m : 0u);
+  append_group<kMaskGroup>(own_sink(D), tile, tyy < tiles_y ? rows_m : 0u, P.vp ? comp : 0u,
+                           (int)cidx(P, max(j, 0), tyy * kTileH), (int)P.pitch,
+                           (long long)P.nx * P.ny);
 }
 
 // q into every stage state (an inactive cell's stage states are its state,
@@ -323,7 +326,7 @@ __device__ __forceinline__ void assemble_cell(const DevParams& P, const DevPtrs&
 // chain 60 us, as one launch and one mask 26; 500 x 386 with profiles and model
 // 8: 750 us for stages and assembly, 630 as one launch.
 template <int NS, bool VP, int RM, bool LAST>
-__global__ void __launch_bounds__(256, 2) kg_stage(DevParams P, DevPtrs D, RkPtrs G, RkTableau T,
+__global__ void __launch_bounds__(256, (VP && RM == 8) ? 3 : 2) kg_stage(DevParams P, DevPtrs D, RkPtrs G, RkTableau T,
                                                    int st, int policy) {
   constexpr int NV = 4 + NS;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -343,20 +346,14 @@ __global__ void __launch_bounds__(256, 2) kg_stage(DevParams P, DevPtrs D, RkPtr
   }
   const size_t pl = plane(P);
   const size_t sp = (size_t)NV * pl;  // planes of one stage
-  const int tiles_x = (P.nx + kStripW - 1) / kStripW;
-  const int nrows = (int)*ctr(D, C_ROWS, 0);
+  const int n = (int)*ctr(D, VP ? C_CELLS : C_ROWS, 0);
   const double a_diag = T.a_dirk[st][st];
   const bool flux = T.omega_tilde[st] > 0.0;
   int imax = 0;
-  for (int it = blockIdx.x * 4 + w; live && it < nrows; it += gridDim.x * 4) {
-    const int row = D.row_list[it];
-    const int tile = row / kTileH;
-    if (LAST && lane == 0) mark_dirty(P, D, tile);
-    const int j = (tile % tiles_x) * kStripW - 2 + lane;
-    const int k = (tile / tiles_x) * kTileH + row % kTileH;
-    if (!(lane >= 2 && lane < 2 + kStripW && j < P.nx && k < P.ny)) continue;
-    const size_t c = cidx(P, j, k);
-    if (!(D.mask[c] & M_COMPUTE)) continue;
+  for (int it = blockIdx.x * 4 + w; live && it < item_count<VP>(P, n); it += gridDim.x * 4) {
+    const int cell = item_cell<VP>(P, D, it, n, LAST);
+    if (cell < 0 || !(D.mask[cell] & M_COMPUTE)) continue;
+    const size_t c = (size_t)cell;
     double q0[NV], s1[NV], s2[NV], qr[NV], im[NV];
 #pragma unroll
     for (int i = 0; i < NV; i++) {
@@ -437,17 +434,11 @@ __global__ void __launch_bounds__(256) kg_assemble(DevParams P, DevPtrs D, RkPtr
   }
   const size_t pl = plane(P);
   const size_t sp = (size_t)NV * pl;
-  const int tiles_x = (P.nx + kStripW - 1) / kStripW;
-  const int nrows = (int)*ctr(D, C_ROWS, 0);
-  for (int it = blockIdx.x * 4 + w; live && it < nrows; it += gridDim.x * 4) {
-    const int row = D.row_list[it];
-    const int tile = row / kTileH;
-    if (lane == 0) mark_dirty(P, D, tile);
-    const int j = (tile % tiles_x) * kStripW - 2 + lane;
-    const int k = (tile / tiles_x) * kTileH + row % kTileH;
-    if (!(lane >= 2 && lane < 2 + kStripW && j < P.nx && k < P.ny)) continue;
-    const size_t c = cidx(P, j, k);
-    if (!(D.mask[c] & M_COMPUTE)) continue;
+  const int n = (int)*ctr(D, VP ? C_CELLS : C_ROWS, 0);
+  for (int it = blockIdx.x * 4 + w; live && it < item_count<VP>(P, n); it += gridDim.x * 4) {
+    const int cell = item_cell<VP>(P, D, it, n, true);
+    if (cell < 0 || !(D.mask[cell] & M_COMPUTE)) continue;
+    const size_t c = (size_t)cell;
     double q[NV];
 #pragma unroll
     for (int i = 0; i < NV; i++) {
