@@ -93,8 +93,10 @@ __global__ void kb_dtpolicy(const DevParams* __restrict__ Ps, const DevPtrs* __r
 
 // rows of all members; each wavefront flushes its event counters into the
 // member of the row it just finished
+// (two waves a SIMD: 24 members, 128 to 512 wide: stage update 237 us at one,
+// with 262 registers, 206 at two with 256)
 template <int NS, int PH>
-__global__ void __launch_bounds__(256) kb_local(const DevParams* __restrict__ Ps,
+__global__ void __launch_bounds__(256, 2) kb_local(const DevParams* __restrict__ Ps,
                                                 const DevPtrs* __restrict__ Ds, BatchLists L,
                                                 int ops) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
