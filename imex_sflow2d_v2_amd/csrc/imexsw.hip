@@ -274,32 +274,28 @@ int init_stages(imexsw_ctx* c) {
 }
 
 // one time step of the main loop (src/IMEX_SfloW2D.f90:337-531), all on the
-// context's stream.  The stage kernel applies the time-step policy itself;
-// k_step_begin of the next step (commit_prev) or end_steps commits it and
-// advances t.
-int enqueue_step(imexsw_ctx* c, bool commit_prev) {
-  {
+// context's stream, of a sequence whose first and last steps are marked.  The
+// last pass over the cells ends the step (time step policy, t, counters), for
+// which the stage kernel applies the policy itself.
+int enqueue_step(imexsw_ctx* c, bool first, bool last) {
+  if (first) {
     Timed tm(c, K_DTPOLICY);
-    hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D,
-                       commit_prev ? 1 : 0, 1);
+    hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D);
   }
+  const int end = OP_POLICY | OP_END | (last ? 0 : OP_NEXT);
   if (c->general) {
     if (run_mask(c, 0, 1) || init_stages(c)) return -1;
     if (run_stencil(c, c->P.cfl != -1.0)) return -1;
     if (run_stages(c, 1)) return -1;
-    if (run_local(c, OP_EROSION | OP_POST | OP_POLICY, K_LOCAL)) return -1;
+    if (run_local(c, OP_EROSION | OP_POST | end, K_LOCAL)) return -1;
     if (c->P.topo && run_topo(c, 1)) return -1;
-    return check_launch(c, "k_step_begin");
+    return check_launch(c, "step");
   }
   if (run_mask(c, 0, 1)) return -1;
   if (run_stencil(c, c->P.cfl != -1.0, c->sparse)) return -1;
-  if (run_local(c, OP_RK | OP_EROSION | OP_POST | OP_POLICY, K_LOCAL, c->sparse)) return -1;
+  if (run_local(c, OP_RK | OP_EROSION | OP_POST | end, K_LOCAL, c->sparse)) return -1;
   if (c->P.topo && run_topo(c, c->sparse ? 2 : 1)) return -1;
-  return check_launch(c, "k_step_begin");
-}
-int end_steps(imexsw_ctx* c) {
-  hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D, 1, 0);
-  return check_launch(c, "k_step_begin");
+  return check_launch(c, "step");
 }
 
 void drop_ctx_graph(imexsw_ctx* c) {
@@ -334,8 +330,8 @@ int capture_steps(imexsw_ctx* c, int m) {
   const bool sparse = c->sparse;
   c->sparse = (m == 1);
   int rc = 0;
-  for (int i = 0; i < kGraphSteps && !rc; i++) rc = enqueue_step(c, i > 0);
-  if (!rc) rc = end_steps(c);
+  for (int i = 0; i < kGraphSteps && !rc; i++)
+    rc = enqueue_step(c, i == 0, i == kGraphSteps - 1);
   c->sparse = sparse;
   hipGraph_t g = nullptr;
   hipError_t err = hipStreamEndCapture(c->stream, &g);
@@ -1262,7 +1258,7 @@ int imexsw_advance(imexsw_ctx* c, int32_t nsteps, double dt0, double* t_io, doub
       HIPCHK(c, hipStreamSynchronize(c->stream));
       if (done != 0.0) break;
     }
-    if (enqueue_step(c, false) || end_steps(c)) return -1;
+    if (enqueue_step(c, true, true)) return -1;
     if (c->sparse) c->sparse_steps++;
   }
   c->d_valid = false;

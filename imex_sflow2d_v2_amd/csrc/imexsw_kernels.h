@@ -92,7 +92,11 @@ enum CounterSlot { C_SOLVE_CELLS = 0, C_NEWTON_CELLS, C_NEWTON_ITERS, C_NONCONV,
                    C_HIST0, C_HIST1, C_HIST2, C_HIST3, C_HIST4, C_HIST5, C_HIST6,
                    C_HIST7, C_WARM_USED, C_WARM_FALLBACK, C_ITMAX, C_STEPS,
                    C_ACTIVE_UPD, C_COMPUTE_CELLS, C_TILES, C_ROWS, C_HARVEST,
-                   C_COMPUTE_UPD, C_CELLS, C_NCOUNTERS };
+                   C_COMPUTE_UPD, C_CELLS, C_ARRIVE, C_ARRIVED = C_ARRIVE + 16,
+                   C_NCOUNTERS };
+// workgroups of a step's last kernel arrive at kArrive counters, the last at
+// each of them at C_ARRIVED (step_arrive); zero between kernels
+constexpr int kArrive = C_ARRIVED - C_ARRIVE;
 // k_local's per-cell event counters, in CounterSlot order from C_NEWTON_CELLS
 constexpr int kLocalEvents = C_ITMAX - C_NEWTON_CELLS;  // summed ones
 // Newton iteration histogram buckets: 1, 2, 3, 4, 5-8, 9-16, 17-32, 33-100
@@ -2029,7 +2033,7 @@ __global__ void __launch_bounds__(384) k_stencil_rows(DevParams P, DevPtrs D, in
 // the host loop's time-step policy, src/IMEX_SfloW2D.f90:357-381, on the
 // device: step_dt evaluates it from the step's scalars and the CFL minimum
 // without writing anything (every workgroup of the stage kernel does), and
-// dtpolicy_member commits the result
+// step_commit (dtpolicy_member for a member of an ensemble) commits the result
 // ---------------------------------------------------------------------------
 struct StepDt {
   bool done;       // the run was over, or t >= t_end: no update this step
@@ -2108,64 +2112,90 @@ __device__ __forceinline__ void reset_member(const DevParams& P, const DevPtrs& 
   *ctr(D, C_CELLS, 0) = 0;
 }
 
-// Between two steps of imexsw_advance: commit the previous step (its time
-// step policy, t = t + dt, counters) when `commit`, then reset the per-step
-// counters for the next one.  With commit and without reset: the end of the
-// last step.  One wavefront, a counter slot per lane: the same as
-// dtpolicy_member, advance_member and reset_member with every load in one
-// round (one thread walking the slots took 4.5 us).
+// per-step counters for the step to come: one wavefront, a slot per lane
+__device__ __forceinline__ void step_reset(const DevParams& P, const DevPtrs& D, int lane) {
+  *ctr(D, C_COMPUTE_CELLS, lane) = 0;
+  if (lane == 0) {
+    *D.dt_bits = (unsigned long long)__double_as_longlong(P.max_dt);
+    *ctr(D, C_TILES, 0) = 0;
+    *ctr(D, C_ROWS, 0) = 0;
+    *ctr(D, C_CELLS, 0) = 0;
+  }
+}
+
+// before the first step of a sequence
 template <int = 0>
-__global__ void __launch_bounds__(64) k_step_begin(DevParams P, DevPtrs D, int commit,
-                                                   int reset) {
-  const int lane = threadIdx.x;
-  double done = D.scal[S_DONE];
+__global__ void __launch_bounds__(64) k_step_begin(DevParams P, DevPtrs D) {
+  if (threadIdx.x <= kArrive) *ctr(D, C_ARRIVE + (int)threadIdx.x, 0) = 0;
+  if (D.scal[S_DONE] == 0.0) step_reset(P, D, threadIdx.x);
+}
+
+// The end of a step, by one wavefront: its time step policy, t = t + dt and
+// counters, then, unless it is the last of its sequence or the run stops, the
+// per-step counters for the next one.  The same as dtpolicy_member,
+// advance_member and reset_member with every load in one round.
+__device__ __forceinline__ void step_commit(const DevParams& P, const DevPtrs& D, bool reset,
+                                            int lane) {
   unsigned long long n = *ctr(D, C_SOLVE_CELLS, lane), nc = *ctr(D, C_COMPUTE_CELLS, lane);
   unsigned long long c0 = *ctr(D, C_STEPS, 0), c1 = *ctr(D, C_ACTIVE_UPD, 0),
-                     c2 = *ctr(D, C_COMPUTE_UPD, 0);
-  double t = D.scal[S_T], dt_old = D.scal[S_DT_OLD];
+                     c2 = *ctr(D, C_COMPUTE_UPD, 0), nt = *ctr(D, C_TILES, 0);
+  double done = D.scal[S_DONE], t = D.scal[S_T], dt_old = D.scal[S_DT_OLD];
   const StepDt r = step_dt(P, D);
   pin(done);
   pin(n);
   pin(nc);
   pin(t);
   pin(dt_old);
+  // the topography pass that follows reads the tile list by this count
+  if (lane == 0) *ctr(D, C_TILES, 1) = nt;
   if (done != 0.0) return;
-  if (commit) {
-    if (r.done) {
-      if (lane == 0) D.scal[S_DONE] = 1.0;
-      return;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      n += __shfl_xor(n, off, 64);
-      nc += __shfl_xor(nc, off, 64);
-    }
-    const double t1 = t + r.dt;
-    // the run stops once t reaches the output time (t_output, snapped to t_end
-    // by the policy), where the reference's loop writes its output
-    const bool stop = t1 >= r.t_out;
-    if (lane == 0) {
-      D.scal[S_DT_CFL] = r.dt_cfl;
-      D.scal[S_DT_OLD_OLD] = dt_old;
-      D.scal[S_DT_OLD] = r.dt;
-      D.scal[S_DT] = r.dt;
-      D.scal[S_T_OUT] = r.t_out;
-      D.scal[S_T] = t1;
-      *ctr(D, C_STEPS, 0) = c0 + 1;
-      *ctr(D, C_ACTIVE_UPD, 0) = c1 + n;
-      *ctr(D, C_COMPUTE_UPD, 0) = c2 + nc;
-      if (stop) D.scal[S_DONE] = 1.0;
-    }
-    if (stop) return;
+  if (r.done) {
+    if (lane == 0) D.scal[S_DONE] = 1.0;
+    return;
   }
-  if (reset) {
-    *ctr(D, C_COMPUTE_CELLS, lane) = 0;
-    if (lane == 0) {
-      *D.dt_bits = (unsigned long long)__double_as_longlong(P.max_dt);
-      *ctr(D, C_TILES, 0) = 0;
-      *ctr(D, C_ROWS, 0) = 0;
-      *ctr(D, C_CELLS, 0) = 0;
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    n += __shfl_xor(n, off, 64);
+    nc += __shfl_xor(nc, off, 64);
   }
+  const double t1 = t + r.dt;
+  // the run stops once t reaches the output time (t_output, snapped to t_end
+  // by the policy), where the reference's loop writes its output
+  const bool stop = t1 >= r.t_out;
+  if (lane == 0) {
+    D.scal[S_DT_CFL] = r.dt_cfl;
+    D.scal[S_DT_OLD_OLD] = dt_old;
+    D.scal[S_DT_OLD] = r.dt;
+    D.scal[S_DT] = r.dt;
+    D.scal[S_T_OUT] = r.t_out;
+    D.scal[S_T] = t1;
+    *ctr(D, C_STEPS, 0) = c0 + 1;
+    *ctr(D, C_ACTIVE_UPD, 0) = c1 + n;
+    *ctr(D, C_COMPUTE_UPD, 0) = c2 + nc;
+    if (stop) D.scal[S_DONE] = 1.0;
+  }
+  if (reset && !stop) step_reset(P, D, lane);
+}
+
+// A workgroup of the step's last pass over the cells has read what it needs of
+// the step's scalars and list lengths (wavefront 0 calls, after a barrier behind
+// those loads); the last one to say so ends the step while the others work.
+// Nothing waits: a workgroup counts itself and goes on.  Two levels, 16
+// counters 512 bytes apart, so that the arrivals of a few hundred workgroups
+// don't queue at one address.  As a launch of its own the step's end took 4.4 us
+// and the gap before it.
+__device__ __forceinline__ void step_arrive(const DevParams& P, const DevPtrs& D, bool reset) {
+  const int lane = threadIdx.x & 63;
+  int last = 0;
+  if (lane == 0) {
+    const unsigned slot = blockIdx.x % kArrive;
+    const unsigned long long quota = (gridDim.x - slot + kArrive - 1) / kArrive;
+    if (atomicAdd(ctr(D, C_ARRIVE + (int)slot, 0), 1ull) == quota - 1)
+      last = atomicAdd(ctr(D, C_ARRIVED, 0), 1ull) ==
+             (unsigned long long)min((int)gridDim.x, kArrive) - 1;
+  }
+  if (!__builtin_amdgcn_readfirstlane(last)) return;
+  if (lane <= kArrive) *ctr(D, C_ARRIVE + lane, 0) = 0;
+  step_commit(P, D, reset, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2173,10 +2203,12 @@ __global__ void __launch_bounds__(64) k_step_begin(DevParams P, DevPtrs D, int c
 // deposition (update_erosion_deposition_cell :2380-2595) and the post-step
 // loop (src/IMEX_SfloW2D.f90:391-447), fused per cell.
 // ---------------------------------------------------------------------------
-// OP_POLICY: the step's dt is step_dt (the policy is committed after the
-// step), else the scalar S_DT
+// OP_POLICY: the step's dt is step_dt (the policy is committed at the end of
+// the step), else the scalar S_DT.  OP_END: this pass ends the step
+// (step_arrive), OP_NEXT: and another one follows in the sequence
 enum LocalOps { OP_RK = 1, OP_EROSION = 2, OP_POST = 4, OP_SUMS = 8, OP_WARM = 16,
-                OP_HARVEST = 32, OP_POLICY = 64, OP_CLOSED = 128 };
+                OP_HARVEST = 32, OP_POLICY = 64, OP_CLOSED = 128, OP_END = 256,
+                OP_NEXT = 512 };
 
 // The assembly checks of imex_RK_solver (src/solver_2d.f90:1379-1624) on
 // the assembled state q of cell c: NaN trap, small or negative thickness,
@@ -2707,6 +2739,10 @@ __global__ void __launch_bounds__(256, (!VP && (PH == 0 || PH == 1)) ? 2 : 1)
     dt = D.scal[S_DT];
   }
   pin(nl_raw);
+  if (ops & OP_END) {
+    __syncthreads();
+    if (w == 0) step_arrive(P, D, ops & OP_NEXT);
+  }
   const int nlist = cells ? (int)min(nl_raw, (unsigned long long)P.nx * P.ny) : (int)nl_raw;
   const int items = (PH >= 3) ? (nlist + kCellsPerWave - 1) / kCellsPerWave
                               : item_count<CELLS>(P, nlist);
@@ -2825,7 +2861,8 @@ __global__ void __launch_bounds__(256) k_topo_list(DevParams P, DevPtrs D) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int tiles_x = (P.nx + kStripW - 1) / kStripW;
   const int tiles_y = (P.ny + kTileH - 1) / kTileH;
-  const int n = (int)*ctr(D, C_TILES, 0);
+  // (the list's length at the step's end: its counter is the next step's already)
+  const int n = (int)*ctr(D, C_TILES, 1);
   for (int item = blockIdx.x; item < 9 * n; item += gridDim.x) {
     const int t = D.tile_list[item / 9], dd = item % 9;
     const int tx = t % tiles_x + dd % 3 - 1, ty = t / tiles_x + dd / 3 - 1;

@@ -317,8 +317,9 @@ int imexsw_stats_get(imexsw_ctx *ctx, imexsw_stats *stats, int reset);
 
 /* Per-kernel device time, measured with HIP events recorded on the
  * context's stream around every launch.  names: mask, stencil, local,
- * topo, dtpolicy (the kernel between steps that commits the time-step
- * policy), post, erosion.  ms[i] accumulates milliseconds, calls[i]
+ * topo, dtpolicy (the kernel before a sequence of steps that clears the
+ * per-step counters; a step's last pass over the cells commits the
+ * time-step policy), post, erosion.  ms[i] accumulates milliseconds, calls[i]
  * launches.  Returns the number of kernels (<= cap).  Timing is enabled by
  * imexsw_set_timing(ctx, 1); while it is on, imexsw_advance launches every
  * kernel directly (the events slow the step). */
