@@ -6,8 +6,7 @@
 // conservative state is NV such planes, the explicit residual D another NV.
 //
 // Kernels per time step (N_RK = 2):
-//   k_step_begin  commit the previous step (host-loop dt policy, t += dt,
-//                 counters) and reset the step's counters
+//   k_step_begin  before a sequence of steps: reset the per-step counters
 //   k_mask        check_solve: active mask (wet cells dilated N_RK times)
 //                 and the step's work lists
 //   k_stencil, k_stencil_rows
@@ -17,7 +16,8 @@
 //                 six wavefronts per listed row on sparse steps
 //   k_local       stage-2 Newton + assembly checks, erosion/deposition,
 //                 post-step diagnostics (dense: two kernels; sparse: one
-//                 pass, four lanes per cell)
+//                 pass, four lanes per cell); its last workgroup to start ends
+//                 the step (host-loop dt policy, t += dt, counters, reset)
 //   k_topo[_list] topography_reconstruction of the slope fields (when the
 //                 topography changes)
 #pragma once
@@ -975,10 +975,10 @@ __device__ __forceinline__ void load_src(const DevParams& P, const DevPtrs& D, i
 // ---------------------------------------------------------------------------
 // k_stencil: the stage-1 stencil pass (timestep + eval_hyperbolic_terms +
 // eval_expl_terms at q^n).  One wavefront marches up a strip of rows keeping
-// a three-row window of physical states in registers; lane l owns column
+// the rows it still needs in registers; lane l owns column
 // j = 60*tile_x - 2 + l.  Lanes 2..61 are the strip's cells, lanes 1 and
 // 62 reconstruct the halo sides of the strip's outer faces, lanes 0 and 63
-// only supply states.  x neighbours are exchanged with wave shuffles; rows
+// only supply states.  x neighbours are exchanged with wave rotations; rows
 // k0-2 .. k1+1 are read once each.
 // ---------------------------------------------------------------------------
 // Conservative state of cell (j, k) from a clamped, always valid address:
