@@ -7,17 +7,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "imexsw_ctx.h"
+#include "imexsw_pin.h"
 #include "imexsw_q2d.h"
 
 using namespace imexsw;
@@ -466,12 +465,26 @@ int put(imexsw_ctx* c, const Put& p) {
 }
 
 // the active-cell count and the CFL minimum, written by the device into pinned
-// host memory; waits for the stream
-int get_results(imexsw_ctx* c) {
-  if (!c->h_res) HIPCHK(c, hipHostMalloc((void**)&c->h_res, 2 * sizeof(unsigned long long)));
+// host memory, or copied if there is none; waits for the stream
+int get_results(imexsw_ctx* c, unsigned long long* cells, unsigned long long* dt_bits) {
+  if (!c->h_res &&
+      hipHostMalloc((void**)&c->h_res, 2 * sizeof(unsigned long long)) != hipSuccess) {
+    c->h_res = nullptr;
+    (void)hipGetLastError();
+    unsigned long long v[kSlots];
+    HIPCHK(c, hipMemcpyAsync(v, c->D.counters + C_SOLVE_CELLS * kSlots, sizeof v,
+                             hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(dt_bits, c->D.dt_bits, sizeof *dt_bits, hipMemcpyDeviceToHost,
+                             c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    *cells = sum_slots(v);
+    return 0;
+  }
   hipLaunchKernelGGL(k_host_get<>, dim3(1), dim3(64), 0, c->stream, c->D, c->h_res);
   if (check_launch(c, "k_host_get")) return -1;
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  *cells = c->h_res[0];
+  *dt_bits = c->h_res[1];
   return 0;
 }
 
@@ -491,136 +504,10 @@ int ensure_stage(imexsw_ctx* c, size_t bytes) {
   return 0;
 }
 
-// Pinned memory that large downloads pass through: two chunks for the process,
-// held while contexts exist and used by one download at a time (another that
-// overlaps it copies directly).
-constexpr size_t kPinChunk = (size_t)4 << 20;
-constexpr size_t kPinMin = (size_t)256 << 10;  // downloads below it are copied directly
-struct PinPool {
-  std::mutex mu;       // the chunks
-  std::mutex count_mu; // users
-  int users = 0;
-  char* mem = nullptr;
-  hipEvent_t ev[2] = {nullptr, nullptr};
-  int device = -1;
-};
-PinPool g_pin;
-
-void pin_acquire() {
-  std::lock_guard<std::mutex> lk(g_pin.count_mu);
-  g_pin.users++;
-}
-void pin_drop() {
-  for (hipEvent_t& e : g_pin.ev) {
-    if (e) (void)hipEventDestroy(e);
-    e = nullptr;
-  }
-  if (g_pin.mem) (void)hipHostFree(g_pin.mem);
-  g_pin.mem = nullptr;
-  g_pin.device = -1;
-}
-void pin_release() {
-  std::lock_guard<std::mutex> lk(g_pin.count_mu);
-  if (--g_pin.users > 0) return;
-  std::lock_guard<std::mutex> lk2(g_pin.mu);
-  pin_drop();
-}
-
-// The chunks of one download: chunk i of the device memory arrives in half
-// i % 2 of the pinned memory, and the caller and its helpers copy a slice each
-// to the host array.
-struct ChunkCopy {
-  char* host;
-  const char* pin;
-  size_t bytes, chunks;
-  int parts;
-  std::atomic<size_t> ready{0};  // chunks that have arrived
-  std::atomic<size_t> done[2];   // slices copied out of each half, in all
-  std::atomic<bool> stop{false};
-  void slice(size_t i, int part) {
-    const size_t at = i * kPinChunk, len = std::min(kPinChunk, bytes - at);
-    const size_t per = (len / parts + 4095) / 4096 * 4096;
-    const size_t o = std::min(len, per * part);
-    const size_t n = (part == parts - 1) ? len - o : std::min(per, len - o);
-    if (n) std::memcpy(host + at + o, pin + (i & 1) * kPinChunk + o, n);
-    done[i & 1].fetch_add(1, std::memory_order_release);
-  }
-  void help(int part) {
-    for (size_t i = 0; i < chunks; i++) {
-      while (ready.load(std::memory_order_acquire) <= i) {
-        if (stop.load(std::memory_order_acquire)) return;
-        std::this_thread::yield();
-      }
-      slice(i, part);
-    }
-  }
-};
-
-// Device memory to a host array, after the stream's work.  A copy into
-// pageable memory runs at 17 GB/s, and at 10 GB/s into an array whose pages are
-// touched for the first time, as an output array's are; through pinned chunks
-// the transfer overlaps the copy out of them, which several threads make for a
-// large array (they fault its pages side by side).
-int copy_to_host(imexsw_ctx* c, void* host, const void* dev, size_t bytes) {
-  std::unique_lock<std::mutex> lk(g_pin.mu, std::defer_lock);
-  if (bytes < kPinMin || !lk.try_lock()) {
-    HIPCHK(c, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return 0;
-  }
-  if (g_pin.device != c->device) pin_drop();
-  if (!g_pin.mem) {
-    HIPCHK(c, hipHostMalloc((void**)&g_pin.mem, 2 * kPinChunk));
-    g_pin.device = c->device;
-    for (hipEvent_t& e : g_pin.ev) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
-  ChunkCopy w;
-  w.host = static_cast<char*>(host);
-  w.pin = g_pin.mem;
-  w.bytes = bytes;
-  w.chunks = (bytes + kPinChunk - 1) / kPinChunk;
-  w.done[0] = w.done[1] = 0;
-  // one thread for every 4 MiB, at most 8
-  w.parts = (int)std::min<size_t>(8, std::max<size_t>(1, bytes / kPinChunk));
-  std::vector<std::thread> helpers;
-  int started = 1;
-  try {
-    helpers.reserve(w.parts);
-    // (the slices are fixed before the first helper runs: a helper that
-    // cannot be started leaves its slices to the caller)
-    for (int p = 1; p < w.parts; p++, started++) helpers.emplace_back([&w, p] { w.help(p); });
-  } catch (...) {
-  }
-  const char* d = static_cast<const char*>(dev);
-  auto send = [&](size_t i) -> hipError_t {
-    const size_t at = i * kPinChunk;
-    hipError_t e = hipMemcpyAsync(g_pin.mem + (i & 1) * kPinChunk, d + at,
-                                  std::min(kPinChunk, bytes - at), hipMemcpyDeviceToHost,
-                                  c->stream);
-    return e == hipSuccess ? hipEventRecord(g_pin.ev[i & 1], c->stream) : e;
-  };
-  hipError_t err = send(0);
-  if (err == hipSuccess && w.chunks > 1) err = send(1);
-  for (size_t i = 0; err == hipSuccess && i < w.chunks; i++) {
-    err = hipEventSynchronize(g_pin.ev[i & 1]);
-    if (err != hipSuccess) break;
-    w.ready.store(i + 1, std::memory_order_release);
-    w.slice(i, 0);
-    for (int p = started; p < w.parts; p++) w.slice(i, p);
-    if (i + 2 < w.chunks) {
-      // the half is free once every slice of this chunk is out of it
-      const size_t want = (size_t)w.parts * (i / 2 + 1);
-      while (w.done[i & 1].load(std::memory_order_acquire) < want) std::this_thread::yield();
-      err = send(i + 2);
-    }
-  }
-  if (err != hipSuccess) w.stop.store(true, std::memory_order_release);
-  for (std::thread& t : helpers) t.join();
-  if (err != hipSuccess) {
-    (void)hipStreamSynchronize(c->stream);
-    return fail(c, "download: %s", hipGetErrorString(err));
-  }
-  return 0;
+// device memory to a host array, after the work queued on the context's stream
+int to_host(imexsw_ctx* c, void* host, const void* dev, size_t bytes) {
+  const hipError_t e = copy_to_host(c->stream, c->device, host, dev, bytes);
+  return e == hipSuccess ? 0 : fail(c, "download: %s", hipGetErrorString(e));
 }
 
 // host (nvar, nx, ny) Fortran array -> nvar device planes
@@ -641,7 +528,7 @@ int download_aos(imexsw_ctx* c, const double* src, int nvar, double* host) {
   hipLaunchKernelGGL(k_planes_to_aos<>, c->grid_tiles, dim3(256), 0, c->stream, c->P, src, nvar,
                      c->stage, 0, c->P.ny);
   if (check_launch(c, "k_planes_to_aos")) return -1;
-  return copy_to_host(c, host, c->stage, n * sizeof(double));
+  return to_host(c, host, c->stage, n * sizeof(double));
 }
 
 // host (nx, ny) Fortran plane <-> device plane with pitch
@@ -663,7 +550,7 @@ int download_plane(imexsw_ctx* c, const T* src, T* host) {
   T* st = reinterpret_cast<T*>(c->stage);
   hipLaunchKernelGGL(k_plane_pack<T>, c->grid_tiles, dim3(256), 0, c->stream, c->P, src, st);
   if (check_launch(c, "k_plane_pack")) return -1;
-  return copy_to_host(c, host, st, n * sizeof(T));
+  return to_host(c, host, st, n * sizeof(T));
 }
 // the staggered planes (set-up only): w x h values, pitch d
 int upload_staggered(imexsw_ctx* c, const double* host, double* dst, int w, int h, size_t d) {
@@ -1091,8 +978,9 @@ int imexsw_check_solve(imexsw_ctx* c, int solve_all, double t, int32_t* solve_ce
   HIPCHK(c, hipMemsetAsync(c->D.tile_dirty, 1, (size_t)c->n_tiles, c->stream));
   c->d_valid = false;
   if (solve_cells) {
-    if (get_results(c)) return -1;
-    *solve_cells = (int32_t)c->h_res[0];
+    unsigned long long n, bits;
+    if (get_results(c, &n, &bits)) return -1;
+    *solve_cells = (int32_t)n;
   }
   return 0;
 }
@@ -1103,9 +991,10 @@ int imexsw_timestep(imexsw_ctx* c, double* dt) {
   // stopped in
   if (put(c, Put().scal(S_DONE, 0.0).dt_bits())) return -1;
   if (run_stencil(c, c->P.cfl != -1.0)) return -1;
-  if (get_results(c)) return -1;
+  unsigned long long n, bits;
+  if (get_results(c, &n, &bits)) return -1;
   double v;
-  std::memcpy(&v, &c->h_res[1], sizeof v);
+  std::memcpy(&v, &bits, sizeof v);
   *dt = (c->P.cfl != -1.0) ? v : c->P.max_dt;
   return 0;
 }
@@ -1283,7 +1172,7 @@ int imexsw_download(imexsw_ctx* c, double* q, double* qp, double* hmax, double* 
     NS_SWITCH(c->ns, CALL)
 #undef CALL
     if (check_launch(c, "k_qp_out")) return -1;
-    if (copy_to_host(c, qp, c->stage, n * sizeof(double))) return -1;
+    if (to_host(c, qp, c->stage, n * sizeof(double))) return -1;
   }
   if (hmax && download_plane(c, c->D.hmax, hmax)) return -1;
   if (pdynmax && download_plane(c, c->D.pdynmax, pdynmax)) return -1;
