@@ -25,7 +25,8 @@ PARTS = range(0, 5)
 SOURCES = ["imexsw.hip", "imexsw_ns.hip"]
 HEADERS = ["imexsw_math.h", "imexsw_physics.h", "imexsw_newton.h", "imexsw_kernels.h",
            "imexsw_batch.h", "imexsw_mlp.h", "imexsw_q2d.h", "imexsw_ctx.h",
-           "imexsw_stages.h", "imexsw_profiles.h", "imexsw_pin.h"]
+           "imexsw_stages.h", "imexsw_profiles.h", "imexsw_pin.h",
+           "imexsw_strips.h"]
 ARCH = os.environ.get("IMEXSW_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

@@ -3,6 +3,7 @@
 // -DIMEXSW_PART=<0..4> so that the instantiations build in parallel (the C
 // ABI is in imexsw.hip).
 #include "imexsw_ctx.h"
+#include "imexsw_strips.h"
 
 #if !defined(IMEXSW_NS) || !defined(IMEXSW_PART)
 #error "compile with -DIMEXSW_NS=<number of solid classes> -DIMEXSW_PART=<0..4>"
@@ -10,23 +11,12 @@
 
 namespace imexsw {
 
-// Rows per whole-column strip (k_stencil) for `slots` resident wavefronts: the
-// height whose rounds take least, with the strip's own overhead; 0 with a
-// tuning other than the default, which asks for the tile strips it describes.
+// Rows per whole-column strip (k_stencil) for `slots` resident wavefronts; 0
+// with a tuning other than the default, which asks for the tile strips it
+// describes.
 static int column_height(const imexsw_ctx* c, int slots) {
   if (c->P.ny < 2 || c->strip_h != kTileH || c->target_strips != kDefaultStrips) return 0;
-  const int tiles_x = (c->P.nx + kStripW - 1) / kStripW;
-  int best = 1;
-  long cost = -1;
-  for (int h = 1; h <= c->P.ny; h++) {
-    const long items = (long)tiles_x * ((c->P.ny + h - 1) / h);
-    const long t = (items + slots - 1) / slots * (h + kStripOver);
-    if (cost < 0 || t < cost) {
-      cost = t;
-      best = h;
-    }
-  }
-  return best;
+  return column_rows((c->P.nx + kStripW - 1) / kStripW, c->P.ny, slots, kStripOver);
 }
 
 // Workgroups of four wavefronts for every item of item_cell: cells 64 to a
