@@ -272,11 +272,44 @@ int init_stages(imexsw_ctx* c) {
   return check_launch(c, "kg_stage_init");
 }
 
+// Sparse steps with few computed cells, N_RK = 2 and no harvest (the harvest
+// runs in the dense stage kernel).  The sparse form spends four lanes on a
+// cell and six wavefronts on a row to shorten one cell's chain, the dense form
+// has twice its latency and a quarter of its work: with the default tuning the
+// line is at 24576 cells (step times, three classes: 10.9k cells 148 us sparse,
+// 171 dense; 16.8k 183 / 171; 42k 325 / 206; two classes: 17k 123 / 135, 27k
+// 148 / 137).  With another tuning it is where its strips become one row high.
+constexpr unsigned long long kSparseCells = 24576;
+bool has_sparse(const imexsw_ctx* c) { return !c->general && !c->D.harvest && c->P.ny >= 2; }
+bool want_sparse(const imexsw_ctx* c, unsigned long long w) {
+  if (!has_sparse(c)) return false;
+  if (c->strip_h == kTileH && c->target_strips == kDefaultStrips) return w < kSparseCells;
+  return c->strip_h < 2 ||
+         w / (unsigned long long)(kStripW * 2) < (unsigned long long)c->target_strips;
+}
+
+unsigned long long sum_slots(const unsigned long long* v) {
+  unsigned long long s = 0;
+  for (int i = 0; i < kSlots; i++) s += v[i];
+  return s;
+}
+
+// The form of the step just begun from its own mask's count; waits for the mask.
+int choose_form(imexsw_ctx* c) {
+  HIPCHK(c, hipMemcpyAsync(c->h_cnt, c->D.counters + C_COMPUTE_CELLS * kSlots,
+                           kSlots * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                           c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->sparse = want_sparse(c, sum_slots(c->h_cnt));
+  return 0;
+}
+
 // one time step of the main loop (src/IMEX_SfloW2D.f90:337-531), all on the
 // context's stream, of a sequence whose first and last steps are marked.  The
 // last pass over the cells ends the step (time step policy, t, counters), for
-// which the stage kernel applies the policy itself.
-int enqueue_step(imexsw_ctx* c, bool first, bool last) {
+// which the stage kernel applies the policy itself.  choose: its form from its
+// own count of computed cells (choose_form), else the context's.
+int enqueue_step(imexsw_ctx* c, bool first, bool last, bool choose = false) {
   if (first) {
     Timed tm(c, K_DTPOLICY);
     hipLaunchKernelGGL(k_step_begin<>, dim3(1), dim3(64), 0, c->stream, c->P, c->D);
@@ -291,6 +324,7 @@ int enqueue_step(imexsw_ctx* c, bool first, bool last) {
     return check_launch(c, "step");
   }
   if (run_mask(c, 0, 1)) return -1;
+  if (choose && choose_form(c)) return -1;
   if (run_stencil(c, c->P.cfl != -1.0, c->sparse)) return -1;
   if (run_local(c, OP_RK | OP_EROSION | OP_POST | end, K_LOCAL, c->sparse)) return -1;
   if (c->P.topo && run_topo(c, c->sparse ? 2 : 1)) return -1;
@@ -304,21 +338,6 @@ void drop_ctx_graph(imexsw_ctx* c) {
     c->exec[m] = nullptr;
     c->graph[m] = nullptr;
   }
-}
-
-// Sparse steps with few computed cells, N_RK = 2 and no harvest (the harvest
-// runs in the dense stage kernel).  The sparse form spends four lanes on a
-// cell and six wavefronts on a row to shorten one cell's chain, the dense form
-// has twice its latency and a quarter of its work: with the default tuning the
-// line is at 24576 cells (step times, three classes: 10.9k cells 148 us sparse,
-// 171 dense; 16.8k 183 / 171; 42k 325 / 206; two classes: 17k 123 / 135, 27k
-// 148 / 137).  With another tuning it is where its strips become one row high.
-constexpr unsigned long long kSparseCells = 24576;
-bool want_sparse(const imexsw_ctx* c, unsigned long long w) {
-  if (c->general || c->D.harvest || c->P.ny < 2) return false;
-  if (c->strip_h == kTileH && c->target_strips == kDefaultStrips) return w < kSparseCells;
-  return c->strip_h < 2 ||
-         w / (unsigned long long)(kStripW * 2) < (unsigned long long)c->target_strips;
 }
 
 // Capture kGraphSteps steps of the sparse (m = 1) or dense (m = 0) form
@@ -342,12 +361,6 @@ int capture_steps(imexsw_ctx* c, int m) {
   c->graph[m] = g;
   HIPCHK(c, hipGraphInstantiate(&c->exec[m], g, nullptr, nullptr, 0));
   return 0;
-}
-
-unsigned long long sum_slots(const unsigned long long* v) {
-  unsigned long long s = 0;
-  for (int i = 0; i < kSlots; i++) s += v[i];
-  return s;
 }
 
 // Gauss-Legendre points and weights on [-1, 1] in ascending order (the
@@ -931,6 +944,7 @@ int imexsw_set_source(imexsw_ctx* c, const int32_t* source_cell, const uint8_t* 
   HIPCHK(c, hipMemsetAsync(D.tile_dirty, 1, (size_t)c->n_tiles, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->d_valid = false;
+  c->cells_known = false;
   return 0;
 }
 
@@ -949,6 +963,7 @@ int imexsw_upload_q(imexsw_ctx* c, const double* q) {
   HIPCHK(c, hipMemsetAsync(c->D.tile_dirty, 1, (size_t)c->n_tiles, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->d_valid = false;
+  c->cells_known = false;
   // a new state starts a new run: the next imexsw_advance takes its step
   // history from dt0 again
   c->dt_hist = false;
@@ -977,6 +992,7 @@ int imexsw_check_solve(imexsw_ctx* c, int solve_all, double t, int32_t* solve_ce
   // scans every tile again
   HIPCHK(c, hipMemsetAsync(c->D.tile_dirty, 1, (size_t)c->n_tiles, c->stream));
   c->d_valid = false;
+  c->cells_known = false;
   if (solve_cells) {
     unsigned long long n, bits;
     if (get_results(c, &n, &bits)) return -1;
@@ -1092,7 +1108,22 @@ int imexsw_advance(imexsw_ctx* c, int32_t nsteps, double dt0, double* t_io, doub
   HIPCHK(c, hipMemcpyAsync(c->h_cnt, d_cnt, kSlots * sizeof(unsigned long long),
                            hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->sparse = want_sparse(c, sum_slots(c->h_cnt));
+  int n = 0;
+  bool stop = false;
+  if (c->cells_known || !has_sparse(c)) {
+    c->sparse = want_sparse(c, sum_slots(c->h_cnt));
+  } else {
+    // A state without a count of its own (the counter holds another run's last
+    // step, or check_solve's): its first steps one at a time, each in the form
+    // that its own count asks for.  Three, because a new state's thin margin is
+    // computed once or twice and then gone (512 x 512 incline: 91 458 cells,
+    // 34 186, 21 898, 21 405; 256 x 256: 57 786, 25 560, 20 472, 20 079).
+    for (; n < 3 && n < nsteps; n++) {
+      if (enqueue_step(c, true, true, true)) return -1;
+      if (c->sparse) c->sparse_steps++;
+    }
+  }
+  c->cells_known = true;
   // Without per-kernel timing the steps run as replays of a captured graph
   // of kGraphSteps steps (one host call per replay instead of eight kernel
   // launches per step); the rest, and every step when timing, is launched
@@ -1103,8 +1134,6 @@ int imexsw_advance(imexsw_ctx* c, int32_t nsteps, double dt0, double* t_io, doub
   // always has a replay queued), and the flag ends the call once the run has
   // reached t_output or t_end (the steps after that are no-ops on the
   // device).
-  int n = 0;
-  bool stop = false;
   if (!c->timing && nsteps >= kGraphSteps) {
     if (std::memcmp(&c->graph_P, &c->P, sizeof(DevParams)) ||
         std::memcmp(&c->graph_D, &c->D, sizeof(DevPtrs)) ||
@@ -1144,7 +1173,7 @@ int imexsw_advance(imexsw_ctx* c, int32_t nsteps, double dt0, double* t_io, doub
       double done = 0.0;
       HIPCHK(c, hipMemcpyAsync(&done, c->D.scal + S_DONE, sizeof done, hipMemcpyDeviceToHost,
                                c->stream));
-      HIPCHK(c, hipStreamSynchronize(c->stream));
+      if (choose_form(c)) return -1;
       if (done != 0.0) break;
     }
     if (enqueue_step(c, true, true)) return -1;

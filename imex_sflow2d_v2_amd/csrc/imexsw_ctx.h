@@ -62,9 +62,11 @@ struct imexsw_ctx {
   bool closed_start = false;
   MlpDev mlp{};
   // sparse steps (few computed cells): the row stencil and the fused local
-  // kernel; chosen on the host from the computed-cell count of an earlier
-  // step (both ways give the same bits)
+  // kernel; chosen on the host from the computed-cell count of the step or an
+  // earlier one of the same run (both ways give the same bits).  cells_known:
+  // the device's counter is of the last step of the present state.
   bool sparse = false;
+  bool cells_known = false;
   int64_t sparse_steps = 0;
   unsigned long long* h_cnt = nullptr;  // pinned: 2 x kSlots computed-cell counters
   double* h_done = nullptr;             // pinned: 2 copies of the run's done flag

@@ -1,0 +1,69 @@
+"""The form of the steps (sparse or dense) comes from the state they run on, not
+from another run's counter: a state takes as many sparse steps on a new context
+as after a run that left few or many cells behind, and gives the same bits.
+Steps by the captured sequences, one at a time and in several calls."""
+import numpy as np
+import pytest
+
+from imex_sflow2d_v2_amd import decks
+from imex_sflow2d_v2_amd.solver import Solver
+
+pytestmark = pytest.mark.gpu
+
+
+def small():
+    """A column of some 2 000 computed cells on a 260 x 260 grid."""
+    d = decks.small_2d(n=260, seed=5)
+    d.q[:, 130:] = 0.0
+    d.q[:, :, 140:] = 0.0
+    d.q[:, :60] = 0.0
+    d.q[:, :, :100] = 0.0
+    return d
+
+
+def wide():
+    """The same grid, wet everywhere: more cells than any sparse step is for."""
+    return decks.small_2d(n=260, seed=5, wet_floor=0.5)
+
+
+def run(s, d, calls):
+    before = s.stats()["sparse_steps"]
+    s.upload_q(d.q)
+    s.t = 0.0
+    for n in calls:
+        s.advance(n, dt0=d.dt0)
+    return s.stats()["sparse_steps"] - before, s.q()
+
+
+@pytest.mark.parametrize("calls", [(1,), (19,), (20,), (65,), (1, 41, 23)])
+def test_form_of_a_new_state(calls):
+    print("form", calls, flush=True)
+    few, many = small(), wide()
+    # check_solve counts every cell of a new context
+    new = Solver(few.params).load_deck(few)
+    n_few, q_few = run(new, few, calls)
+    assert n_few == sum(calls)
+    # after a run with many cells, and after one with few
+    n_many, q_many = run(new, many, calls)
+    assert n_many == 0
+    n, q = run(new, few, calls)
+    assert n == n_few and np.array_equal(q, q_few)
+    n, q = run(new, few, calls)
+    assert n == n_few and np.array_equal(q, q_few)
+    other = Solver(many.params).load_deck(many)
+    n, q = run(other, many, calls)
+    assert n == 0 and np.array_equal(q, q_many)
+    # timed launches look again, too
+    other.set_timing(True)
+    n, q = run(other, few, calls)
+    assert n == n_few and np.array_equal(q, q_few)
+
+
+def test_new_and_repeated_run_of_a_collapse():
+    """A collapse whose first step has most cells: the same steps in the same
+    form on a new context and again on the same one."""
+    d = decks.incline_2d(n=256)
+    s = Solver(d.params).load_deck(d)
+    a, qa = run(s, d, (80,))
+    b, qb = run(s, d, (80,))
+    assert a == b >= 77 and np.array_equal(qa, qb)
