@@ -273,17 +273,24 @@ int init_stages(imexsw_ctx* c) {
 }
 
 // Sparse steps with few computed cells, N_RK = 2 and no harvest (the harvest
-// runs in the dense stage kernel).  The sparse form spends four lanes on a
-// cell and six wavefronts on a row to shorten one cell's chain, the dense form
-// has twice its latency and a quarter of its work: with the default tuning the
-// line is at 24576 cells (step times, three classes: 10.9k cells 148 us sparse,
-// 171 dense; 16.8k 183 / 171; 42k 325 / 206; two classes: 17k 123 / 135, 27k
-// 148 / 137).  With another tuning it is where its strips become one row high.
-constexpr unsigned long long kSparseCells = 24576;
+// runs in the dense stage kernel).  The sparse form spends four lanes on a cell
+// and six wavefronts on a row to shorten one cell's chain: its time grows with
+// the cells and their classes, while the dense form waits for its longest Newton
+// solves (130 to 190 us a step) and has room for more cells beside them.  With
+// the default tuning the line lies where they cross, us a step, sparse / dense:
+// one class    26k cells 111 / 152, 40k 122 / 131, 55k 146 / 156, 77k 167 / 154;
+// two classes  26k 133 / 161, 35k 153 / 173 to 151 / 153, 39k 153 / 146,
+//              55k 184 / 168;
+// three        24k 126 / 142, 28k 153 / 180, 36k 166 / 170, 43k 171 / 158,
+//              56k 216 / 187
+// (collapses with and without erosion, slope correction, wet beds and the closed
+// start; more classes as three).  With another tuning it is where its strips
+// become one row high.
 bool has_sparse(const imexsw_ctx* c) { return !c->general && !c->D.harvest && c->P.ny >= 2; }
 bool want_sparse(const imexsw_ctx* c, unsigned long long w) {
   if (!has_sparse(c)) return false;
-  if (c->strip_h == kTileH && c->target_strips == kDefaultStrips) return w < kSparseCells;
+  if (c->strip_h == kTileH && c->target_strips == kDefaultStrips)
+    return w < (c->ns < 2 ? 53248u : 36864u);
   return c->strip_h < 2 ||
          w / (unsigned long long)(kStripW * 2) < (unsigned long long)c->target_strips;
 }

@@ -67,3 +67,21 @@ def test_new_and_repeated_run_of_a_collapse():
     a, qa = run(s, d, (80,))
     b, qb = run(s, d, (80,))
     assert a == b >= 77 and np.array_equal(qa, qb)
+
+
+@pytest.mark.parametrize("ns,n,lo,hi,sparse", [
+    (1, 190, 25000, 36000, True), (1, 225, 40000, 53247, True), (1, 270, 53248, 73000, False),
+    (2, 190, 25000, 36863, True), (2, 225, 36864, 53247, False),
+    (3, 190, 25000, 36863, True), (3, 225, 36864, 53247, False)])
+def test_line_between_the_forms(ns, n, lo, hi, sparse):
+    """The default's form on either side of the line of each number of classes."""
+    d = decks.small_2d(n=n, seed=4, wet_floor=0.5, n_solid=ns)
+    s = Solver(d.params).load_deck(d)
+    taken, q = run(s, d, (4,))
+    st = s.stats()
+    print("line", ns, n, st["compute_cells"], taken, flush=True)
+    assert lo <= st["compute_cells"] <= hi
+    assert taken == (4 if sparse else 0)
+    s.set_tuning(16, 1 if sparse else 1 << 20)  # the other form
+    other, q2 = run(s, d, (4,))
+    assert other == 4 - taken and np.array_equal(q, q2)
