@@ -13,16 +13,19 @@ from oracle import Oracle
 
 pytestmark = pytest.mark.gpu
 
-# Found by this test and independent of where a step ends: with N_RK = 3 the
-# device leaves the oracle on some of these decks (130 x 33: 18 Newton iterations
-# fewer over 61 steps, states 1e-13 of the largest apart, then growing), with the
-# same bits when the step's end was a launch of its own.
-NRK3 = pytest.mark.xfail(reason="N_RK = 3 differs from the oracle on some decks", strict=False)
+# With N_RK = 3 and two or three classes a run may reach the NaN trap
+# (src/solver_2d.f90:1379-1394), where the reference stops: at an x face whose mass
+# flux cancels to exactly zero and one of whose classes has no flux, the cap on the
+# solid fluxes (:2832-3047) is 0 / 0.  Whether it does hangs on the last bit of the
+# initial state.  Both sides reach it then, and nothing after it is compared
+# (beside a NaN the device's limited slope is zero, the oracle's is NaN).  One class
+# has no such face.
 
 
 @pytest.mark.parametrize("kw", [{}, dict(erosion=True, topo_change=True),
                                 dict(rheology_model=6, friction_factor=2e-3),
-                                pytest.param(dict(n_rk=3), marks=NRK3)])
+                                dict(n_rk=3), dict(n_rk=3, n_solid=1),
+                                dict(n_rk=3, n_solid=3)])
 @pytest.mark.parametrize("n,ny", [(8, 8), (31, 31), (33, 31), (130, 33)])
 @pytest.mark.parametrize("sparse", [False, True])
 def test_step_end(n, ny, kw, sparse):
@@ -31,10 +34,15 @@ def test_step_end(n, ny, kw, sparse):
     orc = Oracle(d.params, fresh=True).load_deck(d)
     dev = Solver(d.params).load_deck(d)
     dev.set_tuning(target_strips=1 << 20 if sparse else 1)
+    trap = kw.get("n_rk") == 3 and kw.get("n_solid") != 1
     for steps, t_out in ((1, 1e30), (61, 1e30), (1 << 20, None), (1 << 20, None), (27, 1e30)):
         t_out = orc.t + 0.21 if t_out is None else t_out
         a = orc.run(steps, dt0=d.dt0, t_end=1e30, t_output=t_out)
-        assert dev.advance(steps, dt0=d.dt0, t_end=1e30, t_output=t_out) == a
+        b = dev.advance(steps, dt0=d.dt0, t_end=1e30, t_output=t_out)
+        if trap and orc.counters()["nan"]:
+            assert dev.stats()["nan_events"] > 0
+            return
+        assert b == a
         assert dev.t == orc.t and dev.get_dt() == orc.dt_last[0]
         q, ref = dev.q(), orc.q()
         for v in range(ref.shape[0]):

@@ -1,9 +1,9 @@
-"""The strips of the dense stencil pass: whole-column strips (every tile
-listed) at the edges of tiles and of the device's strip heights, tile strips
-with the fitted height, and the fixed heights of imexsw_set_tuning, all
-against the oracle; and an ensemble with the fitted height against the fixed
-ones.  The faces are the same operations in every cut, so the bar is 1e-13 of
-each variable's largest value against the oracle and equality between cuts."""
+"""The strips of the dense stencil pass against the oracle: the fixed heights of
+imexsw_set_tuning at the edges of tiles, and the default's, whole-column strips
+(every tile listed) and tile strips of the fitted height (a dry corner); and an
+ensemble with the fitted height against the fixed ones.  The faces are the same
+operations in every cut, so the bar is 1e-13 of each variable's largest value
+against the oracle and equality between cuts."""
 import numpy as np
 import pytest
 
@@ -29,8 +29,8 @@ def state(d, tuning, steps):
     (181, 5, dict(n_solid=1, alpha=True))])
 def test_strip_cuts(nx, ny, kw, wet):
     d = decks.small_2d(n=nx, ny=ny, seed=3, wet_floor=wet, **kw)
-    # the smallest target leaves the dense form: heights 1 and 16, and the
-    # default's strips on a grid whose computed cells exceed its target
+    # the smallest target leaves the dense form, in tile strips of at most 16, 1
+    # and 4 rows (the default's strips: test_default_strips, test_default_strips_rich)
     cuts = [state(d, t, 21) for t in ((16, 1), (1, 1), (4, 1))]
     orc = Oracle(d.params, fresh=True).load_deck(d)
     orc.run(21, dt0=d.dt0)
@@ -43,8 +43,8 @@ def test_strip_cuts(nx, ny, kw, wet):
 
 @pytest.mark.parametrize("nx,ny,dry", [(601, 420, False), (540, 513, False), (600, 470, True)])
 def test_default_strips(nx, ny, dry):
-    """Above 245 760 computed cells the default takes the dense form with
-    column strips (all tiles wet) or fitted tile strips (a dry corner)."""
+    """Above 53 248 computed cells (one class) the default takes the dense form,
+    with column strips (all tiles wet) or fitted tile strips (a dry corner)."""
     d = decks.small_2d(n=nx, ny=ny, seed=4, wet_floor=0.5, n_solid=1)
     if dry:
         d.q[:, -70:, -20:] = 0.0
@@ -52,6 +52,31 @@ def test_default_strips(nx, ny, dry):
     assert np.array_equal(a, state(d, (8, 1), 5))
     orc = Oracle(d.params, fresh=True).load_deck(d)
     orc.run(5, dt0=d.dt0)
+    ref = orc.q()
+    for v in range(ref.shape[0]):
+        assert np.abs(a[v] - ref[v]).max() <= 1e-13 * max(np.abs(ref[v]).max(), 1e-300)
+
+
+# Grids of 47 000 to 50 000 cells, above the line of two and three classes, with a
+# last tile of one column (241) or one row (193 = 12 * 16 + 1) and strips that do
+# not divide the rows
+@pytest.mark.parametrize("dry", [False, True])
+@pytest.mark.parametrize("nx,ny,kw", [
+    (241, 207, dict(source=True)), (260, 193, dict(slope_correction=True, curvature=True)),
+    (241, 193, dict(limiter=[1, 2, 1, 3, 5, 1])), (259, 191, dict(limiter=4, n_solid=3)),
+    (300, 161, dict(n_solid=3, alpha=True, erosion=True, topo_change=True))])
+def test_default_strips_rich(nx, ny, kw, dry):
+    print("default strips", nx, ny, kw, dry, flush=True)
+    d = decks.small_2d(n=nx, ny=ny, seed=6, wet_floor=0.5, **kw)
+    if dry:
+        d.q[:, -70:, -25:] = 0.0
+    s = Solver(d.params).load_deck(d)
+    s.advance(6, dt0=d.dt0)
+    assert s.stats()["sparse_steps"] == 0
+    a = s.q()
+    assert np.array_equal(a, state(d, (4, 1), 6))
+    orc = Oracle(d.params, fresh=True).load_deck(d)
+    orc.run(6, dt0=d.dt0)
     ref = orc.q()
     for v in range(ref.shape[0]):
         assert np.abs(a[v] - ref[v]).max() <= 1e-13 * max(np.abs(ref[v]).max(), 1e-300)

@@ -1,7 +1,7 @@
 """N_RK = 2 in the tableau-driven pipeline (rheology models 6 and 8, vertical
 profiles): one launch for the second stage and the assembly, the mask of the
 plain path with every active cell computed and rescans of changed tiles only.
-Ragged sizes around the work tile (60 x 32) and the wavefront, dry fronts, the
+Ragged sizes around the work tile (60 x 16) and the wavefront, dry fronts, the
 source ring, erosion with a changing bed.  Against the oracle, by the time loop
 (graph replays and the remainder) and by the procedures one at a time: the
 operations are the same, so states within 1e-13 of each variable's largest
