@@ -115,7 +115,7 @@ __device__ __forceinline__ double vp_h0(const DevParams& P, double r_h) {
 // The mean speed's iteration reads each point's logarithm four to twenty
 // times: the first kVpCache points' stay in LDS, one column per lane of the
 // workgroup (at most kVpLanes), the rest are formed again.  40 KB a workgroup:
-// four fit a CU, one more than the registers allow.  500 x 386, model 8, two
+// four fit a CU, the registers allow two or three.  500 x 386, model 8, two
 // conversions a cell: stage kernel 630 us with every logarithm formed each time,
 // 487 from LDS, 458 with the points unrolled and without range selects, 380 with
 // full wavefronts (item_cell).

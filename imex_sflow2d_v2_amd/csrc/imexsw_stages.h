@@ -321,12 +321,14 @@ __device__ __forceinline__ void assemble_cell(const DevParams& P, const DevPtrs&
 // is q^n, its implicit terms are zero): the stage's state is assembled in place
 // and nothing of it is stored.  Bound by each cell's serial FP64 chain, at 256
 // registers a lane (two waves a SIMD; 301 x 203 cells, N_RK = 3, Newton solves:
-// 64 us a stage, 68 without the bound, and with three waves it spills).  N_RK = 2,
+// 64 us a stage, 68 without the bound, and with three waves it spills; 500 x 386
+// with profiles and model 8: three waves no faster, 560 us with the erosion pass
+// against 554).  N_RK = 2,
 // 100 x 68 cells, model 6: a step's two stages, assembly, stage copies and mask
 // chain 60 us, as one launch and one mask 26; 500 x 386 with profiles and model
 // 8: 750 us for stages and assembly, 630 as one launch.
 template <int NS, bool VP, int RM, bool LAST>
-__global__ void __launch_bounds__(256, (VP && RM == 8) ? 3 : 2) kg_stage(DevParams P, DevPtrs D, RkPtrs G, RkTableau T,
+__global__ void __launch_bounds__(256, 2) kg_stage(DevParams P, DevPtrs D, RkPtrs G, RkTableau T,
                                                    int st, int policy) {
   constexpr int NV = 4 + NS;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
