@@ -1299,7 +1299,7 @@ __device__ __forceinline__ int strip_fit(int nrows, int slots, int max_strip) {
 // item is a listed row.  When every tile is listed the strips are cut from
 // whole tile columns instead, col_h rows each (chosen by the host so that
 // they fill the resident wavefronts evenly: 1000 x 1000 cells are 17 columns
-// of 60 strips of 17 rows, one round of 1020 on 1024 SIMDs, where 8-row
+// of 59 strips of at most 17 rows, one round of 1003 on 1024 SIMDs, where 8-row
 // pieces of tiles made three rounds of 2142).
 template <int NS, bool HASY, bool VP = false>
 __global__ void __launch_bounds__(64) k_stencil(DevParams P, DevPtrs D, int unit,
@@ -1633,7 +1633,7 @@ __global__ void __launch_bounds__(64, 3) k_vp_sides(DevParams P, DevPtrs D) {
 
 // the sides of the y face between rows k-1 (B) and k (T) from the stored
 // sides: Bn, the N side of the cell below, and Ts, the S side of the cell
-// above, with the ring overrides of yface_bottom / yface_top
+// above, with the ring overrides of yface_sides
 template <int NS>
 __device__ __forceinline__ void vp_yface(const DevParams& P, const Side<NS>& Bn,
                                          const Side<NS>& Ts_, const SrcInfo Sb,
@@ -1924,7 +1924,7 @@ __device__ __forceinline__ void stencil_row(const DevParams& P, const DevPtrs& D
     if (wv < 4) {
       // y faces: S face of row k (w0 bottom = row k-1, w1 top = row k) and
       // N face (w2 bottom = row k, w3 top = row k+1).  The cases of
-      // yface_bottom / yface_top and the domain boundary only choose the
+      // yface_sides, the domain boundary among them, only choose the
       // input (the bottom row's value hib = va or the top row's lot = vb)
       // or a zero side, so one make_side on the chosen values, zeroed
       // afterwards where the case says so, gives the same side; distinct

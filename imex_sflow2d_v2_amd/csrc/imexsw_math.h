@@ -59,8 +59,9 @@ __device__ __forceinline__ double quot_n(double a, double b) {
   return __builtin_fma(__builtin_fma(-b, q, a), d.r, q);
 }
 
-// sqrt(x) without the scaling of arguments below 2^-767 (the same bits above
-// it, and for zero, infinity and NaN)
+// sqrt(x) by Goldschmidt's iteration from the reciprocal root's estimate, with
+// the two corrections that round it, and without the scaling of arguments below
+// 2^-767 (the same bits above it, and for zero, infinity and NaN)
 __device__ __forceinline__ double fsqrt(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = y * 0.5;

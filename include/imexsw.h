@@ -328,11 +328,20 @@ int imexsw_kernel_times(imexsw_ctx *ctx, double *ms, int64_t *calls, int cap);
 const char *imexsw_kernel_name(int index);
 
 /* Launch shape of the stencil pass (no reference counterpart: the
- * reference's OpenMP loops have no tiling).  Each step the stencil kernel
- * picks the tallest strip of 2^m rows, m >= 0, up to max_strip_rows, that
- * still leaves about target_strips strips for the step's computed cells.
- * max_strip_rows: 1, 2, 4, 8 or 16; target_strips >= 1.  Results do not
- * depend on these settings; defaults 16 and 2048. */
+ * reference's OpenMP loops have no tiling).  max_strip_rows: 1, 2, 4, 8 or
+ * 16; target_strips >= 1; defaults 16 and 2048.  Results do not depend on
+ * these settings.
+ *
+ * With the defaults, set or not, the dense form's strips are cut from whole
+ * columns of the grid (every work tile listed) or are of the 2^m rows (m <= 4)
+ * that the step's listed rows ask for, so that they fill the device in the
+ * fewest rounds, and steps of few computed cells (below 53 248 with at most
+ * one class, else 36 864) take the sparse form.
+ *
+ * With any other values, and always with vertical profiles, each step takes the
+ * tallest strip of 2^m rows, m >= 0, up to max_strip_rows, that still leaves
+ * about target_strips strips for its computed cells; the sparse form, where
+ * there is one, where that is one row. */
 int imexsw_set_tuning(imexsw_ctx *ctx, int max_strip_rows, int target_strips);
 
 /* Wait for all work queued on the context's stream. */
