@@ -844,7 +844,8 @@ __device__ __forceinline__ void make_side(const DevParams& P, const double* qp, 
   for (int i = 0; i < NS; i++) s.qc[4 + i] = xs[i] * q0;
   s.vel = (DIR == 1) ? u : v;
   s.pt = 0.5 * rho_m * gc * rg * (h * h);
-  if (!__all(wet)) {
+  const bool dry = !__all(wet);
+  if (dry) {
     // dry lanes
 #pragma unroll
     for (int i = 0; i < NV; i++) s.qc[i] = wet ? s.qc[i] : 0.0;
@@ -855,6 +856,8 @@ __device__ __forceinline__ void make_side(const DevParams& P, const double* qp, 
   const double cel = fsqrt((DIR == 1) ? rgh * gc : gc * rg * h);
   s.vmin = (rgh < 0.0) ? s.vel : s.vel - cel;
   s.vmax = (rgh < 0.0) ? s.vel : s.vel + cel;
+  // no flux on a dry side, whatever its velocity (NaN times zero is not zero)
+  if (dry) s.vel = wet ? s.vel : 0.0;
   s.zv = (DIR == 1) ? qp[1] : s.qc[2];
 }
 // with the profiles (bx, by: the slope of the cell the state belongs to, read

@@ -1,0 +1,45 @@
+"""Face sides at the ends of the number range, against the oracle: a dry side
+whose velocity is NaN carries no flux (limiter 0, so that the reconstruction
+itself passes no NaN on).  One step in every form of the stencil and of the
+stage update; equal NaN masks, values within 1e-13 of each variable's largest."""
+import numpy as np
+import pytest
+
+from imex_sflow2d_v2_amd import decks
+from imex_sflow2d_v2_amd.solver import Solver
+from oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+FORMS = [(None, {}), ((16, 1), {}), ((1, 1), {}), (None, dict(n_rk=3)),
+         (None, dict(rheology_model=6, friction_factor=2e-3)), (None, dict(ny=1))]
+
+
+def step(d, tuning):
+    orc, dev = Oracle(d.params, fresh=True), Solver(d.params)
+    orc.load_deck(d)
+    dev.load_deck(d)
+    if tuning:
+        dev.set_tuning(*tuning)
+    assert dev.advance(1, dt0=d.dt0) == orc.run(1, dt0=d.dt0) == 1
+    assert dev.get_dt() == orc.dt_last[0]
+    q, ref = dev.q(), orc.q()
+    assert np.array_equal(np.isnan(q), np.isnan(ref))
+    for v in range(ref.shape[0]):
+        big = np.nanmax(np.abs(ref[v]), initial=0.0)
+        assert np.nanmax(np.abs(q[v] - ref[v]), initial=0.0) <= 1e-13 * max(big, 1e-300), v
+    return dev, ref
+
+
+@pytest.mark.parametrize("tuning,kw", FORMS)
+def test_dry_side_with_a_nan_velocity(tuning, kw):
+    print("dry side", tuning, kw, flush=True)
+    kw = dict(kw)
+    d = decks.small_2d(n=70, ny=kw.pop("ny", 37), seed=3, limiter=0, wet_floor=0.4, n_solid=3, **kw)
+    ny = d.q.shape[2]
+    # mass above the least that counts as wet, thickness below it
+    for j, k in ((20, 5 % ny), (41, 21 % ny), (60, 30 % ny)):
+        d.q[:, j, k] *= 1.0e-15 / d.q[0, j, k]
+        d.q[1:3, j, k] = np.nan
+    _, ref = step(d, tuning)
+    assert np.isnan(ref).any(axis=0).sum() <= 3
