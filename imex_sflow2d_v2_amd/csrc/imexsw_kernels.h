@@ -541,9 +541,8 @@ __device__ __forceinline__ void qp2_uv(const double* qp, double& u, double& v) {
     u = 0.0;
     v = 0.0;
   } else {
-    const Rcp r = rcp_of(qp[0]);
-    u = div_by(qp[1], r);
-    v = div_by(qp[2], r);
+    u = qp[1] / qp[0];
+    v = qp[2] / qp[0];
   }
 }
 
@@ -888,11 +887,11 @@ __device__ __forceinline__ void expand(const DevParams& P, const LeanSide<NS>& s
     o.f[i] = (i == DIR) ? f + s.pt : (i == 3 && P.energy) ? s.vel * (s.qc[3] + s.pt) : f;
     if (i >= 4) sf += f;
   }
-  // (the rounded quotient sf / f0 exceeds 1 exactly when sf exceeds f0 > 0)
+  // (the rounded quotient sf / f0 exceeds 1 exactly when sf exceeds f0 > 0; rare,
+  // and met by subnormal fluxes, whose rounding is coarse: full division)
   if (o.f[0] > 0.0 && sf > o.f[0]) {
-    const Rcp rs = rcp_of(sf);
 #pragma unroll
-    for (int i = 4; i < NV; i++) o.f[i] = div_by(o.f[i], rs) * o.f[0];
+    for (int i = 4; i < NV; i++) o.f[i] = o.f[i] / sf * o.f[0];
   }
   o.vmin = s.vmin;
   o.vmax = s.vmax;
@@ -2263,7 +2262,7 @@ __device__ __forceinline__ void assembly_checks(const DevParams& P, const DevPtr
   if (ssol > q[0]) {
     if ((fdiv(ssol - q[0], q[0]) < 1.0e-10) || (q[0] < kEps)) {
 #pragma unroll
-      for (int i = 0; i < NS; i++) q[4 + i] = fdiv(q[4 + i], ssol) * q[0];
+      for (int i = 0; i < NS; i++) q[4 + i] = q[4 + i] / ssol * q[0];
       cur = false;
     } else {
       if (counts) atomicAdd(&e[C_SUMS - C_NEWTON_CELLS], 1ull);
@@ -2454,8 +2453,9 @@ __device__ __forceinline__ void local_cell(const DevParams& P, const DevPtrs& D,
 #pragma unroll
     for (int i = 0; i < NS; i++) ssol += q[4 + i];
     if (ssol > q[0] && q[0] < 1.0e-10) {
+      // (ssol may be subnormal)
 #pragma unroll
-      for (int i = 0; i < NS; i++) q[4 + i] = fdiv(q[4 + i], ssol) * q[0];
+      for (int i = 0; i < NS; i++) q[4 + i] = q[4 + i] / ssol * q[0];
     }
     double rg = 0.0;
     if (q[0] > 0.0) {

@@ -466,11 +466,11 @@ __device__ __forceinline__ void fluxes(const DevParams& P, const double* qc,
   double sf = 0.0;
 #pragma unroll
   for (int i = 0; i < NS; i++) sf += f[4 + i];
-  // (the rounded quotient sf / f0 exceeds 1 exactly when sf exceeds f0 > 0)
+  // (the rounded quotient sf / f0 exceeds 1 exactly when sf exceeds f0 > 0; rare,
+  // and met by subnormal fluxes: full division)
   if ((f[0] > 0.0) && (sf > f[0])) {
-    const Rcp rs = rcp_of(sf);
 #pragma unroll
-    for (int i = 0; i < NS; i++) f[4 + i] = div_by(f[4 + i], rs) * f[0];
+    for (int i = 0; i < NS; i++) f[4 + i] = f[4 + i] / sf * f[0];
   }
 }
 
@@ -500,25 +500,24 @@ __device__ __forceinline__ void kt_flux(const double* fL, const double* fR,
 #pragma unroll
   for (int i = 0; i < NS; i++) s += H[4 + i];
   // s / H0 >= 1 (DIR 1) or > 1 (DIR 2): the rounded quotient compares with 1
-  // as s compares with H0
-  const bool zcap = H[0] == 0.0 && s != 0.0 && signbit(s) == signbit(H[0]);
+  // as s compares with H0 (infinities apart).  Rare, and met by subnormal fluxes:
+  // full divisions.
+  const bool zcap = H[0] == 0.0 && (s < 0.0 || s > 0.0) && signbit(s) == signbit(H[0]);
   if (DIR == 1) {
     const bool cap = H[0] > 0.0 ? s >= H[0] : H[0] < 0.0 ? s <= H[0] : zcap;
-    if (cap) {
-      const Rcp rH = rcp_of(H[0]);
+    if (cap && fabs(H[0]) < INFINITY) {
       double sr = 0.0;
 #pragma unroll
-      for (int i = 0; i < NS; i++) sr += div_by(H[4 + i], rH);
-      const Rcp rs = rcp_of(sr);
+      for (int i = 0; i < NS; i++) sr += H[4 + i] / H[0];
 #pragma unroll
-      for (int i = 0; i < NS; i++) H[4 + i] = div_by(H[4 + i], rs);
+      for (int i = 0; i < NS; i++) H[4 + i] = H[4 + i] / sr;
     }
   } else {
     const bool cap = H[0] > 0.0 ? s > H[0] : H[0] < 0.0 ? s < H[0] : zcap;
     if (cap) {
-      const Rcp r = rcp_of(fdiv(s, H[0]));
+      const double r = s / H[0];
 #pragma unroll
-      for (int i = 0; i < NS; i++) H[4 + i] = div_by(H[4 + i], r);
+      for (int i = 0; i < NS; i++) H[4 + i] = H[4 + i] / r;
     }
   }
   if (zvL == 0.0 && zvR == 0.0) {

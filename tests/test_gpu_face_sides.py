@@ -1,7 +1,9 @@
-"""Face sides at the ends of the number range, against the oracle: a dry side
-whose velocity is NaN carries no flux (limiter 0, so that the reconstruction
-itself passes no NaN on).  One step in every form of the stencil and of the
-stage update; equal NaN masks, values within 1e-13 of each variable's largest."""
+"""Face sides and solid fluxes at the ends of the number range, against the
+oracle: a dry side whose velocity is NaN carries no flux (limiter 0, so that the
+reconstruction itself passes no NaN on), and momenta of a few hundred subnormal units,
+whose rounded class fluxes exceed the rounded mass flux, stay finite.  One step
+in every form of the stencil and of the stage update; equal NaN masks, values
+within 1e-13 of each variable's largest (1e-313 where that is smaller)."""
 import numpy as np
 import pytest
 
@@ -43,3 +45,22 @@ def test_dry_side_with_a_nan_velocity(tuning, kw):
         d.q[1:3, j, k] = np.nan
     _, ref = step(d, tuning)
     assert np.isnan(ref).any(axis=0).sum() <= 3
+
+
+@pytest.mark.parametrize("tuning,kw", FORMS)
+def test_subnormal_momenta(tuning, kw):
+    print("subnormal momenta", tuning, kw, flush=True)
+    kw = dict(kw)
+    d = decks.small_2d(n=70, ny=kw.pop("ny", 37), seed=3, wet_floor=0.4, n_solid=3, settling=False,
+                       rheology="rheology_model" in kw, **kw)
+    # the same layer everywhere on a flat bed, of mass 0.9 a cell (a class carries a
+    # third of it) and at rest but for a few hundred units
+    d.B_cent[:] = 1.0
+    d.q[:] = d.q[:, 30, :1][:, None, :1] * (0.9 / d.q[0, 30, 0])
+    rng = np.random.default_rng(5)
+    for i in (1, 2):
+        d.q[i] = rng.integers(-400, 401, d.q[i].shape) * 5e-324
+    if d.q.shape[2] == 1:
+        d.q[2] = 0.0
+    _, ref = step(d, tuning)
+    assert not np.isnan(ref).any()
