@@ -486,15 +486,22 @@ __device__ __forceinline__ void kt_flux(const double* fL, const double* fR,
                                         double zvR, double* H) {
   constexpr int NV = 4 + NS;
   const bool same = (aN == aP);
-  // every variable is divided by aP - aN: one reciprocal (speeds below
-  // 1e-290, whose fluxes vanish, are kept off the reciprocal's range)
+  // every variable is divided by aP - aN: one reciprocal, and full divisions for
+  // speeds below its range (a buoyant layer's are its velocity alone, and weigh
+  // the two sides' pressures however small they are)
   const double den = aP - aN;
-  const Rcp rd = rcp_of(den > 1.0e-290 ? den : 1.0);
+  const Rcp rd = rcp_of(den);
   const double aa = div_by(aP * aN, rd);
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const double avg = div_by(aP * fL[i] - aN * fR[i], rd);
     H[i] = same ? 0.0 : avg + aa * (qR[i] - qL[i]);
+  }
+  if (den > 0.0 && den < 1.0e-290) {
+    const double a2 = aP * aN / den;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+      H[i] = (aP * fL[i] - aN * fR[i]) / den + a2 * (qR[i] - qL[i]);
   }
   double s = 0.0;
 #pragma unroll

@@ -1,9 +1,10 @@
 """Face sides and solid fluxes at the ends of the number range, against the
 oracle: a dry side whose velocity is NaN carries no flux (limiter 0, so that the
-reconstruction itself passes no NaN on), and momenta of a few hundred subnormal units,
-whose rounded class fluxes exceed the rounded mass flux, stay finite.  One step
-in every form of the stencil and of the stage update; equal NaN masks, values
-within 1e-13 of each variable's largest (1e-313 where that is smaller)."""
+reconstruction itself passes no NaN on); momenta of a few hundred subnormal
+units, whose rounded class fluxes exceed the rounded mass flux, stay finite; and
+face speeds of 1e-295 weigh the sides as any others do.  One step in every form of
+the stencil and of the stage update; equal NaN masks, values within 1e-13 of each
+variable's largest (1e-313 where that is smaller)."""
 import numpy as np
 import pytest
 
@@ -64,3 +65,24 @@ def test_subnormal_momenta(tuning, kw):
         d.q[2] = 0.0
     _, ref = step(d, tuning)
     assert not np.isnan(ref).any()
+
+
+@pytest.mark.parametrize("kw", [{}, dict(n_rk=3), dict(rheology_model=6, friction_factor=2e-3)])
+def test_tiny_speeds_of_a_buoyant_layer(kw):
+    """Hot gas, lighter than the air: a side's speeds are its velocity alone, and a
+    transverse velocity of 1e-295 weighs the pressures of the two sides.  By the
+    procedures (the erosion pass lets such a layer rise and leaves nothing)."""
+    print("tiny speeds", kw, flush=True)
+    d = decks.small_2d(n=70, ny=37, seed=3, wet_floor=0.4, n_solid=0, settling=False, **kw)
+    rng = np.random.default_rng(6)
+    d.q[2] = rng.uniform(-1.0, 1.0, d.q[2].shape) * 1e-295
+    orc = Oracle(d.params, fresh=True).load_deck(d)
+    dev = Solver(d.params).load_deck(d)
+    assert orc.check_solve(False) == dev.check_solve(False, t=0.0)
+    assert orc.timestep() == dev.timestep()
+    orc.imex_rk(0.0, 1e-3)
+    dev.imex_RK_solver(1e-3, t=0.0)
+    q, ref = dev.q(), orc.q()
+    assert not np.isnan(ref).any() and np.abs(ref[2]).max() > 1e-4
+    for v in range(ref.shape[0]):
+        assert np.abs(q[v] - ref[v]).max() <= 1e-13 * max(np.abs(ref[v]).max(), 1e-300), v
