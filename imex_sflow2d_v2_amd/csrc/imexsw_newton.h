@@ -66,11 +66,13 @@ struct NewtonOut {
 // J1[], J2[] (d nh_{1,2} / d rel_1, rel_2): the partitioned solve of
 // src/solver_2d.f90:1846-1925 on the 2x2 momentum block (the other unknowns'
 // columns are the diagonal org, their right-hand side terms are zero).
-// L receives the block (11, 21, 12, 22).
+// L receives the block (11, 21, 12, 22).  first: the first iteration, in which
+// another unknown's residual that is not finite makes the momenta NaN through
+// those zero terms (later ones have small residuals or NaN momenta already).
 template <int NS>
 __device__ __forceinline__ void newton_step(const double* org, const double* rt, double dta,
                                             const double* J1, const double* J2, double* L,
-                                            double* desc) {
+                                            double* desc, bool first) {
   constexpr int NV = 4 + NS;
   L[0] = org[1] - dta * J1[0];
   L[1] = 0.0 - dta * J1[1];
@@ -82,6 +84,14 @@ __device__ __forceinline__ void newton_step(const double* org, const double* rt,
     if (i == 1) desc[i] = -((rt[1] * L[3] - rt[2] * L[2]) * inv_det) + 0.0;
     else if (i == 2) desc[i] = -((L[0] * rt[2] - L[1] * rt[1]) * inv_det) + 0.0;
     else desc[i] = 0.0 + -fdiv(rt[i], org[i]);
+  }
+  if (first) {
+    double z = 0.0;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+      if (i != 1 && i != 2) z += desc[i] * 0.0;
+    desc[1] += z;
+    desc[2] += z;
   }
 }
 
@@ -258,7 +268,7 @@ __device__ __forceinline__ NewtonOut solve_rk_step(const DevParams& P, double* q
       J2[0] = J2[0] * P.one_by_h;
       J2[1] = J2[1] * P.one_by_h;
     }
-    newton_step<NS>(org, rt, dt * a_diag, J1, J2, L, desc);
+    newton_step<NS>(org, rt, dt * a_diag, J1, J2, L, desc, it == 1);
 #pragma unroll
     for (int i = 0; i < NV; i++) old[i] = rel[i];
     double alam = 1.0;
@@ -377,7 +387,7 @@ __device__ __forceinline__ NewtonOut solve_rk_step_quad(const DevParams& P, doub
       break;
     }
     double L[4];
-    newton_step<NS>(org, rt, dt * a_diag, J1, J2, L, desc);
+    newton_step<NS>(org, rt, dt * a_diag, J1, J2, L, desc, it == 1);
 #pragma unroll
     for (int i = 0; i < NV; i++) old[i] = rel[i];
     LineSearch ls{};
