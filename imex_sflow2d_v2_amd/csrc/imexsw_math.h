@@ -33,8 +33,9 @@ constexpr double kInvLn2 = 1.44269504088896338700e+00;
 // quotient has the same bits for |b| in [2^-1022, 2^1021] and |a| in
 // [2^-969, 2^767 |b|], and for a zero, an infinity or a NaN (the fix-up
 // decides those).  Numerators below 2^-969 lose the exact last bit of a
-// quotient of order 1e-290.  Divisions by one value share its reciprocal:
-// 4 instructions each after the first.
+// quotient of order 1e-290.  A subnormal divisor gives an infinity: where one
+// can be met the division is written in full.  Divisions by one value share its
+// reciprocal: 4 instructions each after the first.
 // ---------------------------------------------------------------------------
 struct Rcp {
   double b, r;  // the divisor and its refined reciprocal
